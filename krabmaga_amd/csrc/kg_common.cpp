@@ -1,6 +1,7 @@
 // kg_common.cpp -- host-side helpers shared by the C ABI implementations:
 // per-thread error messages, the gather switch and the flock kernel's LDS
 // capacity clamp.
+#include <algorithm>
 #include "kg_common.hpp"
 
 #include <cstdlib>
@@ -58,6 +59,35 @@ int clamp_lds_cap(int cap) {
   const size_t budget = (size_t)max_lds - 8192;
   while (cap > 64 && flock_lds_bytes(cap) > budget) cap -= 64;
   return cap;
+}
+
+NearPlan near_plan(int cap, int cols, uint32_t ntiles) {
+  int dev = 0, max_lds = 65536, cu_lds = 160 * 1024;
+  if (hipGetDevice(&dev) == hipSuccess) {
+    int v = 0;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
+        v > 0)
+      max_lds = v;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) ==
+            hipSuccess &&
+        v > 0)
+      cu_lds = v;
+  }
+  // LDS is handed out in steps of 1,280 bytes; the kernel's static tables are
+  // about 1.1 KB.  The capacity grows to the largest that keeps the
+  // work-groups per CU, which its waves also bound.
+  constexpr size_t kStatic = 1280, kStep = 1280;
+  const size_t waves = near_wide(ntiles) ? 4 : 8;  // work-groups of 8 (4) waves per CU
+  const size_t per_wg = (near_lds_bytes(cap, cols) + kStatic + kStep - 1) / kStep * kStep;
+  const size_t fit = std::max<size_t>(1, std::min(waves, (size_t)cu_lds / per_wg));
+  const size_t share = std::min((size_t)cu_lds / fit / kStep * kStep, (size_t)max_lds) - kStatic;
+  while (near_lds_bytes(cap + 16, cols) <= share) cap += 16;
+  while (cap > 64 && near_lds_bytes(cap, cols) > share) cap -= 16;
+  NearPlan p;
+  p.on = true;
+  p.cap = std::min(cap, 4096);
+  p.cols = cols;
+  return p;
 }
 
 }  // namespace kg

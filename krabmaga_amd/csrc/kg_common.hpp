@@ -23,6 +23,10 @@ void clear_error();
 // dynamic plus static LDS fits the device's per-block limit.
 int clamp_lds_cap(int cap);
 
+// The near flock kernel's staging for tiles of `cols` columns expected to
+// stage `cap` birds (pick_lds_cap), `ntiles` work-groups in the launch.
+NearPlan near_plan(int cap, int cols, uint32_t ntiles);
+
 // The gather rebinning after flock steps; KG_REBIN_GATHER=0 turns it off
 // (scatter and bin sort every step), for comparison.
 bool rebin_gather_enabled();

@@ -116,6 +116,7 @@ struct kg_ensemble {
   size_t cap_gflag = 0;
   uint64_t* gstep = nullptr;
   int lds_cap = 1024;
+  NearPlan near{};  // off unless every run is near
   int parity = 0;  // bin-grouped steps taken since the build, mod 2
   // two-step graphs by parity + 2 * gather
   std::vector<std::pair<int, hipGraphExec_t>> bgraphs;
@@ -502,6 +503,13 @@ int rebuild(kg_ensemble* e) {
     int cap = 256;
     for (const EnsRun& r : e->runs) cap = std::max(cap, pick_lds_cap(r.g, r.desc.agents));
     e->lds_cap = clamp_lds_cap(cap);
+    int cols = 1;
+    bool near = true;
+    for (const RepDev& rp : e->h_reps) {
+      cols = std::max(cols, std::min(kMaxStageCols, rp.g.tx + 2 * rp.disc_dist));
+      near = near && rp.near;
+    }
+    e->near = near ? near_plan(cap, cols, e->ntiles) : NearPlan{};
     e->parity = 0;
     e->gather = rebin_gather_enabled();
     for (const RepDev& rp : e->h_reps)
@@ -539,7 +547,8 @@ hipError_t binned_step(kg_ensemble* e, const WorkList& w) {
   if ((err = launch_flock(w, e->R.b, e->offset, e->W.b, count, e->gstep, e->err, e->lds_cap,
                           e->gflag, e->nagents, e->stream,
                           e->gather ? e->outbox : Outbox{}, false,
-                          summed ? e->tsum[p] : nullptr, kEnsGlobalGrid)) != hipSuccess)
+                          summed ? e->tsum[p] : nullptr, kEnsGlobalGrid, e->near)) !=
+      hipSuccess)
     return err;
   const uint32_t nscan = (e->nbins + kScanTile - 1) / kScanTile;
   if (summed) err = launch_scan_prefix(e->tsum[p], nscan, e->stream);

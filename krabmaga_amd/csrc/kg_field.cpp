@@ -43,6 +43,7 @@ struct kg_field {
   Geom g{};
   uint32_t cap = 0;
   int lds_cap = 1024;
+  NearPlan near{};  // of the current parameters' window
   hipStream_t stream = nullptr;
 
   DevBuf R, R2, W, A;
@@ -299,7 +300,7 @@ int flock_impl(kg_field* f, const uint64_t* gstep) {
                       summed ? f->counts(f->parity) : f->count, gstep, f->err,
                       f->lds_cap, f->gflag, (uint32_t)f->nR, f->stream,
                       f->gather_ok ? f->outbox : Outbox{}, f->global_inline,
-                      summed ? f->tsum[f->parity] : nullptr));
+                      summed ? f->tsum[f->parity] : nullptr, 0, f->near));
   f->outbox_filled = f->gather_ok;
   f->nW = f->nR;
   f->w_aligned = true;
@@ -312,6 +313,10 @@ int set_params(kg_field* f, const kg_flock_params* p, uint64_t step_base) {
   if (!params_valid(*p, &why)) return set_error(KG_E_INVALID, "%s", why.c_str());
   set_rep_params(&f->h_rep, *p);
   f->h_rep.step_base = step_base;
+  const int cols = std::min(kMaxStageCols, f->g.tx + 2 * std::max(0, f->h_rep.disc_dist));
+  if (f->h_rep.near && f->near.cols != cols)
+    f->near = near_plan(pick_lds_cap(f->g, f->cap), cols, f->g.ntiles);
+  f->near.on = f->h_rep.near != 0;
   return upload_rep(f);
 }
 

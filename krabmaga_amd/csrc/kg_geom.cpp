@@ -112,6 +112,38 @@ bool params_valid(const kg_flock_params& p, std::string* why) {
   return true;
 }
 
+// The near form's conditions (kg_near.hpp).  `ulp` is the spacing of floats
+// at the far edge of the field: a bird of cell c lies within 2 ulp of
+// [c d, (c + 1) d], and an edge computed in f32 within one.
+static void set_near(RepDev* r) {
+  const Geom& g = r->g;
+  const double d = g.d, w = g.w, h = g.h, dd = r->disc_dist, T = r->sq_thresh;
+  const float edge = std::max(g.w, g.h);
+  const double ulp = (double)std::nextafter(edge, INFINITY) - (double)edge;
+  r->near = r->far = 0;
+  r->sq_near = r->sq_thresh;
+  if (!r->lds_ok || !(T < 0x1p40)) return;
+  // finite sums: a heading is NaN in both parts or in neither
+  for (float v : {r->p.cohesion, r->p.avoidance, r->p.consistency, r->p.randomness,
+                  r->p.momentum, r->p.jump})
+    if (!(std::fabs(v) <= 0x1p30f)) return;
+  // columns and rows in z; a field this wide has ulp <= d / 64
+  if (g.max_x > 65536 || g.max_y > 65536) return;
+  // two birds of one window are less than (dd + 1.25) cells apart: less than
+  // half the torus, where toroidal_distance is the plain difference
+  if (!((dd + 1.25) * d <= 0.5 * std::min(w, h))) return;
+  // positions wrap without fmod (y wraps by the width too)
+  if (!(std::fabs((double)r->p.jump) <= 0.3 * w) || !(h <= 1.5 * w)) return;
+  r->near = 1;
+  // the nearest corner of a window cell: at most dd cells (half a cell for
+  // dd = 0) away per axis
+  const double c = (std::max(dd, 0.5) + 0.05) * d;
+  r->far = 2.0 * c * c * (1.0 + 1e-5) <= T ? 0 : 1;
+  // a bird whose cell's corners are within the radius
+  const double reach = (double)r->p.radius * (1.0 + 1e-6) + 8.0 * ulp;
+  r->sq_near = std::nextafter((float)(reach * reach * (1.0 + 1e-5)), INFINITY);
+}
+
 void set_rep_params(RepDev* r, const kg_flock_params& p) {
   r->p.cohesion = p.cohesion;
   r->p.avoidance = p.avoidance;
@@ -135,6 +167,7 @@ void set_rep_params(RepDev* r, const kg_flock_params& p) {
                r->g.tx + 2 * dd <= kMaxStageCols)
                   ? 1
                   : 0;
+  set_near(r);
 }
 
 }  // namespace kg

@@ -8,6 +8,8 @@
 //   flock     fused neighbour query + Bird::step     field_2d.rs:386-440, bird.rs:38-154
 //             + bin histogram of the new positions
 //   query/... single-replica API queries             field_2d.rs:472-808
+#include "kg_launch.hpp"
+#include "kg_near.hpp"
 #include "kg_phases.hpp"
 #include "kg_rt.hpp"
 
@@ -604,6 +606,109 @@ __global__ __launch_bounds__(kFlockThreads) void k_flock(
   }
 }
 
+// k_flock on a near field (kg_near.hpp): the same tiles, chunks, global path
+// and sinks, the birds staged as sorted records.  A tile with a bird outside
+// the near form takes the global path.  kT threads: the tile's own birds fit
+// one round of 512 where tiles are few.
+// Eight waves per SIMD (64 VGPRs): only the inline global walk spills.
+constexpr uint32_t kNearWideTiles = 1024;
+
+template <int kT, bool kInlineGlobal>
+__global__ __launch_bounds__(kT, 8) void k_flock_near(
+    const RepDev* __restrict__ reps, int nreps, const uint32_t* __restrict__ tile_prefix, Buf R,
+    const uint32_t* __restrict__ offset, Buf W, uint32_t* __restrict__ count_next,
+    const uint64_t* __restrict__ gstep, uint32_t* __restrict__ err, int lds_cap, int cols,
+    uint32_t* __restrict__ gflag, Outbox ob, uint32_t* __restrict__ tile_sum) {
+  extern __shared__ __align__(16) uint8_t smem_raw[];
+  __shared__ uint32_t s_warp[kT / kWave];
+  __shared__ uint32_t s_outn;
+  __shared__ uint32_t s_bad;
+  __shared__ uint32_t s_hist[kGatherMaxBins];
+
+  const int t = threadIdx.x;
+  const uint32_t item = xcd_remap(blockIdx.x, gridDim.x);
+  const FlockTile ft = flock_tile(reps, nreps, tile_prefix, item, *gstep);
+  const RepDev& rp = reps[ft.r];
+  const uint32_t nbt = ft.tb1 - ft.tb0;
+  const NearSmem S = near_carve(smem_raw, lds_cap, cols);
+  if (tile_sum)
+    for (uint32_t b = t; b < nbt; b += kT) s_hist[b] = 0u;
+  const uint32_t len =
+      t < ft.ncols ? flock_segments(rp, ft, t, offset, S.seg_start, S.seg_len) : 0u;
+  uint32_t L;
+  const uint32_t ex = block_exclusive_scan<kT>(len, s_warp, &L);
+  if (t < ft.ncols) S.col_base[t] = ex;
+  if (t == 0) {
+    S.col_base[ft.ncols] = L;
+    s_outn = 0;
+    s_bad = 0;
+  }
+  __syncthreads();
+  const int32_t own_lo = ft.c0 - ft.sc_lo, own_hi = ft.c1 - ft.sc_lo;
+  const uint32_t cap = (uint32_t)lds_cap;
+  const bool chunked = L > cap;
+  bool use_lds = rp.near != 0;
+  if (use_lds && chunked) {
+    use_lds = L <= kFlockChunkFactor * cap;
+    for (int32_t c = own_lo; use_lds && c < own_hi; ++c)
+      if (flock_chunk_size(rp, ft, S.col_base, c, c + 1) > cap) use_lds = false;
+    if (use_lds) {
+      // every bird is looked at before the first chunk is stepped
+      const NearChunk all = near_chunk(rp, ft, S, own_lo, own_hi);
+      for (uint32_t i = t; i < all.n; i += kT)
+        if (!near_item_ok(rp, all, i, R, S)) s_bad = 1u;
+      __syncthreads();
+      use_lds = s_bad == 0u;
+    }
+  }
+  const FlockSinks lv{ob, item - ft.tile, &s_outn, tile_sum ? s_hist : nullptr, tile_sum};
+  for (int32_t oa = own_lo; use_lds && oa < own_hi;) {
+    const int32_t ob2 =
+        chunked ? flock_chunk_end(rp, ft, S.col_base, oa, own_hi, cap) : own_hi;
+    const NearChunk k = near_chunk(rp, ft, S, oa, ob2);
+    for (uint32_t i = t; i < k.n; i += kT)
+      if (!near_stage(rp, ft, k, i, R, S)) s_bad = 1u;
+    if (t == 0) S.bird[k.n].z = ~0u;
+    __syncthreads();
+    use_lds = s_bad == 0u;
+    if (use_lds)
+      for (uint32_t o = t; o < k.nown; o += kT)
+        near_agent(rp, ft, k, o, S, W, count_next, err, lv);
+    oa = ob2;
+    if (oa < own_hi) __syncthreads();  // the next chunk reuses the LDS
+  }
+  if (t == 0) {
+    gflag[item] = use_lds ? 0u : 1u;
+    if (!use_lds) {
+      gflag[gridDim.x] = (uint32_t)*gstep + 1u;
+      atomicAdd(&gflag[gridDim.x + 1], 1u);
+      if (ob.n) ob.n[item] = 0u;  // the global path lists the leavers
+    }
+  }
+  if (use_lds) {
+    if (ob.n || tile_sum) __syncthreads();
+    if (ob.n && t == 0) ob.n[item] = s_outn;
+    if (tile_sum) {
+      // the stayers into their bins; all of them into the one scan tile
+      // that holds the tile's bins, one atomic per wave
+      uint32_t h = 0;
+      for (uint32_t b = t; b < nbt; b += kT) {
+        const uint32_t v = s_hist[b];
+        if (v) atomicAdd(&count_next[ft.tb0 + b], v);
+        h += v;
+      }
+      for (int off = kWave / 2; off > 0; off >>= 1) h += __shfl_xor(h, off, kWave);
+      if ((t & (kWave - 1)) == 0 && h) atomicAdd(&tile_sum[ft.tb0 / (uint32_t)kScanTile], h);
+    }
+  } else if (kInlineGlobal) {
+    __syncthreads();  // the outbox count is cleared
+    const uint32_t lo = offset[ft.tb0], hi = offset[ft.tb1];
+    const FlockSinks lg{ob, item - ft.tile, nullptr, nullptr, tile_sum};
+    for (uint32_t gi = lo + (uint32_t)t; gi < hi; gi += kT)
+      flock_agent_global(rp, ft.step, gi, R, offset, W, count_next, err, lg);
+  }
+}
+
 // The birds of flagged tiles, one thread per read-buffer slot.  The read
 // buffer holds the replicas one after another (replica r at
 // app_prefix[r], its tiles one after another), each tile's bins in order.
@@ -665,15 +770,29 @@ __global__ __launch_bounds__(kFlockThreads) void k_flock_global(
   }
 }
 
+bool near_wide(uint32_t ntiles) { return ntiles <= kNearWideTiles; }
+size_t near_lds_bytes(int cap, int cols) { return near_smem_bytes(cap, cols); }
+
 hipError_t launch_flock(const WorkList& wl, Buf R, const uint32_t* offset, Buf W,
                         uint32_t* count_next, const uint64_t* gstep, uint32_t* err, int lds_cap,
                         uint32_t* gflag, uint32_t nagents, hipStream_t s, const Outbox& ob,
-                        bool inline_global, uint32_t* tile_sum, uint32_t global_grid) {
+                        bool inline_global, uint32_t* tile_sum, uint32_t global_grid,
+                        const NearPlan& near) {
   if (wl.ntiles == 0) return hipSuccess;
-  hipLaunchKernelGGL(inline_global ? k_flock<true> : k_flock<false>, dim3(wl.ntiles),
-                     dim3(kFlockThreads), flock_lds_bytes(lds_cap), s, wl.reps, wl.nreps,
-                     wl.tile_prefix, R, offset, W, count_next, gstep, err, lds_cap, gflag, ob,
-                     tile_sum);
+  if (near.on) {
+    const bool wide = near_wide(wl.ntiles);
+    auto kern = wide ? (inline_global ? k_flock_near<512, true> : k_flock_near<512, false>)
+                     : (inline_global ? k_flock_near<256, true> : k_flock_near<256, false>);
+    hipLaunchKernelGGL(kern, dim3(wl.ntiles), dim3(wide ? 512 : 256),
+                       near_smem_bytes(near.cap, near.cols), s, wl.reps, wl.nreps,
+                       wl.tile_prefix, R, offset, W, count_next, gstep, err, near.cap, near.cols,
+                       gflag, ob, tile_sum);
+  } else {
+    hipLaunchKernelGGL(inline_global ? k_flock<true> : k_flock<false>, dim3(wl.ntiles),
+                       dim3(kFlockThreads), flock_lds_bytes(lds_cap), s, wl.reps, wl.nreps,
+                       wl.tile_prefix, R, offset, W, count_next, gstep, err, lds_cap, gflag, ob,
+                       tile_sum);
+  }
   const uint32_t nruns = (nagents + kFlockThreads - 1) / kFlockThreads;
   if (nagents && !inline_global) {
     const bool stride = global_grid && global_grid < nruns;

@@ -50,6 +50,18 @@ hipError_t launch_rebin_fallback(const WorkList& wl, Buf R, Buf W, const uint32_
                                  uint32_t* cursor, Buf R2, const uint32_t* offset_new, Buf T,
                                  const Gate& gate, uint32_t* err, bool count_down,
                                  hipStream_t s);
+// Whether a launch of ntiles takes 512-thread work-groups.
+bool near_wide(uint32_t ntiles);
+// Bytes of dynamic LDS for `cap` birds and `cols` columns.
+size_t near_lds_bytes(int cap, int cols);
+
+// How the flock step's tiles are staged on a near field (kg_near.hpp): birds
+// and columns of LDS per work-group; off: the general kernel.
+struct NearPlan {
+  bool on = false;
+  int cap = 0, cols = 0;
+};
+
 // gflag: one word per tile plus two (the last counts global-path tiles and
 // starts at zero), nagents: R's count; ob: the outboxes for the gather
 // rebinning that follows, or none; inline_global: each global-path tile is
@@ -57,12 +69,13 @@ hipError_t launch_rebin_fallback(const WorkList& wl, Buf R, Buf W, const uint32_
 // tile_sum: the scan's tile sums to add the counts to (zero on entry; tiles
 // of at most kGatherMaxBins bins, whole tiles per scan tile), or none;
 // global_grid: k_flock_global's work-groups, each looping over runs of
-// birds, or 0 for one per run.
+// birds, or 0 for one per run; near: every replica's near form applies.
 hipError_t launch_flock(const WorkList& wl, Buf R, const uint32_t* offset, Buf W,
                         uint32_t* count_next, const uint64_t* gstep, uint32_t* err, int lds_cap,
                         uint32_t* gflag, uint32_t nagents, hipStream_t s,
                         const Outbox& ob = Outbox{}, bool inline_global = false,
-                        uint32_t* tile_sum = nullptr, uint32_t global_grid = 0);
+                        uint32_t* tile_sum = nullptr, uint32_t global_grid = 0,
+                        const NearPlan& near = NearPlan{});
 hipError_t launch_materialize(Buf R, Buf W, uint32_t n, Buf A, hipStream_t s);
 
 // Tile-resident step (one launch per schedule step); with load != 0 the

@@ -1,0 +1,432 @@
+// kg_near.hpp -- Bird::step on "near" fields: toroidal fields whose windows
+// never reach across the seam, which is every field more than a few cells
+// wide.  There the reference's rules simplify exactly:
+//
+// - Two birds of one window lie within (dd + 1) cells of each other, at most
+//   half the torus, so toroidal_distance is the plain difference.
+// - check_circle's answer rarely matters.  A candidate within the radius is
+//   returned unless all four corners of its cell are beyond it; on a field
+//   whose cells are small against the radius (rep.far == 0) some corner of
+//   every window cell is always within it.  A candidate beyond the radius is
+//   returned only if all four corners are within it, and then it lies at
+//   most a few ulps beyond: only squared distances in (T, Tm] need the
+//   corners looked at.
+// - Quotients by a shared divisor take one reciprocal in f64 (recip_of).
+//
+// Every function gives the bits of the general form (kg_device.hpp).  A
+// neighbourhood that holds a bird outside [0, w] x [0, h], a coordinate below
+// 2^-60, a heading above 2^60 or a NaN is not near (near_bad); the caller
+// takes the general form for it.
+//
+// The walk reads a list of birds in LDS (or any memory) sorted by z =
+// column << kNearRowBits | row, then id: the reference's bag-scan order, in
+// which the rows of one window column are one contiguous run.
+#pragma once
+
+#include "kg_phases.hpp"
+
+namespace kg {
+
+constexpr int kNearRowBits = 20;
+
+struct alignas(16) NearBird {
+  float x, y;
+  uint32_t z, id;
+};
+struct alignas(8) NearHead {
+  float hx, hy;
+};
+
+KG_HD uint32_t f_bits(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __float_as_uint(v);
+#else
+  uint32_t u;
+  __builtin_memcpy(&u, &v, 4);
+  return u;
+#endif
+}
+
+// Whether a bird takes its neighbourhood out of the near form.  (bits - 1)
+// is huge for a zero of either sign: zeros are fine.
+KG_HD bool near_bad(const Geom& g, float x, float y, float hx, float hy) {
+  constexpr uint32_t kTiny = (127u - 60u) << 23;
+  // false for NaN
+  const bool in = x <= g.w && y <= g.h && fabsf(hx) <= 0x1p60f && fabsf(hy) <= 0x1p60f;
+  return !in || f_bits(x) - 1u < kTiny - 1u || f_bits(y) - 1u < kTiny - 1u;
+}
+
+// 1 / b to 2^-52 relative, b a float with |b| in [2^-60, 2^81] (or 0, which
+// gives NaN, as 0 / 0 does).  From the 2^-23 of v_rcp_f32, one third-order
+// step: with e = 1 - b y, y (1 + e + e^2) is off by e^3.
+//
+// (float)((double)a * recip_of(b)) is the correctly rounded a / b for floats
+// a, b with a normal quotient (or a zero or infinite a): a / b lies at least
+// 2^-49 (relative) from every boundary between two floats' rounding
+// intervals (with 24-bit significands A, B and a 25-bit odd boundary M, A 2^k
+// - M B is a nonzero integer), and the product is off by less than 2^-51.
+// f32 division takes 45 cycles of a SIMD's issue per wave, this 13 for each
+// quotient after 34 for the reciprocal (measured on MI355X; f64 operations
+// and conversions issue at the f32 rate there).
+KG_HD double recip_of(float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double d = (double)b;
+  const double y = (double)__builtin_amdgcn_rcpf(b);
+  const double e = __builtin_fma(-d, y, 1.0);
+  return __builtin_fma(y, __builtin_fma(e, e, e), y);
+#else
+  return b == 0.0f ? (double)NAN : 1.0 / (double)b;
+#endif
+}
+
+KG_HD float quot(float a, double r) { return (float)((double)a * r); }
+
+// Bird::step's neighbour sums (bird.rs:54-81); n counts the neighbours.
+struct NearAcc {
+  float x_avoid = 0.0f, y_avoid = 0.0f;
+  float x_cohe = 0.0f, y_cohe = 0.0f;
+  float x_cons = 0.0f, y_cons = 0.0f;
+  int32_t n = 0;
+  bool same = false;  // a bird with the own id was found (itself)
+
+  KG_HD void add(float dx, float dy, float square, float ehx, float ehy) {
+    const double r = recip_of(square * square + 1.0f);
+    n += 1;
+    x_avoid += quot(dx, r);
+    y_avoid += quot(dy, r);
+    x_cohe += dx;
+    y_cohe += dy;
+    x_cons += ehx;
+    y_cons += ehy;
+  }
+};
+
+// check_circle (field_2d.rs:934-972) of cell (bx, by) for a bird at (lx, ly)
+// with plain differences: all four corners within T (want = 1) or all four
+// beyond it (want = -1); see window_checks for the two comparisons.
+KG_HD bool near_corners(const Geom& g, int32_t bx, int32_t by, float lx, float ly, float T,
+                        int want) {
+  const float x0 = (float)bx * g.d, y0 = (float)by * g.d;
+  const float x1 = fminf(x0 + g.d, g.w), y1 = fminf(y0 + g.d, g.h);
+  const float ax = x0 - lx, bx2 = x1 - lx, ay = y0 - ly, by2 = y1 - ly;
+  if (want == 1)
+    return fmaxf(ax * ax, bx2 * bx2) + fmaxf(ay * ay, by2 * by2) <= T;
+  return fminf(ax * ax, bx2 * bx2) + fminf(ay * ay, by2 * by2) > T;
+}
+
+// One candidate of the bird `qid` at (qx, qy): c (its column relative to
+// col0) and its heading.
+KG_HD void near_candidate(const RepDev& rp, int32_t col0, float qx, float qy, uint32_t qid,
+                          const NearBird& c, const NearHead& h, NearAcc* acc) {
+  const float dx = qx - c.x, dy = qy - c.y;
+  const float s = dx * dx + dy * dy;
+  bool ok = s <= rp.sq_thresh;
+  // both exceptions are rare: the corners decide
+  if (ok ? rp.far != 0 : s <= rp.sq_near) {
+    const int32_t bx = col0 + (int32_t)(c.z >> kNearRowBits);
+    const int32_t by = (int32_t)(c.z & ((1u << kNearRowBits) - 1u));
+    if (near_corners(rp.g, bx, by, qx, qy, rp.sq_thresh, ok ? -1 : 1)) ok = !ok;
+  }
+  if (!ok) return;
+  if (c.id != qid) acc->add(dx, dy, s, h.hx, h.hy);
+  else acc->same = true;
+}
+
+// Whether every one of six sums is zero, infinite, NaN or at least 2^-60 in
+// magnitude (doubling the bits drops the sign; minus one makes zero huge).
+KG_HD uint32_t mag_key(float v) { return (f_bits(v) << 1) - 1u; }
+KG_HD uint32_t umin2(uint32_t a, uint32_t b) { return a < b ? a : b; }
+constexpr uint32_t kMagTiny = ((127u - 60u) << 24) - 1u;
+constexpr uint32_t kMagHuge = ((127u + 60u) << 24) - 1u;
+
+// bird.rs:83-153 with the shared reciprocals; flock_finish's arguments and
+// results.
+KG_HD void near_finish(const NearAcc& a, const FlockParams& p, uint32_t id, uint64_t step,
+                       float px, float py, float hx, float hy, float width, float* nx,
+                       float* ny, float* nhx, float* nhy) {
+  const uint32_t m = umin2(umin2(umin2(mag_key(a.x_avoid), mag_key(a.y_avoid)),
+                                 umin2(mag_key(a.x_cohe), mag_key(a.y_cohe))),
+                           umin2(mag_key(a.x_cons), mag_key(a.y_cons)));
+  const bool plain = m >= kMagTiny;
+  float avoid_x = 0.0f, avoid_y = 0.0f, cohe_x = 0.0f, cohe_y = 0.0f;
+  float rand_x = 0.0f, rand_y = 0.0f, cons_x = 0.0f, cons_y = 0.0f;
+  if (a.same || a.n != 0) {
+    float x_avoid = a.x_avoid, y_avoid = a.y_avoid, x_cohe = a.x_cohe, y_cohe = a.y_cohe;
+    cons_x = a.x_cons;
+    cons_y = a.y_cons;
+    if (a.n > 0) {
+      const float c = (float)a.n;
+      if (plain) {
+        const double r = recip_of(c);
+        x_avoid = quot(x_avoid, r);
+        y_avoid = quot(y_avoid, r);
+        x_cohe = quot(x_cohe, r);
+        y_cohe = quot(y_cohe, r);
+        cons_x = quot(quot(cons_x, r), r);
+        cons_y = quot(quot(cons_y, r), r);
+      } else {
+        x_avoid /= c;
+        y_avoid /= c;
+        x_cohe /= c;
+        y_cohe /= c;
+        cons_x = cons_x / c / c;
+        cons_y = cons_y / c / c;
+      }
+    }
+    avoid_x = 400.0f * x_avoid;
+    avoid_y = 400.0f * y_avoid;
+    if (plain) {
+      // 0.1 is off by 2^-56 relative: the same argument as recip_of's
+      cohe_x = quot(-x_cohe, 0.1);
+      cohe_y = quot(-y_cohe, 0.1);
+    } else {
+      cohe_x = -x_cohe / 10.0f;
+      cohe_y = -y_cohe / 10.0f;
+    }
+    float r1, r2;
+    step_uniforms(p.seed, id, step, &r1, &r2);
+    const float x_rand = r1 * 2.0f - 1.0f;
+    const float y_rand = r2 * 2.0f - 1.0f;
+    // the draws are multiples of 2^-23: sq is zero or at least that
+    const float sq = sqrtf(x_rand * x_rand + y_rand * y_rand);
+    const double rs = recip_of(sq);
+    rand_x = quot(0.05f * x_rand, rs);
+    rand_y = quot(0.05f * y_rand, rs);
+  }
+  float dx = p.cohesion * cohe_x + p.avoidance * avoid_x + p.consistency * cons_x +
+             p.randomness * rand_x + p.momentum * hx;
+  float dy = p.cohesion * cohe_y + p.avoidance * avoid_y + p.consistency * cons_y +
+             p.randomness * rand_y + p.momentum * hy;
+  const float dis = sqrtf(dx * dx + dy * dy);
+  if (dis > 0.0f) {
+    if (umin2(mag_key(dx), mag_key(dy)) >= kMagTiny && mag_key(dis) >= kMagTiny &&
+        mag_key(dis) < kMagHuge) {
+      const double r = recip_of(dis);
+      dx = quot(dx, r) * p.jump;
+      dy = quot(dy, r) * p.jump;
+    } else {
+      dx = dx / dis * p.jump;
+      dy = dy / dis * p.jump;
+    }
+  }
+  *nhx = dx;
+  *nhy = dy;
+  // |dx|, |dy| <= 1.5 |jump| <= 0.45 width and py <= 1.5 width, or both NaN:
+  // toroidal_transform without its fmod case
+  const float vx = px + dx, vy = py + dy;  // bird.rs:147 wraps y by width
+  *nx = vx >= width ? vx - width : (vx < 0.0f ? vx + width : vx);
+  *ny = vy >= width ? vy - width : (vy < 0.0f ? vy + width : vy);
+}
+
+// First entry of birds[lo, hi) (sorted by z) with z >= key.
+KG_HD uint32_t near_lower(const NearBird* birds, uint32_t lo, uint32_t hi, uint32_t key) {
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (birds[mid].z < key) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo;
+}
+
+// The neighbour sums of the bird at (qx, qy), cell row cy and relative
+// column c: every window column's run of birds[], found between col_base[]
+// of the column and of the next (less `base`).  birds[] ends in an entry with
+// z = ~0u.  Columns are relative to col0.
+template <class ColBase>
+KG_HD void near_walk(const RepDev& rp, int32_t col0, float qx, float qy, uint32_t qid, int32_t c,
+                     int32_t cy, const ColBase* col_base, uint32_t base, const NearBird* birds,
+                     const NearHead* heads, NearAcc* acc) {
+  const Geom& g = rp.g;
+  const int32_t dd = rp.disc_dist;
+  // clamped window (field_2d.rs:401-416)
+  const int32_t min_j = imax(0, cy - dd), max_j = imin(cy + dd, g.max_y - 1);
+  const int32_t min_c = imax(-col0, c - dd), max_c = imin(c + dd, g.max_x - 1 - col0);
+  if (max_j < min_j || max_c < min_c) return;
+  const uint32_t rows = (uint32_t)(max_j - min_j);
+  if (dd == 1) {
+    // the three columns' starts bisected side by side (three LDS reads in
+    // flight), then one loop over their runs: a wave's trips are those of
+    // its busiest lane, not of each column's
+    uint32_t lo[3], n[3], key[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int32_t cc = min_c + q;
+      const bool in = cc <= max_c;
+      key[q] = ((uint32_t)cc << kNearRowBits) + (uint32_t)min_j;
+      lo[q] = in ? (uint32_t)col_base[cc] - base : 0u;
+      n[q] = in ? (uint32_t)col_base[cc + 1] - base - lo[q] : 0u;
+      if (!in) key[q] = 0u;
+    }
+    while (n[0] | n[1] | n[2]) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const uint32_t half = n[q] >> 1;
+        const uint32_t mid = lo[q] + half;
+        const bool up = n[q] != 0u && birds[mid].z < key[q];
+        lo[q] = up ? mid + 1u : lo[q];
+        n[q] = up ? n[q] - half - 1u : half;
+      }
+    }
+    const int32_t cols = max_c - min_c;  // 0 .. 2
+    uint32_t e = lo[0], last = key[0] + rows;
+    for (int32_t q = 0;;) {
+      const NearBird b = birds[e];
+      const NearHead h = heads[e];
+      if (b.z <= last) {
+        near_candidate(rp, col0, qx, qy, qid, b, h, acc);
+        ++e;
+      } else {
+        if (++q > cols) break;
+        e = q == 1 ? lo[1] : lo[2];
+        last = (q == 1 ? key[1] : key[2]) + rows;
+      }
+    }
+    return;
+  }
+  for (int32_t cc = min_c; cc <= max_c; ++cc) {
+    const uint32_t key = ((uint32_t)cc << kNearRowBits) + (uint32_t)min_j;
+    uint32_t e = near_lower(birds, (uint32_t)col_base[cc] - base,
+                            (uint32_t)col_base[cc + 1] - base, key);
+    for (;; ++e) {
+      const NearBird b = birds[e];
+      if (b.z > key + rows) break;
+      near_candidate(rp, col0, qx, qy, qid, b, heads[e], acc);
+    }
+  }
+}
+
+// ---- staging a tile ---------------------------------------------------------
+//
+// A tile's own birds are one run of the read buffer, so they are enumerated
+// by their read-buffer index; the halo's (the bands above and below the own
+// columns, whole columns beside them) follow.  Both go to their place in the
+// z order.
+
+// LDS of a staged tile: `cap` birds and the per-column tables of `cols`
+// columns.
+struct NearSmem {
+  NearBird* bird;       // cap + 1
+  NearHead* head;       // cap + 1
+  uint32_t* seg_start;  // 3 per column (flock_segments)
+  uint32_t* seg_len;    // 3 per column
+  uint32_t* col_base;   // cols + 1
+  uint16_t* own;        // cap: slots of the own birds, in read-buffer order
+};
+
+KG_HD size_t near_smem_bytes(int cap, int cols) {
+  return (size_t)(cap + 1) * (sizeof(NearBird) + sizeof(NearHead)) +
+         (size_t)(7 * cols + 1) * sizeof(uint32_t) + (size_t)((cap + 1) & ~1) * sizeof(uint16_t);
+}
+
+KG_HD NearSmem near_carve(uint8_t* p, int cap, int cols) {
+  NearSmem s;
+  s.bird = (NearBird*)p;
+  s.head = (NearHead*)(s.bird + cap + 1);
+  s.seg_start = (uint32_t*)(s.head + cap + 1);
+  s.seg_len = s.seg_start + 3 * cols;
+  s.col_base = s.seg_len + 3 * cols;
+  s.own = (uint16_t*)(s.col_base + cols + 1);
+  return s;
+}
+
+// The staged items of own columns [oa, ob): staged columns [sa, sb), n items
+// of which nown are the own birds [own_lo, own_lo + nown) of the read buffer.
+struct NearChunk {
+  int32_t oa, ob, sa, sb;
+  uint32_t base, n, own_lo, nown;
+};
+
+KG_HD NearChunk near_chunk(const RepDev& rp, const FlockTile& ft, const NearSmem& S, int32_t oa,
+                           int32_t ob) {
+  NearChunk k;
+  k.oa = oa;
+  k.ob = ob;
+  flock_chunk_cols(rp, ft, oa, ob, &k.sa, &k.sb);
+  k.base = S.col_base[k.sa];
+  k.n = S.col_base[k.sb] - k.base;
+  k.own_lo = S.seg_start[3 * oa + 1];
+  k.nown = S.seg_start[3 * (ob - 1) + 1] + S.seg_len[3 * (ob - 1) + 1] - k.own_lo;
+  return k;
+}
+
+// Halo items in staged columns [sa, c).
+KG_HD uint32_t near_halo_before(const NearChunk& k, const NearSmem& S, int32_t c) {
+  const uint32_t all = S.col_base[c] - k.base;
+  if (c <= k.oa) return all;
+  return all - (c >= k.ob ? k.nown : S.seg_start[3 * c + 1] - k.own_lo);
+}
+
+// Read-buffer index of halo item m, and its slot.
+KG_HD uint32_t near_halo(const NearChunk& k, const NearSmem& S, uint32_t m, uint32_t* slot) {
+  int32_t lo = k.sa, hi = k.sb;  // column c with before(c) <= m < before(c + 1)
+  while (hi - lo > 1) {
+    const int32_t mid = (lo + hi) >> 1;
+    if (near_halo_before(k, S, mid) <= m) lo = mid;
+    else hi = mid;
+  }
+  uint32_t off = m - near_halo_before(k, S, lo);
+  const uint32_t l0 = S.seg_len[3 * lo], l1 = S.seg_len[3 * lo + 1];
+  const uint32_t first = S.col_base[lo] - k.base;
+  if (off < l0) {
+    *slot = first + off;
+    return S.seg_start[3 * lo] + off;
+  }
+  off -= l0;
+  if (lo < k.oa || lo >= k.ob) {
+    if (off < l1) {
+      *slot = first + l0 + off;
+      return S.seg_start[3 * lo + 1] + off;
+    }
+    off -= l1;
+  }
+  *slot = first + l0 + l1 + off;
+  return S.seg_start[3 * lo + 2] + off;
+}
+
+// Stages item i (< k.n: own birds first); false if it is not near.
+KG_HD bool near_stage(const RepDev& rp, const FlockTile& ft, const NearChunk& k, uint32_t i,
+                      Buf R, const NearSmem& S) {
+  const Geom& g = rp.g;
+  uint32_t slot = 0, gi;
+  const bool mine = i < k.nown;
+  if (mine) gi = k.own_lo + i;
+  else gi = near_halo(k, S, i - k.nown, &slot);
+  const float x = R.x[gi], y = R.y[gi];
+  const float hx = R.hx[gi], hy = R.hy[gi];
+  const uint32_t id = R.id[gi];
+  const int32_t c = disc_axis(x, g.d, g.inv_d) - ft.sc_lo;
+  const int32_t cy = disc_axis(y, g.d, g.inv_d);
+  if (mine) {
+    slot = S.col_base[c] - k.base + S.seg_len[3 * c] + (gi - S.seg_start[3 * c + 1]);
+    S.own[i] = (uint16_t)slot;
+  }
+  S.bird[slot] = NearBird{x, y, ((uint32_t)c << kNearRowBits) | (uint32_t)cy, id};
+  S.head[slot] = NearHead{hx, hy};
+  return !near_bad(g, x, y, hx, hy);
+}
+
+// Whether staged item i of a chunk is near (without staging it).
+KG_HD bool near_item_ok(const RepDev& rp, const NearChunk& k, uint32_t i, Buf R,
+                        const NearSmem& S) {
+  uint32_t slot;
+  const uint32_t gi = i < k.nown ? k.own_lo + i : near_halo(k, S, i - k.nown, &slot);
+  return !near_bad(rp.g, R.x[gi], R.y[gi], R.hx[gi], R.hy[gi]);
+}
+
+// Bird::step of own bird o of a staged chunk.
+KG_HD void near_agent(const RepDev& rp, const FlockTile& ft, const NearChunk& k, uint32_t o,
+                      const NearSmem& S, Buf W, uint32_t* count_next, uint32_t* err,
+                      const FlockSinks& lv) {
+  const uint32_t slot = S.own[o];
+  const NearBird b = S.bird[slot];
+  const NearHead h = S.head[slot];
+  NearAcc acc;
+  near_walk(rp, ft.sc_lo, b.x, b.y, b.id, (int32_t)(b.z >> kNearRowBits),
+            (int32_t)(b.z & ((1u << kNearRowBits) - 1u)), S.col_base, k.base, S.bird, S.head,
+            &acc);
+  float nx, ny, nhx, nhy;
+  near_finish(acc, rp.p, b.id, ft.step, b.x, b.y, h.hx, h.hy, rp.g.w, &nx, &ny, &nhx, &nhy);
+  flock_emit(rp.g, rp.bin_base, W, k.own_lo + o, nx, ny, nhx, nhy, count_next, err, ft.tile, lv);
+}
+
+}  // namespace kg

@@ -16,6 +16,7 @@
 // different streams or host threads) race on it.  Everything a call reads
 // before writing is cleared by the call itself (bin counts, error word, step
 // counter) with fill kernels, so the previous call's contents never leak.
+#include <algorithm>
 #include <mutex>
 
 #include "kg_common.hpp"
@@ -203,7 +204,12 @@ extern "C" int kg_schedule_step_static(const kg_field_desc* desc, const kg_flock
     return set_error(KG_E_RANGE, "an input location discretizes outside the bag grid");
   // Bird::step of every agent at schedule step `step` (schedule.rs:395-408),
   // then Flocker::update's lazy_update into the caller's output
-  KG_HIP(launch_flock(wl, c.R, c.offset, c.W, c.count, c.gstep, c.err, lds_cap, c.gflag, n, s));
+  NearPlan near;
+  if (h.near)
+    near = near_plan(pick_lds_cap(g, desc->capacity),
+                     std::min(kMaxStageCols, g.tx + 2 * h.disc_dist), g.ntiles);
+  KG_HIP(launch_flock(wl, c.R, c.offset, c.W, c.count, c.gstep, c.err, lds_cap, c.gflag, n, s,
+                      Outbox{}, false, nullptr, 0, near));
   KG_HIP(launch_scan(c.count, c.offset2, c.cursor, g.nbins, ss, nullptr, s));
   KG_HIP(launch_scatter_aligned(wl, c.R, c.W, c.offset, c.cursor, out, s));
   KG_HIP(launch_sort_bins(wl, out, c.offset2, c.W, s));
