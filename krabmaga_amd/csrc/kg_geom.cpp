@@ -44,6 +44,7 @@ bool make_geom(float w, float h, float d, int tor, uint64_t expected_agents, uin
   g->h = h;
   g->d = d;
   g->inv_d = 1.0f / d;
+  g->inv_d64 = 1.0 / (double)d;
   g->tor = tor ? 1 : 0;
   g->max_x = (int32_t)cw;
   g->max_y = (int32_t)ch;
@@ -120,7 +121,8 @@ static void set_near(RepDev* r) {
   const double d = g.d, w = g.w, h = g.h, dd = r->disc_dist, T = r->sq_thresh;
   const float edge = std::max(g.w, g.h);
   const double ulp = (double)std::nextafter(edge, INFINITY) - (double)edge;
-  r->near = r->far = 0;
+  r->near = 0;
+  r->sq_sure = -1.0f;
   r->sq_near = r->sq_thresh;
   if (!r->lds_ok || !(T < 0x1p40)) return;
   // finite sums: a heading is NaN in both parts or in neither
@@ -138,7 +140,7 @@ static void set_near(RepDev* r) {
   // the nearest corner of a window cell: at most dd cells (half a cell for
   // dd = 0) away per axis
   const double c = (std::max(dd, 0.5) + 0.05) * d;
-  r->far = 2.0 * c * c * (1.0 + 1e-5) <= T ? 0 : 1;
+  if (2.0 * c * c * (1.0 + 1e-5) <= T) r->sq_sure = r->sq_thresh;
   // a bird whose cell's corners are within the radius
   const double reach = (double)r->p.radius * (1.0 + 1e-6) + 8.0 * ulp;
   r->sq_near = std::nextafter((float)(reach * reach * (1.0 + 1e-5)), INFINITY);

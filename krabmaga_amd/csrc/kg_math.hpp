@@ -190,7 +190,23 @@ struct Geom {
   uint32_t ntiles;
   uint32_t nbins;          // ntiles * tx * tr
   float inv_d;             // fl(1 / d), for disc_axis
+  double inv_d64;          // 1 / d in f64, for cell_axis
 };
+
+// a / b, correctly rounded, from r = 1 / b known to 2^-52 relative (floats a,
+// b; a zero, infinite or NaN, or a / b a normal float): a / b lies at least
+// 2^-49 (relative) from every boundary between two floats' rounding intervals
+// (with 24-bit significands A, B and a 25-bit odd boundary M, A 2^k - M B is
+// a nonzero integer), and a r is off by less than 2^-51.
+KG_HD float quot(float a, double r) { return (float)((double)a * r); }
+
+// disc_axis for a coordinate v that lies in a cell of the grid (or is NaN,
+// cell 0): floor(fl(v / d)) without a branch, a third of disc_axis'
+// instructions.  A quotient too small to be normal floors to 0 either way.
+KG_HD int32_t cell_axis(const Geom& g, float v) {
+  const float q = fmaxf(floorf(quot(v, g.inv_d64)), 0.0f);
+  return (int32_t)q;
+}
 
 // floor(v / d) as Rust's `(v / d).floor() as i32` computes it: the correctly
 // rounded quotient, floored, converted with saturation.  Fast path: with

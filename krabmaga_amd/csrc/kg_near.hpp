@@ -6,7 +6,7 @@
 //   half the torus, so toroidal_distance is the plain difference.
 // - check_circle's answer rarely matters.  A candidate within the radius is
 //   returned unless all four corners of its cell are beyond it; on a field
-//   whose cells are small against the radius (rep.far == 0) some corner of
+//   whose cells are small against the radius (rep.sq_sure) some corner of
 //   every window cell is always within it.  A candidate beyond the radius is
 //   returned only if all four corners are within it, and then it lies at
 //   most a few ulps beyond: only squared distances in (T, Tm] need the
@@ -57,17 +57,11 @@ KG_HD bool near_bad(const Geom& g, float x, float y, float hx, float hy) {
 }
 
 // 1 / b to 2^-52 relative, b a float with |b| in [2^-60, 2^81] (or 0, which
-// gives NaN, as 0 / 0 does).  From the 2^-23 of v_rcp_f32, one third-order
-// step: with e = 1 - b y, y (1 + e + e^2) is off by e^3.
-//
-// (float)((double)a * recip_of(b)) is the correctly rounded a / b for floats
-// a, b with a normal quotient (or a zero or infinite a): a / b lies at least
-// 2^-49 (relative) from every boundary between two floats' rounding
-// intervals (with 24-bit significands A, B and a 25-bit odd boundary M, A 2^k
-// - M B is a nonzero integer), and the product is off by less than 2^-51.
-// f32 division takes 45 cycles of a SIMD's issue per wave, this 13 for each
-// quotient after 34 for the reciprocal (measured on MI355X; f64 operations
-// and conversions issue at the f32 rate there).
+// gives NaN, as 0 / 0 does), for quot.  From the 2^-23 of v_rcp_f32, one
+// third-order step: with e = 1 - b y, y (1 + e + e^2) is off by e^3.  f32
+// division takes 45 cycles of a SIMD's issue per wave, quot 13 after 34 for
+// the reciprocal (measured on MI355X, where f64 operations and conversions
+// issue at the f32 rate).
 KG_HD double recip_of(float b) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const double d = (double)b;
@@ -79,15 +73,12 @@ KG_HD double recip_of(float b) {
 #endif
 }
 
-KG_HD float quot(float a, double r) { return (float)((double)a * r); }
-
 // Bird::step's neighbour sums (bird.rs:54-81); n counts the neighbours.
 struct NearAcc {
   float x_avoid = 0.0f, y_avoid = 0.0f;
   float x_cohe = 0.0f, y_cohe = 0.0f;
   float x_cons = 0.0f, y_cons = 0.0f;
   int32_t n = 0;
-  bool same = false;  // a bird with the own id was found (itself)
 
   KG_HD void add(float dx, float dy, float square, float ehx, float ehy) {
     const double r = recip_of(square * square + 1.0f);
@@ -121,15 +112,19 @@ KG_HD void near_candidate(const RepDev& rp, int32_t col0, float qx, float qy, ui
   const float dx = qx - c.x, dy = qy - c.y;
   const float s = dx * dx + dy * dy;
   bool ok = s <= rp.sq_thresh;
-  // both exceptions are rare: the corners decide
-  if (ok ? rp.far != 0 : s <= rp.sq_near) {
+  if (s > rp.sq_sure && s <= rp.sq_near) {  // rare: the corners decide
     const int32_t bx = col0 + (int32_t)(c.z >> kNearRowBits);
     const int32_t by = (int32_t)(c.z & ((1u << kNearRowBits) - 1u));
     if (near_corners(rp.g, bx, by, qx, qy, rp.sq_thresh, ok ? -1 : 1)) ok = !ok;
   }
-  if (!ok) return;
-  if (c.id != qid) acc->add(dx, dy, s, h.hx, h.hy);
-  else acc->same = true;
+  if (ok && c.id != qid) acc->add(dx, dy, s, h.hx, h.hy);
+}
+
+// Whether the bird at (qx, qy) of cell (cx, cy) finds itself: its own bag is
+// in the window and not all of the bag's corners are beyond the radius.
+KG_HD bool near_self(const RepDev& rp, float qx, float qy, int32_t cx, int32_t cy) {
+  if (cx >= rp.g.max_x || cy >= rp.g.max_y) return false;
+  return !(rp.sq_sure < 0.0f && near_corners(rp.g, cx, cy, qx, qy, rp.sq_thresh, -1));
 }
 
 // Whether every one of six sums is zero, infinite, NaN or at least 2^-60 in
@@ -140,17 +135,18 @@ constexpr uint32_t kMagTiny = ((127u - 60u) << 24) - 1u;
 constexpr uint32_t kMagHuge = ((127u + 60u) << 24) - 1u;
 
 // bird.rs:83-153 with the shared reciprocals; flock_finish's arguments and
-// results.
-KG_HD void near_finish(const NearAcc& a, const FlockParams& p, uint32_t id, uint64_t step,
-                       float px, float py, float hx, float hy, float width, float* nx,
-                       float* ny, float* nhx, float* nhy) {
+// results.  found: the neighbour vector is not empty.
+KG_HD void near_finish(const NearAcc& a, bool found, const FlockParams& p, uint32_t id,
+                       uint64_t step,
+                       float px, float py, float hx, float hy, float width, float* nx, float* ny,
+                       float* nhx, float* nhy) {
   const uint32_t m = umin2(umin2(umin2(mag_key(a.x_avoid), mag_key(a.y_avoid)),
                                  umin2(mag_key(a.x_cohe), mag_key(a.y_cohe))),
                            umin2(mag_key(a.x_cons), mag_key(a.y_cons)));
   const bool plain = m >= kMagTiny;
   float avoid_x = 0.0f, avoid_y = 0.0f, cohe_x = 0.0f, cohe_y = 0.0f;
   float rand_x = 0.0f, rand_y = 0.0f, cons_x = 0.0f, cons_y = 0.0f;
-  if (a.same || a.n != 0) {
+  if (found) {
     float x_avoid = a.x_avoid, y_avoid = a.y_avoid, x_cohe = a.x_cohe, y_cohe = a.y_cohe;
     cons_x = a.x_cons;
     cons_y = a.y_cons;
@@ -228,47 +224,95 @@ KG_HD uint32_t near_lower(const NearBird* birds, uint32_t lo, uint32_t hi, uint3
   return lo;
 }
 
-// The neighbour sums of the bird at (qx, qy), cell row cy and relative
-// column c: every window column's run of birds[], found between col_base[]
-// of the column and of the next (less `base`).  birds[] ends in an entry with
-// z = ~0u.  Columns are relative to col0.
-template <class ColBase>
-KG_HD void near_walk(const RepDev& rp, int32_t col0, float qx, float qy, uint32_t qid, int32_t c,
-                     int32_t cy, const ColBase* col_base, uint32_t base, const NearBird* birds,
-                     const NearHead* heads, NearAcc* acc) {
-  const Geom& g = rp.g;
-  const int32_t dd = rp.disc_dist;
-  // clamped window (field_2d.rs:401-416)
-  const int32_t min_j = imax(0, cy - dd), max_j = imin(cy + dd, g.max_y - 1);
-  const int32_t min_c = imax(-col0, c - dd), max_c = imin(c + dd, g.max_x - 1 - col0);
-  if (max_j < min_j || max_c < min_c) return;
-  const uint32_t rows = (uint32_t)(max_j - min_j);
-  if (dd == 1) {
-    // the three columns' starts bisected side by side (three LDS reads in
-    // flight), then one loop over their runs: a wave's trips are those of
-    // its busiest lane, not of each column's
-    uint32_t lo[3], n[3], key[3];
+// Where a window column's run starts: the first entry of birds[] at or after
+// z = key = c << kNearRowBits | row, of one column or of three neighbouring
+// ones.
+//
+// TileFind: birds[] holds the staged columns of a tile, column c from
+// col_base[c] - base; bisected, three columns side by side (three LDS reads
+// in flight).
+struct TileFind {
+  const NearBird* birds;
+  const uint32_t* col_base;
+  uint32_t base;
+
+  KG_HD uint32_t one(int32_t c, int32_t row) const {
+    return near_lower(birds, col_base[c] - base, col_base[c + 1] - base,
+                      ((uint32_t)c << kNearRowBits) + (uint32_t)row);
+  }
+  KG_HD void three(int32_t c, int32_t cols, int32_t row, uint32_t* lo) const {
+    uint32_t n[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      const int32_t cc = min_c + q;
-      const bool in = cc <= max_c;
-      key[q] = ((uint32_t)cc << kNearRowBits) + (uint32_t)min_j;
-      lo[q] = in ? (uint32_t)col_base[cc] - base : 0u;
-      n[q] = in ? (uint32_t)col_base[cc + 1] - base - lo[q] : 0u;
-      if (!in) key[q] = 0u;
+      lo[q] = q <= cols ? col_base[c + q] - base : 0u;
+      n[q] = q <= cols ? col_base[c + q + 1] - base - lo[q] : 0u;
     }
+    const uint32_t key = ((uint32_t)c << kNearRowBits) + (uint32_t)row;
     while (n[0] | n[1] | n[2]) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         const uint32_t half = n[q] >> 1;
         const uint32_t mid = lo[q] + half;
-        const bool up = n[q] != 0u && birds[mid].z < key[q];
+        const bool up = n[q] != 0u && birds[mid].z < key + ((uint32_t)q << kNearRowBits);
         lo[q] = up ? mid + 1u : lo[q];
         n[q] = up ? n[q] - half - 1u : half;
       }
     }
-    const int32_t cols = max_c - min_c;  // 0 .. 2
-    uint32_t e = lo[0], last = key[0] + rows;
+  }
+};
+
+// CellFind: birds[] holds a whole field in bins of 1 << shift rows, column by
+// column, `rows` bins to a column, bin b from start[b].
+struct CellFind {
+  const NearBird* birds;
+  const uint32_t* start;
+  int32_t rows, shift;
+
+  KG_HD uint32_t one(int32_t c, int32_t row) const {
+    uint32_t e = start[c * rows + (row >> shift)];
+    if (shift) {
+      const uint32_t key = ((uint32_t)c << kNearRowBits) + (uint32_t)row;
+      while (birds[e].z < key) ++e;  // the last entry's z is ~0u
+    }
+    return e;
+  }
+  KG_HD void three(int32_t c, int32_t cols, int32_t row, uint32_t* lo) const {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) lo[q] = q <= cols ? one(c + q, row) : 0u;
+  }
+};
+
+// The clamped window of a bird in cell (c + col0, cy) (field_2d.rs:401-416),
+// columns relative to col0; empty if cols < 0 or rows < 0.
+struct NearWindow {
+  int32_t c, cols, row, rows;
+};
+
+KG_HD NearWindow near_window(const RepDev& rp, int32_t col0, int32_t c, int32_t cy) {
+  const int32_t dd = rp.disc_dist;
+  NearWindow w;
+  w.c = imax(-col0, c - dd);
+  w.cols = imin(c + dd, rp.g.max_x - 1 - col0) - w.c;
+  w.row = imax(0, cy - dd);
+  w.rows = imin(cy + dd, rp.g.max_y - 1) - w.row;
+  return w;
+}
+
+// The neighbour sums of the bird `qid` at (qx, qy) over window w of birds[],
+// which ends in an entry with z = ~0u.
+template <class Find>
+KG_HD void near_walk(const RepDev& rp, int32_t col0, const NearWindow& w, float qx, float qy,
+                     uint32_t qid, const Find& find, const NearBird* birds,
+                     const NearHead* heads, NearAcc* acc) {
+  if (w.cols < 0 || w.rows < 0) return;
+  const uint32_t key = ((uint32_t)w.c << kNearRowBits) + (uint32_t)w.row;
+  const uint32_t rows = (uint32_t)w.rows;
+  if (rp.disc_dist == 1) {
+    // one loop over the three columns' runs: a wave's trips are those of its
+    // busiest lane, not of each column's
+    uint32_t lo[3];
+    find.three(w.c, w.cols, w.row, lo);
+    uint32_t e = lo[0], last = key + rows;
     for (int32_t q = 0;;) {
       const NearBird b = birds[e];
       const NearHead h = heads[e];
@@ -276,23 +320,57 @@ KG_HD void near_walk(const RepDev& rp, int32_t col0, float qx, float qy, uint32_
         near_candidate(rp, col0, qx, qy, qid, b, h, acc);
         ++e;
       } else {
-        if (++q > cols) break;
+        if (++q > w.cols) break;
         e = q == 1 ? lo[1] : lo[2];
-        last = (q == 1 ? key[1] : key[2]) + rows;
+        last += 1u << kNearRowBits;
       }
     }
     return;
   }
-  for (int32_t cc = min_c; cc <= max_c; ++cc) {
-    const uint32_t key = ((uint32_t)cc << kNearRowBits) + (uint32_t)min_j;
-    uint32_t e = near_lower(birds, (uint32_t)col_base[cc] - base,
-                            (uint32_t)col_base[cc + 1] - base, key);
-    for (;; ++e) {
+  for (int32_t q = 0; q <= w.cols; ++q) {
+    const uint32_t last = key + ((uint32_t)q << kNearRowBits) + rows;
+    for (uint32_t e = find.one(w.c + q, w.row);; ++e) {
       const NearBird b = birds[e];
-      if (b.z > key + rows) break;
+      if (b.z > last) break;
       near_candidate(rp, col0, qx, qy, qid, b, heads[e], acc);
     }
   }
+}
+
+// Whether the window holds any bird the query returns (near_walk skips those
+// with the own id): for a bird that does not find itself.
+template <class Find>
+KG_HD bool near_any(const RepDev& rp, int32_t col0, const NearWindow& w, float qx, float qy,
+                    const Find& find, const NearBird* birds) {
+  for (int32_t q = 0; q <= w.cols && w.rows >= 0; ++q) {
+    const uint32_t last =
+        ((uint32_t)(w.c + q) << kNearRowBits) + (uint32_t)w.row + (uint32_t)w.rows;
+    for (uint32_t e = find.one(w.c + q, w.row); birds[e].z <= last; ++e) {
+      const float dx = qx - birds[e].x, dy = qy - birds[e].y;
+      const float s = dx * dx + dy * dy;
+      const bool in = s <= rp.sq_thresh;
+      const int32_t by = (int32_t)(birds[e].z & ((1u << kNearRowBits) - 1u));
+      const bool flip = s > rp.sq_sure && s <= rp.sq_near &&
+                        near_corners(rp.g, col0 + w.c + q, by, qx, qy, rp.sq_thresh, in ? -1 : 1);
+      if (in != flip) return true;
+    }
+  }
+  return false;
+}
+
+// Bird::step of bird b with heading h, relative column c and row cy.
+template <class Find>
+KG_HD void near_step(const RepDev& rp, int32_t col0, uint64_t step, const NearBird& b,
+                     const NearHead& h, const Find& find, const NearBird* birds,
+                     const NearHead* heads, float* nx, float* ny, float* nhx, float* nhy) {
+  const int32_t c = (int32_t)(b.z >> kNearRowBits);
+  const int32_t cy = (int32_t)(b.z & ((1u << kNearRowBits) - 1u));
+  const NearWindow w = near_window(rp, col0, c, cy);
+  NearAcc acc;
+  near_walk(rp, col0, w, b.x, b.y, b.id, find, birds, heads, &acc);
+  bool found = acc.n != 0 || near_self(rp, b.x, b.y, col0 + c, cy);
+  if (!found) found = near_any(rp, col0, w, b.x, b.y, find, birds);
+  near_finish(acc, found, rp.p, b.id, step, b.x, b.y, h.hx, h.hy, rp.g.w, nx, ny, nhx, nhy);
 }
 
 // ---- staging a tile ---------------------------------------------------------
@@ -394,8 +472,8 @@ KG_HD bool near_stage(const RepDev& rp, const FlockTile& ft, const NearChunk& k,
   const float x = R.x[gi], y = R.y[gi];
   const float hx = R.hx[gi], hy = R.hy[gi];
   const uint32_t id = R.id[gi];
-  const int32_t c = disc_axis(x, g.d, g.inv_d) - ft.sc_lo;
-  const int32_t cy = disc_axis(y, g.d, g.inv_d);
+  const int32_t c = cell_axis(g, x) - ft.sc_lo;
+  const int32_t cy = cell_axis(g, y);
   if (mine) {
     slot = S.col_base[c] - k.base + S.seg_len[3 * c] + (gi - S.seg_start[3 * c + 1]);
     S.own[i] = (uint16_t)slot;
@@ -418,14 +496,9 @@ KG_HD void near_agent(const RepDev& rp, const FlockTile& ft, const NearChunk& k,
                       const NearSmem& S, Buf W, uint32_t* count_next, uint32_t* err,
                       const FlockSinks& lv) {
   const uint32_t slot = S.own[o];
-  const NearBird b = S.bird[slot];
-  const NearHead h = S.head[slot];
-  NearAcc acc;
-  near_walk(rp, ft.sc_lo, b.x, b.y, b.id, (int32_t)(b.z >> kNearRowBits),
-            (int32_t)(b.z & ((1u << kNearRowBits) - 1u)), S.col_base, k.base, S.bird, S.head,
-            &acc);
   float nx, ny, nhx, nhy;
-  near_finish(acc, rp.p, b.id, ft.step, b.x, b.y, h.hx, h.hy, rp.g.w, &nx, &ny, &nhx, &nhy);
+  near_step(rp, ft.sc_lo, ft.step, S.bird[slot], S.head[slot],
+            TileFind{S.bird, S.col_base, k.base}, S.bird, S.head, &nx, &ny, &nhx, &nhy);
   flock_emit(rp.g, rp.bin_base, W, k.own_lo + o, nx, ny, nhx, nhy, count_next, err, ft.tile, lv);
 }
 

@@ -171,8 +171,8 @@ KG_HD uint32_t gather_src(const Outbox& ob, const uint32_t* sitem, const uint32_
 // The tile-local bin of a bird at (x, y) if it lies in local tile `tile`,
 // else kGatherMaxBins; *cy: its cell row.
 KG_HD uint32_t gather_bin(const Geom& g, uint32_t tile, float x, float y, int32_t* cy) {
-  int32_t cx;
-  discretize(g, x, y, &cx, cy);
+  const int32_t cx = cell_axis(g, x);
+  *cy = cell_axis(g, y);
   if (!cell_valid(g, cx, *cy)) return kGatherMaxBins;
   const uint32_t nb = bin_of(g, cx, *cy);
   if ((nb >> (g.tx_log2 + g.tr_log2)) != tile) return kGatherMaxBins;
@@ -234,7 +234,7 @@ KG_HD void scatter_aligned_one(const RepDev& rp, Buf R, Buf W, uint32_t i, uint3
 // ascending id -- the canonical bag order -- and a query walks the run.
 
 KG_HD uint64_t bin_key(const Geom& g, float y, uint32_t id) {
-  return ((uint64_t)(uint32_t)disc_axis(y, g.d, g.inv_d) << 32) | id;
+  return ((uint64_t)(uint32_t)cell_axis(g, y) << 32) | id;
 }
 
 // Bins of at most kSortSmall entries are sorted by one lane: keys in
@@ -491,8 +491,8 @@ KG_HD void flock_emit(const Geom& g, uint32_t bin_base, Buf W, uint32_t gi, floa
   W.y[gi] = ny;
   W.hx[gi] = nhx;
   W.hy[gi] = nhy;
-  int32_t cx, cy;
-  discretize(g, nx, ny, &cx, &cy);
+  // a step's position is in [0, width] or NaN
+  const int32_t cx = cell_axis(g, nx), cy = cell_axis(g, ny);
   if (!cell_valid(g, cx, cy)) {
     atom_or(err, 1u);
     return;

@@ -18,7 +18,7 @@ struct RepDev {
   int32_t disc_dist;   // floor(p.radius / g.d)
   int32_t lds_ok;      // the LDS tile path applies (toroidal, window fits one tile of halo)
   int32_t near;        // the near form applies (kg_near.hpp; implies lds_ok)
-  int32_t far;         // near form: all corners of a window cell may lie beyond the radius
+  float sq_sure;       // near form: a bird within it is returned whatever its cell's corners
   float sq_near;       // near form: no bird past it lies in a cell whose corners are within it
   uint32_t bin_base;   // first global bin of this replica
   uint32_t app_base;   // first append-buffer entry of this replica
