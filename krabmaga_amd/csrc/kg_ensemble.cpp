@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "kg_common.hpp"
+#include "kg_resident.hpp"
 #include "kg_rt_state.hpp"
 
 using namespace kg;
@@ -41,6 +42,7 @@ struct EnsRun {
   uint64_t steps_done = 0;  // schedule steps completed
   bool fresh = true;        // initial state not generated yet
   bool dead = false;        // retired; dropped at the next build
+  uint32_t res_bins = 0;    // bin table of the resident step, 0: the run does not fit it
   uint32_t app_base = 0;    // slot in the append buffer of the current layout
   uint32_t tile0 = 0, ntiles = 0;
 };
@@ -80,6 +82,15 @@ bool run_geom(const kg_run_desc& d, const kg_tuning& tu, Geom* g, RepDev* rep, s
   return true;
 }
 
+// The bin table of the resident step for this run, or 0 if it does not fit.
+uint32_t resident_bins(const EnsRun& r, size_t lds) {
+  RepDev rp{};
+  rp.g = r.g;
+  set_rep_params(&rp, r.desc.params);
+  uint32_t bins = 0;
+  return res_fits(rp, r.desc.agents, lds, &bins) ? bins : 0u;
+}
+
 }  // namespace
 
 struct kg_ensemble {
@@ -98,7 +109,8 @@ struct kg_ensemble {
   ScanState ss{};
   size_t cap_bins = 0, cap_scan = 0;
   RepDev* d_reps = nullptr;
-  uint32_t* d_prefix = nullptr;  // tile prefix (nreps + 1), then append prefix (nreps + 1)
+  // tile prefix (nreps + 1), append prefix (nreps + 1), runs by falling size (nreps)
+  uint32_t* d_prefix = nullptr;
   uint32_t* rep_cursor = nullptr;
   size_t cap_reps = 0;
   uint32_t* tcount = nullptr;
@@ -108,6 +120,7 @@ struct kg_ensemble {
   // bin-grouped form: the second read buffer, the write buffer, the next
   // bin offsets, the per-tile global-path flags and the step counter
   bool binned = false;  // the layout's form
+  bool binned_ready = false;  // the buffers of the three-kernel steps are there
   int want = -1;        // requested form: -1 by run size, 0 tile-resident, 1 bin-grouped
   DevBuf R2, W;
   size_t cap_r2 = 0, cap_w = 0;
@@ -246,7 +259,7 @@ int reserve(kg_ensemble* e, size_t bins, size_t reps, size_t tiles) {
     e->d_prefix = e->rep_cursor = nullptr;
     e->cap_reps = 0;
     if ((err = dmalloc(&e->d_reps, n)) != hipSuccess ||
-        (err = dmalloc(&e->d_prefix, 2 * (n + 1))) != hipSuccess ||
+        (err = dmalloc(&e->d_prefix, 3 * (n + 1))) != hipSuccess ||
         (err = dmalloc(&e->rep_cursor, n)) != hipSuccess)
       return set_error(KG_E_NOMEM, "ensemble replica tables: %s", hipGetErrorString(err));
     e->cap_reps = n;
@@ -300,6 +313,7 @@ bool shrink_crowded(kg_ensemble* e, const std::vector<uint32_t>& counts) {
     set_rep_params(&probe, r.desc.params);
     if (!probe.lds_ok) continue;
     r.g = g;
+    r.res_bins = resident_bins(r, e->lds_limit);
     any = true;
   }
   return any;
@@ -309,8 +323,21 @@ bool shrink_crowded(kg_ensemble* e, const std::vector<uint32_t>& counts) {
 // (the single-field crossover of the two paths lies between 16k and 64k).
 constexpr uint64_t kBinnedMeanAgents = 32768;
 
+// Every live run fits the resident step, and no form was asked for.
+bool want_resident(const kg_ensemble* e) {
+  if (e->want >= 0) return false;
+  bool any = false;
+  for (const EnsRun& r : e->runs) {
+    if (r.dead) continue;
+    if (!r.res_bins) return false;
+    any = true;
+  }
+  return any;
+}
+
 bool want_binned(const kg_ensemble* e) {
   if (e->want >= 0) return e->want == 1;
+  if (want_resident(e)) return true;  // it steps the bin-grouped layout
   uint64_t agents = 0, live = 0;
   for (const EnsRun& r : e->runs)
     if (!r.dead) {
@@ -328,8 +355,6 @@ int reserve_binned(kg_ensemble* e, size_t agents, size_t tiles) {
   hipError_t err;
   if ((err = regrow(&e->gflag, &e->cap_gflag, tiles + 2)) != hipSuccess)
     return set_error(KG_E_NOMEM, "ensemble bin-grouped buffers: %s", hipGetErrorString(err));
-  if (!e->gstep && (err = dmalloc(&e->gstep, 1)) != hipSuccess)
-    return set_error(KG_E_NOMEM, "ensemble step counter: %s", hipGetErrorString(err));
   if (tiles > e->cap_outbox) {
     (void)hipFree(e->outbox.n);
     (void)hipFree(e->outbox.slot);
@@ -418,7 +443,7 @@ int rebuild(kg_ensemble* e) {
     // replica table
     const uint32_t nreps = (uint32_t)e->runs.size();
     e->h_reps.assign(nreps, RepDev{});
-    e->h_prefix.assign(2 * (nreps + 1), 0u);
+    e->h_prefix.assign(3 * (nreps + 1), 0u);
     std::vector<RtRepInfo> infos(nreps);
     uint32_t bin_base = 0, tile0 = 0, boff_base = 0;
     for (uint32_t i = 0; i < nreps; ++i) {
@@ -445,6 +470,11 @@ int rebuild(kg_ensemble* e) {
     }
     e->h_prefix[nreps] = tile0;
     e->h_prefix[2 * nreps + 1] = base;
+    uint32_t* const by_size = e->h_prefix.data() + 2 * (nreps + 1);
+    for (uint32_t i = 0; i < nreps; ++i) by_size[i] = i;
+    std::stable_sort(by_size, by_size + nreps, [&](uint32_t a, uint32_t b) {
+      return e->runs[a].desc.agents > e->runs[b].desc.agents;
+    });
     e->nreps = nreps;
     e->ntiles = tile0;
     e->nbins = nreps ? e->h_reps[nreps - 1].bin_base + e->runs[nreps - 1].g.nbins : 0;
@@ -497,25 +527,16 @@ int rebuild(kg_ensemble* e) {
   e->binned = binned;
   if (binned) {
     // every bin into (cell y, id) order, the consumed build buffer as scratch
-    if (int rc = reserve_binned(e, std::max<uint64_t>(agents, 1), e->ntiles)) return rc;
     KG_HIP(launch_sort_bins(w, e->R.b, e->offset, e->A2.b, e->stream));
-    KG_HIP(hipMemsetAsync(e->gstep, 0, sizeof(uint64_t), e->stream));
-    int cap = 256;
-    for (const EnsRun& r : e->runs) cap = std::max(cap, pick_lds_cap(r.g, r.desc.agents));
-    e->lds_cap = clamp_lds_cap(cap);
-    int cols = 1;
-    bool near = true;
-    for (const RepDev& rp : e->h_reps) {
-      cols = std::max(cols, std::min(kMaxStageCols, rp.g.tx + 2 * rp.disc_dist));
-      near = near && rp.near;
+    if (!e->gstep) {
+      const hipError_t err = dmalloc(&e->gstep, 1);
+      if (err != hipSuccess)
+        return set_error(KG_E_NOMEM, "ensemble step counter: %s", hipGetErrorString(err));
     }
-    e->near = near ? near_plan(cap, cols, e->ntiles) : NearPlan{};
+    KG_HIP(hipMemsetAsync(e->gstep, 0, sizeof(uint64_t), e->stream));
+    e->binned_ready = false;
+    e->gather = false;
     e->parity = 0;
-    e->gather = rebin_gather_enabled();
-    for (const RepDev& rp : e->h_reps)
-      if ((uint32_t)(rp.g.tx * rp.g.tr) > kGatherMaxBins) e->gather = false;
-    KG_HIP(hipMemsetAsync(e->gate, 0, 4 * sizeof(uint32_t), e->stream));
-    e->redone_seen = 0;
   } else {
     if (int rc = e->rt.setup(plan, cls, e->nagents, e->stream)) return rc;
     if (int rc = e->rt.reset(G, e->stream)) return rc;
@@ -527,6 +548,46 @@ int rebuild(kg_ensemble* e) {
   }
   for (EnsRun& r : e->runs) r.fresh = false;
   ++e->builds;
+  return KG_OK;
+}
+
+// The three-kernel steps' buffers and plan for a bin-grouped layout (a layout
+// that only takes resident steps needs none of them).
+int ready_binned(kg_ensemble* e) {
+  if (e->binned_ready) return KG_OK;
+  if (int rc = reserve_binned(e, std::max<uint32_t>(e->nagents, 1u), e->ntiles)) return rc;
+  int cap = 256;
+  for (const EnsRun& r : e->runs) cap = std::max(cap, pick_lds_cap(r.g, r.desc.agents));
+  e->lds_cap = clamp_lds_cap(cap);
+  int cols = 1;
+  bool near = true;
+  for (const RepDev& rp : e->h_reps) {
+    cols = std::max(cols, std::min(kMaxStageCols, rp.g.tx + 2 * rp.disc_dist));
+    near = near && rp.near;
+  }
+  e->near = near ? near_plan(cap, cols, e->ntiles) : NearPlan{};
+  e->gather = rebin_gather_enabled();
+  for (const RepDev& rp : e->h_reps)
+    if ((uint32_t)(rp.g.tx * rp.g.tr) > kGatherMaxBins) e->gather = false;
+  KG_HIP(hipMemsetAsync(e->gate, 0, 4 * sizeof(uint32_t), e->stream));
+  e->redone_seen = 0;
+  e->binned_ready = true;
+  return KG_OK;
+}
+
+// `n` (<= kResidentSteps) steps of every run in its own work-group.
+int resident_steps(kg_ensemble* e, uint32_t n) {
+  uint32_t cap = 1, bins = 1;
+  for (const EnsRun& r : e->runs) {
+    if (r.dead) continue;
+    cap = std::max(cap, r.desc.agents);
+    bins = std::max(bins, r.res_bins);
+  }
+  KG_HIP(launch_resident(e->d_reps, e->d_prefix + 2 * (e->nreps + 1), e->nreps, e->R.b,
+                         e->offset, e->gstep, 0, n, e->err, cap, bins, e->stream));
+  KG_HIP(launch_add_u64(e->gstep, n, e->stream));
+  e->steps_run += n;
+  for (EnsRun& r : e->runs) r.steps_done += n;
   return KG_OK;
 }
 
@@ -595,6 +656,7 @@ hipError_t binned_step(kg_ensemble* e, const WorkList& w) {
 // `n` bin-grouped steps (graph replays of two steps when allowed: the
 // buffers are back in place after two).
 int binned_steps(kg_ensemble* e, uint32_t n, bool use_graph) {
+  if (int rc = ready_binned(e)) return rc;
   const WorkList w = e->wl();
   uint32_t left = n;
   // every gathered step is summed: the sums and both gate flags start at
@@ -694,6 +756,8 @@ int check_flags(kg_ensemble* e) {
     KG_HIP(hipMemcpy(&errflag, e->err, sizeof(errflag), hipMemcpyDeviceToHost));
     if (errflag & 2u)
       return set_error(KG_E_HIP, "the rebinning fallback's grid-wide wait timed out");
+    if (errflag & 4u)
+      return set_error(KG_E_STATE, "the resident step found more birds than it was planned for");
     if (errflag) return set_error(KG_E_RANGE, "an agent left its run's bag grid");
     if (e->gather) {
       // steps the gather could not rebin since the last check: a layout
@@ -795,6 +859,7 @@ int kg_ensemble_admit(kg_ensemble* e, const kg_run_desc* runs, uint32_t n, uint3
     if (!run_geom(runs[i], e->tuning, &add[i].g, nullptr, &why))
       return set_error(KG_E_INVALID, "run %u: %s", i, why.c_str());
     add[i].desc = runs[i];
+    add[i].res_bins = resident_bins(add[i], e->lds_limit);
   }
   for (uint32_t i = 0; i < n; ++i) {
     add[i].id = e->next_id++;
@@ -839,9 +904,13 @@ int kg_ensemble_run(kg_ensemble* e, uint32_t nsteps, int flags) {
     if (int rc = rebuild(e)) return rc;
   if (e->nreps == 0) return KG_OK;
   const bool graph = (flags & KG_RUN_GRAPH) != 0;
+  const bool resident = e->binned && want_resident(e);
   while (nsteps > 0) {
-    const uint32_t chunk = std::min(nsteps, kRtCheckEvery);
-    if (int rc = e->binned ? binned_steps(e, chunk, graph) : steps(e, chunk, graph)) return rc;
+    const uint32_t chunk = std::min(nsteps, resident ? kResidentSteps : kRtCheckEvery);
+    if (int rc = resident    ? resident_steps(e, chunk)
+                 : e->binned ? binned_steps(e, chunk, graph)
+                             : steps(e, chunk, graph))
+      return rc;
     nsteps -= chunk;
     if (int rc = check_flags(e)) return rc;
     if (e->replan)

@@ -17,6 +17,7 @@
 #include <map>
 #include <vector>
 
+#include "kg_resident.hpp"
 #include "kg_rt_state.hpp"
 
 using namespace kg;
@@ -178,6 +179,8 @@ int check_poison(kg_field* f) {
     return set_error(KG_E_HIP,
                      "the rebinning fallback's grid-wide wait timed out in an earlier step; "
                      "the field is unusable");
+  if (f->poisoned && (f->poison_bits & 4u))
+    return set_error(KG_E_STATE, "the resident step found more birds than it was planned for");
   if (f->poisoned)
     return set_error(KG_E_RANGE,
                      "a location fell outside the bag grid in an earlier step; the field is "
@@ -1001,6 +1004,21 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
   {
     RepDev probe = f->h_rep;
     set_rep_params(&probe, *p);
+    // by default a field that fits one work-group's LDS steps there, many
+    // steps to a launch
+    uint32_t bins = 0;
+    if (!(use_graph & (KG_RUN_BINNED | KG_RUN_TILE_RESIDENT)) &&
+        res_fits(probe, f->nR, f->lds_limit, &bins)) {
+      if (int rc = ensure_atomic(f)) return rc;
+      if (int rc = set_params(f, p, first_step)) return rc;
+      for (uint32_t k = 0; k < nsteps; k += kResidentSteps) {
+        ProfScope ps(f, KG_KERNEL_RT_STEP);
+        KG_HIP(launch_resident(f->d_rep, nullptr, 1, f->R.b, f->offset, f->zero64, k,
+                               std::min(kResidentSteps, nsteps - k), f->err, f->nR, bins,
+                               f->stream));
+      }
+      return KG_OK;
+    }
     // by default small fields take the one-launch tile-resident step (fewer
     // launches per step) and large ones the three-kernel path (more of its
     // work-groups fit a CU): measured at constant density on MI355X, the two

@@ -78,6 +78,16 @@ hipError_t launch_flock(const WorkList& wl, Buf R, const uint32_t* offset, Buf W
                         const NearPlan& near = NearPlan{});
 hipError_t launch_materialize(Buf R, Buf W, uint32_t n, Buf A, hipStream_t s);
 
+// nsteps (<= kResidentSteps) schedule steps of runs list[0 .. nruns) (or runs
+// 0 .. nruns), one work-group each, in place in R and offset (kg_resident.hpp):
+// step_base + *gstep + koff is the first.  cap: the largest run's agents (<=
+// kResidentMaxAgents), bins: the largest res_fits bin table.  Sets bit 2 of
+// err for a run past them.
+hipError_t launch_resident(const RepDev* reps, const uint32_t* list, uint32_t nruns, Buf R,
+                           uint32_t* offset, const uint64_t* gstep, uint32_t koff,
+                           uint32_t nsteps, uint32_t* err, uint32_t cap, uint32_t bins,
+                           hipStream_t s);
+
 // Tile-resident step (one launch per schedule step); with load != 0 the
 // launch instead moves the bin-grouped read buffer (Ra, offset_a) into the
 // tile-resident layout that step `load_g + 1` reads.

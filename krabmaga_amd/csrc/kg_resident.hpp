@@ -1,0 +1,135 @@
+// kg_resident.hpp -- a whole small field in one work-group's LDS, many
+// schedule steps to a launch.
+//
+// A field of a few thousand birds is far too little work for a launch per
+// step: the tile kernels spend it on launch gaps and on one work-group's
+// chain of global loads.  Here one work-group keeps every bird of a run in
+// LDS for up to kResidentSteps schedule steps.  Each thread owns up to kB
+// birds.  A step is: every thread walks its birds' windows in LDS into
+// registers; then all birds are counted into bins (runs of 1 << shift rows
+// of one column), the counts become starts, each bird's key (row, id) is
+// ranked inside its bin, and the birds go back to LDS in bag-scan order.
+// The last step's order is the read buffer's (tile by tile), so birds and
+// bin offsets are written back as the other paths leave them.
+//
+// The neighbour sums take the near form (kg_near.hpp) while every bird is
+// near, and full_step, the general form, in any step where one is not.
+#pragma once
+
+#include "kg_near.hpp"
+
+namespace kg {
+
+// Steps per launch: a bound on how long one launch can run (a step of the
+// largest field takes about 30 us).
+constexpr uint32_t kResidentSteps = 256;
+constexpr uint32_t kResidentMaxAgents = 4096;
+// z holds 12 bits of column here
+constexpr int32_t kResidentMaxCols = 4095;
+constexpr int32_t kResidentMaxRows = 1 << kNearRowBits;
+
+// LDS of a run of up to `cap` birds and `bins` bins.
+struct ResSmem {
+  NearBird* bird;  // cap + 1; also the keys while birds are in registers
+  NearHead* head;  // cap + 1
+  uint32_t* tab;   // bins + 1
+};
+
+KG_HD size_t res_smem_bytes(uint32_t cap, uint32_t bins) {
+  return (size_t)(cap + 1) * (sizeof(NearBird) + sizeof(NearHead)) +
+         (size_t)(bins + 1) * sizeof(uint32_t);
+}
+
+KG_HD ResSmem res_carve(uint8_t* p, uint32_t cap) {
+  ResSmem s;
+  s.bird = (NearBird*)p;
+  s.head = (NearHead*)(s.bird + cap + 1);
+  s.tab = (uint32_t*)(s.head + cap + 1);
+  return s;
+}
+
+// The field's own bins in LDS: columns of bins of 1 << shift rows, at most
+// `bins` of them.
+struct ResBins {
+  int32_t rows, shift;  // bins per column
+  uint32_t n;
+};
+
+KG_HD ResBins res_bins(const Geom& g, uint32_t bins) {
+  ResBins b;
+  b.shift = 0;
+  while ((uint64_t)g.dw * (uint64_t)(((g.dh - 1) >> b.shift) + 1) > bins) ++b.shift;
+  b.rows = ((g.dh - 1) >> b.shift) + 1;
+  b.n = (uint32_t)(g.dw * b.rows);
+  return b;
+}
+
+// Whether a run fits: `bins` receives the bin table it needs (at least the
+// read buffer's bins, for the write-back, and one bin per column).
+KG_HD bool res_fits(const RepDev& rp, uint32_t agents, size_t lds, uint32_t* bins) {
+  const Geom& g = rp.g;
+  if (!rp.lds_ok || agents == 0 || agents > kResidentMaxAgents || g.dw > kResidentMaxCols ||
+      g.dh > kResidentMaxRows)
+    return false;
+  uint32_t b = agents > 1024u ? agents : 1024u;
+  if (b < g.nbins) b = g.nbins;
+  if (b < (uint32_t)g.dw) b = (uint32_t)g.dw;
+  *bins = b;
+  return res_smem_bytes(agents, b) <= lds;
+}
+
+// A bird between its walk and its place in LDS.
+struct ResBird {
+  float x, y, hx, hy;
+  uint32_t id, z, bin, slot;
+};
+
+// Cell and bin of a bird; api: the read buffer's bins instead of the field's
+// own.  A bird outside the grid is reported and kept in cell 0.
+KG_HD void res_place(const RepDev& rp, const ResBins& rb, bool api, ResBird* b, uint32_t* err) {
+  const Geom& g = rp.g;
+  int32_t cx = cell_axis(g, b->x), cy = cell_axis(g, b->y);
+  if (!cell_valid(g, cx, cy)) {
+    atom_or(err, 1u);
+    cx = cy = 0;
+  }
+  b->z = ((uint32_t)cx << kNearRowBits) | (uint32_t)cy;
+  b->bin = api ? bin_of(g, cx, cy) : (uint32_t)(cx * rb.rows + (cy >> rb.shift));
+}
+
+KG_HD uint64_t res_key(const ResBird& b) {
+  return ((uint64_t)(b.z & ((1u << kNearRowBits) - 1u)) << 32) | b.id;
+}
+
+// Bird::step in the general form (any toroidal field whose windows fit) from
+// the same LDS layout.
+template <class Find>
+KG_HD void full_step(const RepDev& rp, uint64_t step, const NearBird& b, const NearHead& h,
+                     const Find& find, const NearBird* birds, const NearHead* heads, float* nx,
+                     float* ny, float* nhx, float* nhy) {
+  const Geom& g = rp.g;
+  const float T = rp.sq_thresh;
+  const NearWindow w = near_window(rp, 0, (int32_t)(b.z >> kNearRowBits),
+                                   (int32_t)(b.z & ((1u << kNearRowBits) - 1u)));
+  FlockAcc acc;
+  for (int32_t q = 0; q <= w.cols && w.rows >= 0; ++q) {
+    const uint32_t key = ((uint32_t)(w.c + q) << kNearRowBits) + (uint32_t)w.row;
+    int32_t cur = -1;
+    int chk = 0;
+    for (uint32_t e = find.one(w.c + q, w.row); birds[e].z <= key + (uint32_t)w.rows; ++e) {
+      const int32_t row = (int32_t)(birds[e].z & ((1u << kNearRowBits) - 1u));
+      if (row != cur) {
+        cur = row;
+        chk = check_circle_sq(g, w.c + q, row, b.x, b.y, T);
+      }
+      if (chk == -1) continue;
+      const float dx = toroidal_distance(b.x, birds[e].x, g.w);
+      const float dy = toroidal_distance(b.y, birds[e].y, g.h);
+      if (chk == 1 || dx * dx + dy * dy <= T)
+        acc.add(birds[e].id == b.id, dx, dy, heads[e].hx, heads[e].hy);
+    }
+  }
+  flock_finish(acc, rp.p, b.id, step, b.x, b.y, h.hx, h.hy, g.w, nx, ny, nhx, nhy);
+}
+
+}  // namespace kg
