@@ -1025,7 +1025,8 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
     // cross between 16k and 64k birds
     constexpr uint32_t kRtDefaultMaxAgents = 32768;
     const bool want_rt = (use_graph & KG_RUN_TILE_RESIDENT) ||
-                         (!(use_graph & KG_RUN_BINNED) && f->nR < kRtDefaultMaxAgents);
+                         (!(use_graph & KG_RUN_BINNED) && !probe.near &&
+                          f->nR < kRtDefaultMaxAgents);
     if (want_rt && probe.lds_ok) {
       // tile-resident path: the class launches of each step; the capacity
       // flags are read every kRtCheckEvery steps (32 measured ~1.5 % faster

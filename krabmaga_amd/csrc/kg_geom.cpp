@@ -414,6 +414,9 @@ bool make_geom_rt(float w, float h, float d, int tor, uint64_t expected_agents, 
   if (!hb) {
     hb = 1u << g->hb_log2;
     while (hb > ty) hb >>= 1;
+    // a tile of more bins than that cannot be rebinned by gather (the bins'
+    // height does not change the order of the birds)
+    while (hb < ty && tx * (ty / hb) > kGatherMaxBins) hb <<= 1;
   }
   if ((tx & (tx - 1)) || (ty & (ty - 1)) || (hb & (hb - 1)) || hb > ty || tx > 128) {
     *why = "tile sizes must be powers of two with bin rows <= tile rows and tile columns <= 128";

@@ -668,7 +668,7 @@ __global__ __launch_bounds__(kT, 8) void k_flock_near(
     const NearChunk k = near_chunk(rp, ft, S, oa, ob2);
     for (uint32_t i = t; i < k.n; i += kT)
       if (!near_stage(rp, ft, k, i, R, S)) s_bad = 1u;
-    if (t == 0) S.bird[k.n].z = ~0u;
+    if (t == 0) S.b.z[k.n] = ~0u;
     __syncthreads();
     use_lds = s_bad == 0u;
     if (use_lds)

@@ -18,7 +18,7 @@
 // 2^-60, a heading above 2^60 or a NaN is not near (near_bad); the caller
 // takes the general form for it.
 //
-// The walk reads a list of birds in LDS (or any memory) sorted by z =
+// The walk reads a list of birds in LDS sorted by z =
 // column << kNearRowBits | row, then id: the reference's bag-scan order, in
 // which the rows of one window column are one contiguous run.
 #pragma once
@@ -29,13 +29,31 @@ namespace kg {
 
 constexpr int kNearRowBits = 20;
 
-struct alignas(16) NearBird {
-  float x, y;
-  uint32_t z, id;
+struct alignas(16) NearRec {
+  float x, y, hx, hy;
 };
-struct alignas(8) NearHead {
-  float hx, hy;
+
+// Birds in scan order: bird e is rec[e] with key z[e] and id id[e]; one entry
+// past the last has z = ~0u (its record is read, never used).
+struct NearBirds {
+  NearRec* rec;
+  uint32_t* z;
+  uint32_t* id;
 };
+
+KG_HD size_t near_birds_bytes(uint32_t n) {
+  return (size_t)(n + 1) * (sizeof(NearRec) + 2 * sizeof(uint32_t));
+}
+
+// Birds [0, n] at p (16-byte aligned); *end: the first byte after them.
+KG_HD NearBirds near_birds_at(uint8_t* p, uint32_t n, uint8_t** end) {
+  NearBirds b;
+  b.rec = (NearRec*)p;
+  b.z = (uint32_t*)(b.rec + n + 1);
+  b.id = b.z + n + 1;
+  *end = (uint8_t*)(b.id + n + 1);
+  return b;
+}
 
 KG_HD uint32_t f_bits(float v) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -105,19 +123,19 @@ KG_HD bool near_corners(const Geom& g, int32_t bx, int32_t by, float lx, float l
   return fminf(ax * ax, bx2 * bx2) + fminf(ay * ay, by2 * by2) > T;
 }
 
-// One candidate of the bird `qid` at (qx, qy): c (its column relative to
-// col0) and its heading.
+// Candidate e of the bird `qid` at (qx, qy).
 KG_HD void near_candidate(const RepDev& rp, int32_t col0, float qx, float qy, uint32_t qid,
-                          const NearBird& c, const NearHead& h, NearAcc* acc) {
+                          const NearBirds& B, uint32_t e, const NearRec& c, uint32_t cid,
+                          NearAcc* acc) {
   const float dx = qx - c.x, dy = qy - c.y;
   const float s = dx * dx + dy * dy;
   bool ok = s <= rp.sq_thresh;
   if (s > rp.sq_sure && s <= rp.sq_near) {  // rare: the corners decide
-    const int32_t bx = col0 + (int32_t)(c.z >> kNearRowBits);
-    const int32_t by = (int32_t)(c.z & ((1u << kNearRowBits) - 1u));
+    const int32_t bx = col0 + (int32_t)(B.z[e] >> kNearRowBits);
+    const int32_t by = (int32_t)(B.z[e] & ((1u << kNearRowBits) - 1u));
     if (near_corners(rp.g, bx, by, qx, qy, rp.sq_thresh, ok ? -1 : 1)) ok = !ok;
   }
-  if (ok && c.id != qid) acc->add(dx, dy, s, h.hx, h.hy);
+  if (ok && cid != qid) acc->add(dx, dy, s, c.hx, c.hy);
 }
 
 // Whether the bird at (qx, qy) of cell (cx, cy) finds itself: its own bag is
@@ -214,33 +232,38 @@ KG_HD void near_finish(const NearAcc& a, bool found, const FlockParams& p, uint3
   *ny = vy >= width ? vy - width : (vy < 0.0f ? vy + width : vy);
 }
 
-// First entry of birds[lo, hi) (sorted by z) with z >= key.
-KG_HD uint32_t near_lower(const NearBird* birds, uint32_t lo, uint32_t hi, uint32_t key) {
+// First entry of z[lo, hi) at or after key.
+KG_HD uint32_t near_lower(const uint32_t* z, uint32_t lo, uint32_t hi, uint32_t key) {
   while (lo < hi) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (birds[mid].z < key) lo = mid + 1;
+    if (z[mid] < key) lo = mid + 1;
     else hi = mid;
   }
   return lo;
 }
 
-// Where a window column's run starts: the first entry of birds[] at or after
-// z = key = c << kNearRowBits | row, of one column or of three neighbouring
-// ones.
+// Where a window column's run lies: entries [lo, hi) have z in [key, key +
+// rows], key = c << kNearRowBits | row; of one column, or of up to three
+// neighbouring ones (those past `cols` are empty).
 //
-// TileFind: birds[] holds the staged columns of a tile, column c from
-// col_base[c] - base; bisected, three columns side by side (three LDS reads
-// in flight).
+// TileFind: the birds are the staged columns of a tile, column c from
+// col_base[c] - base; the starts of three columns bisected side by side
+// (three LDS reads in flight), the ends found by stepping from them (bisecting
+// the ends too cost more: a 1M-boid step 86.7 us against 77.6, on a field ten
+// times denser 103.8 against 96.6).
 struct TileFind {
-  const NearBird* birds;
+  const uint32_t* z;
   const uint32_t* col_base;
   uint32_t base;
 
-  KG_HD uint32_t one(int32_t c, int32_t row) const {
-    return near_lower(birds, col_base[c] - base, col_base[c + 1] - base,
-                      ((uint32_t)c << kNearRowBits) + (uint32_t)row);
+  KG_HD void one(int32_t c, int32_t row, uint32_t rows, uint32_t* lo, uint32_t* hi) const {
+    const uint32_t key = ((uint32_t)c << kNearRowBits) + (uint32_t)row;
+    const uint32_t end = col_base[c + 1] - base;
+    *lo = near_lower(z, col_base[c] - base, end, key);
+    *hi = near_lower(z, *lo, end, key + rows + 1u);
   }
-  KG_HD void three(int32_t c, int32_t cols, int32_t row, uint32_t* lo) const {
+  KG_HD void three(int32_t c, int32_t cols, int32_t row, uint32_t rows, uint32_t* lo,
+                   uint32_t* hi) const {
     uint32_t n[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -248,37 +271,62 @@ struct TileFind {
       n[q] = q <= cols ? col_base[c + q + 1] - base - lo[q] : 0u;
     }
     const uint32_t key = ((uint32_t)c << kNearRowBits) + (uint32_t)row;
+    // an empty range reads one entry at most past the last bird
     while (n[0] | n[1] | n[2]) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        const uint32_t half = n[q] >> 1;
-        const uint32_t mid = lo[q] + half;
-        const bool up = n[q] != 0u && birds[mid].z < key + ((uint32_t)q << kNearRowBits);
-        lo[q] = up ? mid + 1u : lo[q];
-        n[q] = up ? n[q] - half - 1u : half;
+        const uint32_t hn = n[q] >> 1;
+        const bool un = n[q] != 0u && z[lo[q] + hn] < key + ((uint32_t)q << kNearRowBits);
+        lo[q] = un ? lo[q] + hn + 1u : lo[q];
+        n[q] = un ? n[q] - hn - 1u : hn;
+      }
+    }
+    // the ends from there: a run is short
+    uint32_t last[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      hi[q] = lo[q];
+      last[q] = q <= cols ? key + ((uint32_t)q << kNearRowBits) + rows : 0u;
+    }
+    for (bool more = true; more;) {
+      more = false;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const bool in = (z[hi[q]] <= last[q]) & (q <= cols);  // both sides: no branch
+        hi[q] += in ? 1u : 0u;
+        more |= in;
       }
     }
   }
 };
 
-// CellFind: birds[] holds a whole field in bins of 1 << shift rows, column by
-// column, `rows` bins to a column, bin b from start[b].
+// CellFind: the birds are a whole field in bins of 1 << shift rows, column by
+// column, `per` bins to a column, bin b from start[b].
 struct CellFind {
-  const NearBird* birds;
+  const uint32_t* z;
   const uint32_t* start;
-  int32_t rows, shift;
+  int32_t per, shift;
 
-  KG_HD uint32_t one(int32_t c, int32_t row) const {
-    uint32_t e = start[c * rows + (row >> shift)];
-    if (shift) {
-      const uint32_t key = ((uint32_t)c << kNearRowBits) + (uint32_t)row;
-      while (birds[e].z < key) ++e;  // the last entry's z is ~0u
+  KG_HD void one(int32_t c, int32_t row, uint32_t rows, uint32_t* lo, uint32_t* hi) const {
+    const int32_t b0 = c * per + (row >> shift);
+    const int32_t b1 = c * per + ((row + (int32_t)rows) >> shift);
+    *lo = start[b0];
+    if (shift == 0) {
+      *hi = start[b1 + 1];
+      return;
     }
-    return e;
+    const uint32_t key = ((uint32_t)c << kNearRowBits) + (uint32_t)row;
+    while (z[*lo] < key) ++*lo;  // the last entry's z is ~0u
+    *hi = start[b1] > *lo ? start[b1] : *lo;
+    while (z[*hi] <= key + rows) ++*hi;
   }
-  KG_HD void three(int32_t c, int32_t cols, int32_t row, uint32_t* lo) const {
+  KG_HD void three(int32_t c, int32_t cols, int32_t row, uint32_t rows, uint32_t* lo,
+                   uint32_t* hi) const {
 #pragma unroll
-    for (int q = 0; q < 3; ++q) lo[q] = q <= cols ? one(c + q, row) : 0u;
+    for (int q = 0; q < 3; ++q) {
+      lo[q] = hi[q] = 0u;
+      if (q <= cols) one(c + q, row, rows, &lo[q], &hi[q]);
+    }
   }
 };
 
@@ -298,42 +346,52 @@ KG_HD NearWindow near_window(const RepDev& rp, int32_t col0, int32_t c, int32_t 
   return w;
 }
 
-// The neighbour sums of the bird `qid` at (qx, qy) over window w of birds[],
-// which ends in an entry with z = ~0u.
+// Entry of candidate k of three runs of n0, n1 - n0 and the rest, from o0, o1
+// + n0 and o2 + n1 (by value: two selects, no memory).
+KG_HD uint32_t near_at(uint32_t k, uint32_t n0, uint32_t n1, uint32_t o0, uint32_t o1,
+                       uint32_t o2) {
+  uint32_t o = k < n1 ? o1 : o2;
+  o = k < n0 ? o0 : o;
+  return k + o;
+}
+
+// The neighbour sums of the bird `qid` at (qx, qy) over window w.
 template <class Find>
 KG_HD void near_walk(const RepDev& rp, int32_t col0, const NearWindow& w, float qx, float qy,
-                     uint32_t qid, const Find& find, const NearBird* birds,
-                     const NearHead* heads, NearAcc* acc) {
+                     uint32_t qid, const Find& find, const NearBirds& B, NearAcc* acc) {
   if (w.cols < 0 || w.rows < 0) return;
-  const uint32_t key = ((uint32_t)w.c << kNearRowBits) + (uint32_t)w.row;
   const uint32_t rows = (uint32_t)w.rows;
   if (rp.disc_dist == 1) {
     // one loop over the three columns' runs: a wave's trips are those of its
-    // busiest lane, not of each column's
-    uint32_t lo[3];
-    find.three(w.c, w.cols, w.row, lo);
-    uint32_t e = lo[0], last = key + rows;
-    for (int32_t q = 0;;) {
-      const NearBird b = birds[e];
-      const NearHead h = heads[e];
-      if (b.z <= last) {
-        near_candidate(rp, col0, qx, qy, qid, b, h, acc);
-        ++e;
-      } else {
-        if (++q > w.cols) break;
-        e = q == 1 ? lo[1] : lo[2];
-        last += 1u << kNearRowBits;
-      }
+    // busiest lane, not of each column's.  The next candidate is loaded while
+    // this one is worked on.
+    uint32_t lo[3], hi[3];
+    find.three(w.c, w.cols, w.row, rows, lo, hi);
+    const uint32_t n0 = hi[0] - lo[0], n1 = n0 + hi[1] - lo[1], n = n1 + hi[2] - lo[2];
+    const uint32_t o1 = lo[1] - n0, o2 = lo[2] - n1;
+    const uint32_t o0 = lo[0];
+    if (n == 0u) return;
+    uint32_t e = near_at(0u, n0, n1, o0, o1, o2);
+    NearRec c = B.rec[e];
+    uint32_t id = B.id[e];
+    for (uint32_t k = 1;; ++k) {
+      // past the last candidate this is at most the sentinel
+      const uint32_t en = near_at(k, n0, n1, o0, o1, o2);
+      const NearRec cn = B.rec[en];
+      const uint32_t idn = B.id[en];
+      near_candidate(rp, col0, qx, qy, qid, B, e, c, id, acc);
+      if (k == n) break;
+      e = en;
+      c = cn;
+      id = idn;
     }
     return;
   }
   for (int32_t q = 0; q <= w.cols; ++q) {
-    const uint32_t last = key + ((uint32_t)q << kNearRowBits) + rows;
-    for (uint32_t e = find.one(w.c + q, w.row);; ++e) {
-      const NearBird b = birds[e];
-      if (b.z > last) break;
-      near_candidate(rp, col0, qx, qy, qid, b, heads[e], acc);
-    }
+    uint32_t lo, hi;
+    find.one(w.c + q, w.row, rows, &lo, &hi);
+    for (uint32_t e = lo; e < hi; ++e)
+      near_candidate(rp, col0, qx, qy, qid, B, e, B.rec[e], B.id[e], acc);
   }
 }
 
@@ -341,15 +399,15 @@ KG_HD void near_walk(const RepDev& rp, int32_t col0, const NearWindow& w, float 
 // with the own id): for a bird that does not find itself.
 template <class Find>
 KG_HD bool near_any(const RepDev& rp, int32_t col0, const NearWindow& w, float qx, float qy,
-                    const Find& find, const NearBird* birds) {
+                    const Find& find, const NearBirds& B) {
   for (int32_t q = 0; q <= w.cols && w.rows >= 0; ++q) {
-    const uint32_t last =
-        ((uint32_t)(w.c + q) << kNearRowBits) + (uint32_t)w.row + (uint32_t)w.rows;
-    for (uint32_t e = find.one(w.c + q, w.row); birds[e].z <= last; ++e) {
-      const float dx = qx - birds[e].x, dy = qy - birds[e].y;
+    uint32_t lo, hi;
+    find.one(w.c + q, w.row, (uint32_t)w.rows, &lo, &hi);
+    for (uint32_t e = lo; e < hi; ++e) {
+      const float dx = qx - B.rec[e].x, dy = qy - B.rec[e].y;
       const float s = dx * dx + dy * dy;
       const bool in = s <= rp.sq_thresh;
-      const int32_t by = (int32_t)(birds[e].z & ((1u << kNearRowBits) - 1u));
+      const int32_t by = (int32_t)(B.z[e] & ((1u << kNearRowBits) - 1u));
       const bool flip = s > rp.sq_sure && s <= rp.sq_near &&
                         near_corners(rp.g, col0 + w.c + q, by, qx, qy, rp.sq_thresh, in ? -1 : 1);
       if (in != flip) return true;
@@ -358,19 +416,21 @@ KG_HD bool near_any(const RepDev& rp, int32_t col0, const NearWindow& w, float q
   return false;
 }
 
-// Bird::step of bird b with heading h, relative column c and row cy.
+// Bird::step of entry o.
 template <class Find>
-KG_HD void near_step(const RepDev& rp, int32_t col0, uint64_t step, const NearBird& b,
-                     const NearHead& h, const Find& find, const NearBird* birds,
-                     const NearHead* heads, float* nx, float* ny, float* nhx, float* nhy) {
-  const int32_t c = (int32_t)(b.z >> kNearRowBits);
-  const int32_t cy = (int32_t)(b.z & ((1u << kNearRowBits) - 1u));
+KG_HD void near_step(const RepDev& rp, int32_t col0, uint64_t step, uint32_t o, const Find& find,
+                     const NearBirds& B, NearRec* next) {
+  const NearRec b = B.rec[o];
+  const uint32_t z = B.z[o], id = B.id[o];
+  const int32_t c = (int32_t)(z >> kNearRowBits);
+  const int32_t cy = (int32_t)(z & ((1u << kNearRowBits) - 1u));
   const NearWindow w = near_window(rp, col0, c, cy);
   NearAcc acc;
-  near_walk(rp, col0, w, b.x, b.y, b.id, find, birds, heads, &acc);
+  near_walk(rp, col0, w, b.x, b.y, id, find, B, &acc);
   bool found = acc.n != 0 || near_self(rp, b.x, b.y, col0 + c, cy);
-  if (!found) found = near_any(rp, col0, w, b.x, b.y, find, birds);
-  near_finish(acc, found, rp.p, b.id, step, b.x, b.y, h.hx, h.hy, rp.g.w, nx, ny, nhx, nhy);
+  if (!found) found = near_any(rp, col0, w, b.x, b.y, find, B);
+  near_finish(acc, found, rp.p, id, step, b.x, b.y, b.hx, b.hy, rp.g.w, &next->x, &next->y,
+              &next->hx, &next->hy);
 }
 
 // ---- staging a tile ---------------------------------------------------------
@@ -383,8 +443,7 @@ KG_HD void near_step(const RepDev& rp, int32_t col0, uint64_t step, const NearBi
 // LDS of a staged tile: `cap` birds and the per-column tables of `cols`
 // columns.
 struct NearSmem {
-  NearBird* bird;       // cap + 1
-  NearHead* head;       // cap + 1
+  NearBirds b;          // cap
   uint32_t* seg_start;  // 3 per column (flock_segments)
   uint32_t* seg_len;    // 3 per column
   uint32_t* col_base;   // cols + 1
@@ -392,15 +451,14 @@ struct NearSmem {
 };
 
 KG_HD size_t near_smem_bytes(int cap, int cols) {
-  return (size_t)(cap + 1) * (sizeof(NearBird) + sizeof(NearHead)) +
-         (size_t)(7 * cols + 1) * sizeof(uint32_t) + (size_t)((cap + 1) & ~1) * sizeof(uint16_t);
+  return near_birds_bytes((uint32_t)cap) + (size_t)(7 * cols + 1) * sizeof(uint32_t) +
+         (size_t)((cap + 1) & ~1) * sizeof(uint16_t);
 }
 
 KG_HD NearSmem near_carve(uint8_t* p, int cap, int cols) {
   NearSmem s;
-  s.bird = (NearBird*)p;
-  s.head = (NearHead*)(s.bird + cap + 1);
-  s.seg_start = (uint32_t*)(s.head + cap + 1);
+  s.b = near_birds_at(p, (uint32_t)cap, &p);
+  s.seg_start = (uint32_t*)p;
   s.seg_len = s.seg_start + 3 * cols;
   s.col_base = s.seg_len + 3 * cols;
   s.own = (uint16_t*)(s.col_base + cols + 1);
@@ -478,8 +536,9 @@ KG_HD bool near_stage(const RepDev& rp, const FlockTile& ft, const NearChunk& k,
     slot = S.col_base[c] - k.base + S.seg_len[3 * c] + (gi - S.seg_start[3 * c + 1]);
     S.own[i] = (uint16_t)slot;
   }
-  S.bird[slot] = NearBird{x, y, ((uint32_t)c << kNearRowBits) | (uint32_t)cy, id};
-  S.head[slot] = NearHead{hx, hy};
+  S.b.rec[slot] = NearRec{x, y, hx, hy};
+  S.b.z[slot] = ((uint32_t)c << kNearRowBits) | (uint32_t)cy;
+  S.b.id[slot] = id;
   return !near_bad(g, x, y, hx, hy);
 }
 
@@ -495,11 +554,10 @@ KG_HD bool near_item_ok(const RepDev& rp, const NearChunk& k, uint32_t i, Buf R,
 KG_HD void near_agent(const RepDev& rp, const FlockTile& ft, const NearChunk& k, uint32_t o,
                       const NearSmem& S, Buf W, uint32_t* count_next, uint32_t* err,
                       const FlockSinks& lv) {
-  const uint32_t slot = S.own[o];
-  float nx, ny, nhx, nhy;
-  near_step(rp, ft.sc_lo, ft.step, S.bird[slot], S.head[slot],
-            TileFind{S.bird, S.col_base, k.base}, S.bird, S.head, &nx, &ny, &nhx, &nhy);
-  flock_emit(rp.g, rp.bin_base, W, k.own_lo + o, nx, ny, nhx, nhy, count_next, err, ft.tile, lv);
+  NearRec r;
+  near_step(rp, ft.sc_lo, ft.step, S.own[o], TileFind{S.b.z, S.col_base, k.base}, S.b, &r);
+  flock_emit(rp.g, rp.bin_base, W, k.own_lo + o, r.x, r.y, r.hx, r.hy, count_next, err, ft.tile,
+             lv);
 }
 
 }  // namespace kg

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(kT) void k_resident(const RepDev* __restrict__ reps
   }
   const ResSmem S = res_carve(smem_raw, cap);
   const ResBins rb = res_bins(g, bins);
-  const CellFind find{S.bird, S.tab, rb.rows, rb.shift};
+  const CellFind find{S.b.z, S.tab, rb.rows, rb.shift};
   const uint64_t step0 = rp.step_base + *gstep + koff;
 
   ResBird b[kB];
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kT) void k_resident(const RepDev* __restrict__ reps
     __syncthreads();
     res_scan<kT>(S.tab, nb, s_warp);
     __syncthreads();
-    uint64_t* const key = (uint64_t*)S.bird;
+    uint64_t* const key = (uint64_t*)S.b.rec;
 #pragma unroll
     for (int j = 0; j < kB; ++j)
       if ((uint32_t)j * kT + t < n) key[S.tab[b[j].bin] + b[j].slot] = res_key(b[j]);
@@ -103,35 +103,32 @@ __global__ __launch_bounds__(kT) void k_resident(const RepDev* __restrict__ reps
 #pragma unroll
     for (int j = 0; j < kB; ++j) {
       if ((uint32_t)j * kT + t < n) {
-        S.bird[b[j].slot] = NearBird{b[j].x, b[j].y, b[j].z, b[j].id};
-        S.head[b[j].slot] = NearHead{b[j].hx, b[j].hy};
+        S.b.rec[b[j].slot] = NearRec{b[j].x, b[j].y, b[j].hx, b[j].hy};
+        S.b.z[b[j].slot] = b[j].z;
+        S.b.id[b[j].slot] = b[j].id;
       }
     }
-    if (t == 0) S.bird[n].z = ~0u;
+    if (t == 0) S.b.z[n] = ~0u;
     __syncthreads();
     const bool near = s_bad == 0u;
     // bird i of the sorted order: neighbouring lanes walk neighbouring windows
     for (int j = 0; j < kB && (uint32_t)j * kT < n; ++j) {
       const uint32_t i = (uint32_t)j * kT + t;
-      float nx = 0.0f, ny = 0.0f, nhx = 0.0f, nhy = 0.0f;
+      NearRec r{0.0f, 0.0f, 0.0f, 0.0f};
       uint32_t id = 0;
       if (i < n) {
-        const NearBird o = S.bird[i];
-        const NearHead h = S.head[i];
-        id = o.id;
-        if (near)
-          near_step(rp, 0, step0 + k, o, h, find, S.bird, S.head, &nx, &ny, &nhx, &nhy);
-        else
-          full_step(rp, step0 + k, o, h, find, S.bird, S.head, &nx, &ny, &nhx, &nhy);
+        id = S.b.id[i];
+        if (near) near_step(rp, 0, step0 + k, i, find, S.b, &r);
+        else full_step(rp, step0 + k, i, find, S.b, &r);
       }
       // j is the same on every lane: the birds stay in registers
 #pragma unroll
       for (int q = 0; q < kB; ++q) {
         if (q == j) {
-          b[q].x = nx;
-          b[q].y = ny;
-          b[q].hx = nhx;
-          b[q].hy = nhy;
+          b[q].x = r.x;
+          b[q].y = r.y;
+          b[q].hx = r.hx;
+          b[q].hy = r.hy;
           b[q].id = id;
         }
       }

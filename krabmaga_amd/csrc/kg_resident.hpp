@@ -30,21 +30,18 @@ constexpr int32_t kResidentMaxRows = 1 << kNearRowBits;
 
 // LDS of a run of up to `cap` birds and `bins` bins.
 struct ResSmem {
-  NearBird* bird;  // cap + 1; also the keys while birds are in registers
-  NearHead* head;  // cap + 1
-  uint32_t* tab;   // bins + 1
+  NearBirds b;    // cap; its records hold the keys while birds are in registers
+  uint32_t* tab;  // bins + 1
 };
 
 KG_HD size_t res_smem_bytes(uint32_t cap, uint32_t bins) {
-  return (size_t)(cap + 1) * (sizeof(NearBird) + sizeof(NearHead)) +
-         (size_t)(bins + 1) * sizeof(uint32_t);
+  return near_birds_bytes(cap) + (size_t)(bins + 1) * sizeof(uint32_t);
 }
 
 KG_HD ResSmem res_carve(uint8_t* p, uint32_t cap) {
   ResSmem s;
-  s.bird = (NearBird*)p;
-  s.head = (NearHead*)(s.bird + cap + 1);
-  s.tab = (uint32_t*)(s.head + cap + 1);
+  s.b = near_birds_at(p, cap, &p);
+  s.tab = (uint32_t*)p;
   return s;
 }
 
@@ -101,35 +98,38 @@ KG_HD uint64_t res_key(const ResBird& b) {
   return ((uint64_t)(b.z & ((1u << kNearRowBits) - 1u)) << 32) | b.id;
 }
 
-// Bird::step in the general form (any toroidal field whose windows fit) from
-// the same LDS layout.
+// Bird::step of entry o in the general form (any toroidal field whose windows
+// fit) from the same LDS layout.
 template <class Find>
-KG_HD void full_step(const RepDev& rp, uint64_t step, const NearBird& b, const NearHead& h,
-                     const Find& find, const NearBird* birds, const NearHead* heads, float* nx,
-                     float* ny, float* nhx, float* nhy) {
+KG_HD void full_step(const RepDev& rp, uint64_t step, uint32_t o, const Find& find,
+                     const NearBirds& B, NearRec* next) {
   const Geom& g = rp.g;
   const float T = rp.sq_thresh;
-  const NearWindow w = near_window(rp, 0, (int32_t)(b.z >> kNearRowBits),
-                                   (int32_t)(b.z & ((1u << kNearRowBits) - 1u)));
+  const NearRec b = B.rec[o];
+  const uint32_t id = B.id[o];
+  const NearWindow w = near_window(rp, 0, (int32_t)(B.z[o] >> kNearRowBits),
+                                   (int32_t)(B.z[o] & ((1u << kNearRowBits) - 1u)));
   FlockAcc acc;
   for (int32_t q = 0; q <= w.cols && w.rows >= 0; ++q) {
-    const uint32_t key = ((uint32_t)(w.c + q) << kNearRowBits) + (uint32_t)w.row;
+    uint32_t lo, hi;
+    find.one(w.c + q, w.row, (uint32_t)w.rows, &lo, &hi);
     int32_t cur = -1;
     int chk = 0;
-    for (uint32_t e = find.one(w.c + q, w.row); birds[e].z <= key + (uint32_t)w.rows; ++e) {
-      const int32_t row = (int32_t)(birds[e].z & ((1u << kNearRowBits) - 1u));
+    for (uint32_t e = lo; e < hi; ++e) {
+      const int32_t row = (int32_t)(B.z[e] & ((1u << kNearRowBits) - 1u));
       if (row != cur) {
         cur = row;
         chk = check_circle_sq(g, w.c + q, row, b.x, b.y, T);
       }
       if (chk == -1) continue;
-      const float dx = toroidal_distance(b.x, birds[e].x, g.w);
-      const float dy = toroidal_distance(b.y, birds[e].y, g.h);
-      if (chk == 1 || dx * dx + dy * dy <= T)
-        acc.add(birds[e].id == b.id, dx, dy, heads[e].hx, heads[e].hy);
+      const NearRec c = B.rec[e];
+      const float dx = toroidal_distance(b.x, c.x, g.w);
+      const float dy = toroidal_distance(b.y, c.y, g.h);
+      if (chk == 1 || dx * dx + dy * dy <= T) acc.add(B.id[e] == id, dx, dy, c.hx, c.hy);
     }
   }
-  flock_finish(acc, rp.p, b.id, step, b.x, b.y, h.hx, h.hy, g.w, nx, ny, nhx, nhy);
+  flock_finish(acc, rp.p, id, step, b.x, b.y, b.hx, b.hy, g.w, &next->x, &next->y, &next->hx,
+               &next->hy);
 }
 
 }  // namespace kg

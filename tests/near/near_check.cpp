@@ -150,12 +150,12 @@ static int run(const Case& c, uint64_t seed) {
     for (int32_t oa = lo; oa < hi;) {
       const int32_t ob = L > cap ? flock_chunk_end(rp, ft, S.col_base, oa, hi, cap) : hi;
       const NearChunk k = near_chunk(rp, ft, S, oa, ob);
-      std::fill((uint8_t*)S.bird, (uint8_t*)S.seg_start, 0xA5);
+      std::fill((uint8_t*)S.b.rec, (uint8_t*)S.seg_start, 0xA5);
       for (uint32_t i = k.n; i-- > 0;)  // any order
         if (!near_stage(rp, ft, k, i, R.view(), S)) return 1;
-      S.bird[k.n].z = ~0u;
+      S.b.z[k.n] = ~0u;
       for (uint32_t i = 1; i < k.n; ++i)
-        if (S.bird[i].z < S.bird[i - 1].z) {
+        if (S.b.z[i] < S.b.z[i - 1]) {
           std::printf("%s: staged birds out of order\n", c.name);
           return 1;
         }

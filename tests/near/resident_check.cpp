@@ -101,7 +101,7 @@ static int run(const Case& c, uint64_t seed) {
   std::vector<uint64_t> smem((res_smem_bytes(c.n, bins) + 7) / 8 + 2);
   const ResSmem S = res_carve((uint8_t*)(((uintptr_t)smem.data() + 15) & ~(uintptr_t)15), c.n);
   const ResBins rb = res_bins(g, bins);
-  const CellFind find{S.bird, S.tab, rb.rows, rb.shift};
+  const CellFind find{S.b.z, S.tab, rb.rows, rb.shift};
   std::vector<ResBird> b(c.n);
   for (uint32_t i = 0; i < c.n; ++i)
     b[i] = ResBird{R.x[i], R.y[i], R.hx[i], R.hy[i], R.id[i], 0u, 0u, 0u};
@@ -129,17 +129,18 @@ static int run(const Case& c, uint64_t seed) {
       run += v;
     }
     S.tab[nb] = run;
-    uint64_t* key = (uint64_t*)S.bird;
+    uint64_t* key = (uint64_t*)S.b.rec;
     for (auto& q : b) key[S.tab[q.bin] + q.slot] = res_key(q);
     for (auto& q : b)
       q.slot = S.tab[q.bin] + gather_rank(key, S.tab[q.bin], S.tab[q.bin + 1],
                                           S.tab[q.bin] + q.slot, res_key(q));
     if (last) break;
     for (auto& q : b) {
-      S.bird[q.slot] = NearBird{q.x, q.y, q.z, q.id};
-      S.head[q.slot] = NearHead{q.hx, q.hy};
+      S.b.rec[q.slot] = NearRec{q.x, q.y, q.hx, q.hy};
+      S.b.z[q.slot] = q.z;
+      S.b.id[q.slot] = q.id;
     }
-    S.bird[c.n].z = ~0u;
+    S.b.z[c.n] = ~0u;
     general += bad;
     // the general form on the read buffer
     std::vector<uint32_t> cnt(g.nbins, 0u);
@@ -151,11 +152,15 @@ static int run(const Case& c, uint64_t seed) {
     std::vector<uint32_t> at(c.n);
     for (uint32_t i = 0; i < c.n; ++i) at[W.id[i]] = i;
     for (uint32_t i = 0; i < c.n; ++i) {
-      const NearBird o = S.bird[i];
       ResBird& q = b[i];
-      if (bad) full_step(rp, k, o, S.head[i], find, S.bird, S.head, &q.x, &q.y, &q.hx, &q.hy);
-      else near_step(rp, 0, k, o, S.head[i], find, S.bird, S.head, &q.x, &q.y, &q.hx, &q.hy);
-      q.id = o.id;
+      NearRec r;
+      if (bad) full_step(rp, k, i, find, S.b, &r);
+      else near_step(rp, 0, k, i, find, S.b, &r);
+      q.x = r.x;
+      q.y = r.y;
+      q.hx = r.hx;
+      q.hy = r.hy;
+      q.id = S.b.id[i];
       const uint32_t j = at[q.id];
       if (std::memcmp(&q.x, &W.x[j], 4) || std::memcmp(&q.y, &W.y[j], 4) ||
           std::memcmp(&q.hx, &W.hx[j], 4) || std::memcmp(&q.hy, &W.hy[j], 4)) {
