@@ -640,10 +640,12 @@ hipError_t binned_step(kg_ensemble* e, const WorkList& w) {
       return err;
   } else {
     if ((err = launch_scatter_aligned(w, e->R.b, e->W.b, e->offset, e->cursor, e->R2.b,
-                                      e->stream)) != hipSuccess)
+                                      e->nagents, e->ss.partial, e->stream)) != hipSuccess)
       return err;
     // the write buffer has been consumed: it is the sort's scratch
-    if ((err = launch_sort_bins(w, e->R2.b, e->offset2, e->W.b, e->stream)) != hipSuccess)
+    // (the cursors and the scan's sums, used by then, list its crowded bins)
+    if ((err = launch_sort_bins(w, e->R2.b, e->offset2, e->W.b, e->stream, e->cursor, e->nbins,
+                                e->ss.partial)) != hipSuccess)
       return err;
   }
   std::swap(e->R, e->R2);

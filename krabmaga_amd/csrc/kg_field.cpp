@@ -269,8 +269,8 @@ int lazy_update_impl(kg_field* f, uint64_t* step_gstep) {
                                    summed ? f->counts(p) : f->cursor, f->R2.b, f->offset2,
                                    f->W.b, gt, f->err, summed, f->stream));
     } else {
-      KG_HIP(launch_scatter_aligned(wl, f->R.b, f->W.b, f->offset, f->cursor, f->R2.b,
-                                    f->stream));
+      KG_HIP(launch_scatter_aligned(wl, f->R.b, f->W.b, f->offset, f->cursor, f->R2.b, f->nW,
+                                    f->ss.partial, f->stream));
     }
   }
   if (!gather) {
@@ -280,7 +280,13 @@ int lazy_update_impl(kg_field* f, uint64_t* step_gstep) {
     }
     // the write buffer has been consumed: it is the sort's scratch
     ProfScope ps(f, KG_KERNEL_SORT_BINS);
-    KG_HIP(launch_sort_bins(wl, f->R2.b, f->offset2, f->W.b, f->stream));
+    // the scatters have used the cursors and the scan its sums: they hold the
+    // list of crowded bins
+    if (f->w_aligned && f->nW)
+      KG_HIP(launch_sort_bins(wl, f->R2.b, f->offset2, f->W.b, f->stream, f->cursor, f->g.nbins,
+                              f->ss.partial));
+    else
+      KG_HIP(launch_sort_bins(wl, f->R2.b, f->offset2, f->W.b, f->stream));
   }
   std::swap(f->R, f->R2);
   std::swap(f->offset, f->offset2);

@@ -85,39 +85,49 @@ hipError_t launch_scatter_append(const WorkList& wl, Buf A, uint32_t* cursor, Bu
 }
 
 // Rebinning of the write buffer the flock kernel produced: it is aligned with
-// the current read buffer, so work item (replica, tile) moves exactly the
-// agents of that tile's old range.  fill_base null: cursor[b] is bin b's next
-// free slot; else cursor[b] is bin b's count of agents still to place, and
-// they go to fill_base[b] + count - 1 downwards (the count ends at zero).
-__device__ __forceinline__ void scatter_aligned_tiles(const RepDev* __restrict__ reps, int nreps,
-                                                      const uint32_t* __restrict__ tile_prefix,
-                                                      Buf R, Buf W,
-                                                      const uint32_t* __restrict__ offset_cur,
-                                                      uint32_t* __restrict__ cursor, Buf R2,
-                                                      const uint32_t* __restrict__ fill_base,
-                                                      uint32_t nitems) {
-  for (uint32_t bi = blockIdx.x; bi < nitems; bi += gridDim.x) {
-    const uint32_t item = xcd_remap(bi, nitems);
-    const TileRange tr = tile_range(reps, nreps, tile_prefix, item, offset_cur);
-    const RepDev& rp = reps[tr.r];
-    const Geom& g = rp.g;
-    const uint32_t lane = threadIdx.x & (kWave - 1);
+// the current read buffer, whose slots are taken kScatterRun at a time, a run
+// to a work-group, so a crowded tile is spread over the GPU (one work-group
+// per tile took 270 us for 8.4M birds in blobs of up to 37k birds per tile,
+// most of it in a few hundred work-groups).  fill_base null:
+// cursor[b] is bin b's next free slot; else cursor[b] is bin b's count of
+// agents still to place, and they go to fill_base[b] + count - 1 downwards
+// (the count ends at zero).
+constexpr uint32_t kScatterRun = 1024;
+
+__device__ __forceinline__ void scatter_aligned_runs(const RepDev* __restrict__ reps, int nreps,
+                                                     const uint32_t* __restrict__ app_prefix,
+                                                     Buf R, Buf W,
+                                                     const uint32_t* __restrict__ offset_cur,
+                                                     uint32_t* __restrict__ cursor, Buf R2,
+                                                     const uint32_t* __restrict__ fill_base) {
+  const RepDev& end = reps[nreps - 1];
+  const uint32_t n = offset_cur[end.bin_base + end.g.nbins];
+  const uint32_t nruns = (n + kScatterRun - 1) / kScatterRun;
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  for (uint32_t run = blockIdx.x; run < nruns; run += gridDim.x) {
+    const uint32_t g0 = run * kScatterRun, g1 = min(n, g0 + kScatterRun);
+    // the run's replica, or every bird looks for its own
+    int r0 = 0, r1 = 0;
+    if (nreps > 1) {
+      r0 = find_rep(app_prefix, nreps, g0);
+      r1 = find_rep(app_prefix, nreps, g1 - 1u);
+    }
     // The read buffer is in bin order and birds move little, so neighbouring
     // lanes mostly share a destination bin: one cursor atomic per run of
     // equal bins in a wave (the bin sort that follows fixes the order inside
     // a bin).  Every lane takes part in every round for the wave operations.
-    for (uint32_t i0 = tr.lo; i0 < tr.hi; i0 += blockDim.x) {
+    for (uint32_t i0 = g0; i0 < g1; i0 += blockDim.x) {
       const uint32_t i = i0 + threadIdx.x;
-      bool valid = i < tr.hi;
+      bool valid = i < g1;
       float x = 0.0f, y = 0.0f;
       uint32_t bin = 0xFFFFFFFFu;
       if (valid) {
         x = W.x[i];
         y = W.y[i];
-        int32_t cx, cy;
-        discretize(g, x, y, &cx, &cy);
-        valid = cell_valid(g, cx, cy);  // an invalid cell was reported by the flock kernel
-        if (valid) bin = rp.bin_base + bin_of(g, cx, cy);
+        const RepDev& rp = reps[r0 == r1 ? r0 : find_rep(app_prefix, nreps, i)];
+        const int32_t cx = cell_axis(rp.g, x), cy = cell_axis(rp.g, y);
+        valid = cell_valid(rp.g, cx, cy);  // an invalid cell was reported by the flock kernel
+        if (valid) bin = rp.bin_base + bin_of(rp.g, cx, cy);
       }
       const uint32_t prev = __shfl_up(bin, 1, kWave);
       const bool head = valid && (lane == 0 || prev != bin);
@@ -133,9 +143,9 @@ __device__ __forceinline__ void scatter_aligned_tiles(const RepDev* __restrict__
       const uint64_t to_nh = nh == kWave ? ~0ull : ((1ull << nh) - 1ull);
       uint32_t base = 0;
       if (head) {
-        const uint32_t run = (uint32_t)__popcll(vmask & from_h & to_nh);
-        base = fill_base ? fill_base[bin] + atomicSub(&cursor[bin], run) - run
-                         : atomicAdd(&cursor[bin], run);
+        const uint32_t len = (uint32_t)__popcll(vmask & from_h & to_nh);
+        base = fill_base ? fill_base[bin] + atomicSub(&cursor[bin], len) - len
+                         : atomicAdd(&cursor[bin], len);
       }
       base = __shfl(base, h, kWave);
       if (valid) {
@@ -152,13 +162,13 @@ __device__ __forceinline__ void scatter_aligned_tiles(const RepDev* __restrict__
 }
 
 __global__ __launch_bounds__(256) void k_scatter_aligned(const RepDev* __restrict__ reps, int nreps,
-                                                         const uint32_t* __restrict__ tile_prefix,
+                                                         const uint32_t* __restrict__ app_prefix,
                                                          Buf R, Buf W,
                                                          const uint32_t* __restrict__ offset_cur,
                                                          uint32_t* __restrict__ cursor, Buf R2,
-                                                         uint32_t nitems) {
-  scatter_aligned_tiles(reps, nreps, tile_prefix, R, W, offset_cur, cursor, R2, nullptr,
-                        nitems);
+                                                         uint32_t* __restrict__ nlist) {
+  if (nlist && blockIdx.x == 0 && threadIdx.x < 2) nlist[threadIdx.x] = 0u;  // for the sort
+  scatter_aligned_runs(reps, nreps, app_prefix, R, W, offset_cur, cursor, R2, nullptr);
 }
 
 // Work-groups of the gated fallback: in most steps they only read the gate
@@ -167,10 +177,12 @@ __global__ __launch_bounds__(256) void k_scatter_aligned(const RepDev* __restric
 constexpr uint32_t kGatedGrid = 256;
 
 hipError_t launch_scatter_aligned(const WorkList& wl, Buf R, Buf W, const uint32_t* offset_cur,
-                                  uint32_t* cursor, Buf R2, hipStream_t s) {
-  if (wl.ntiles == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_scatter_aligned, dim3(wl.ntiles), dim3(256), 0, s, wl.reps, wl.nreps,
-                     wl.tile_prefix, R, W, offset_cur, cursor, R2, wl.ntiles);
+                                  uint32_t* cursor, Buf R2, uint32_t nagents, uint32_t* nlist,
+                                  hipStream_t s) {
+  if (wl.ntiles == 0 || nagents == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_scatter_aligned, dim3((nagents + kScatterRun - 1) / kScatterRun),
+                     dim3(256), 0, s, wl.reps, wl.nreps, wl.app_prefix, R, W, offset_cur, cursor,
+                     R2, nlist);
   return hipGetLastError();
 }
 
@@ -709,6 +721,132 @@ __global__ __launch_bounds__(kT, 8) void k_flock_near(
   }
 }
 
+// The birds of flagged tiles of near fields, kRun consecutive read-buffer
+// slots to a work-group.  Birds lie tile by tile, column by column, row by
+// row, so a run of a crowded tile is a strip of one or two columns: it is
+// staged with its neighbourhood (near_piece) and walked from LDS, piece by
+// piece where it crosses tiles or does not fit.  A piece that does not fit
+// even so, or is not near, takes the general walk, one thread per bird.
+// What bounds it: VALU issue in the walk (about 45 instructions per
+// candidate; 65 neighbours per bird in blobs of 105k birds, sigma 200).
+// kRun = 512: two work-groups of eight waves share a CU's LDS; the longer the
+// run the smaller the staged share that is halo.
+// kStride: as k_flock_global.
+constexpr int kRun = 512;
+constexpr int kRunCap = 2000;  // staged birds of a piece
+
+template <bool kStride>
+__global__ __launch_bounds__(kRun, 6) void k_flock_runs(
+    const RepDev* __restrict__ reps, int nreps, const uint32_t* __restrict__ tile_prefix,
+    const uint32_t* __restrict__ app_prefix, Buf R, const uint32_t* __restrict__ offset, Buf W,
+    uint32_t* __restrict__ count_next, const uint64_t* __restrict__ gstep,
+    uint32_t* __restrict__ err, const uint32_t* __restrict__ gflag, uint32_t ntiles, uint32_t n,
+    Outbox ob, uint32_t* __restrict__ tile_sum, int cols) {
+  extern __shared__ __align__(16) uint8_t smem_raw[];
+  __shared__ uint32_t s_warp[kRun / kWave];
+  __shared__ uint32_t s_any, s_bad;
+  // no tile took the global path in this step
+  if (gflag[ntiles] != (uint32_t)*gstep + 1u) return;
+  const int t = threadIdx.x;
+  const NearSmem S = near_carve(smem_raw, kRunCap, cols);
+  // replica and global tile of read-buffer slot q, or false for a bird
+  // outside its grid
+  auto tile_at = [&](uint32_t q, int* r, uint32_t* tile) {
+    *r = nreps == 1 ? 0 : find_rep(app_prefix, nreps, q);
+    const Geom& g = reps[*r].g;
+    int32_t cx, cy;
+    discretize(g, R.x[q], R.y[q], &cx, &cy);
+    if (!cell_valid(g, cx, cy)) return false;
+    *tile = tile_prefix[*r] + tile_of(g, cx, cy);
+    return true;
+  };
+  auto one_run = [&](uint32_t run) {
+    const uint32_t g0 = run * kRun, g1 = min(n, g0 + kRun);
+    if (t == 0) {
+      int r;
+      uint32_t t0 = 0, t1 = 0, any = 1u;
+      if (tile_at(g0, &r, &t0) && tile_at(g1 - 1u, &r, &t1) && t1 - t0 < kRun) {
+        any = 0u;
+        for (uint32_t q = t0; q <= t1; ++q) any |= gflag[q];
+      }
+      s_any = any;
+    }
+    __syncthreads();
+    const uint32_t any = s_any;
+    __syncthreads();  // s_any is rewritten for the next run
+    if (!any) return;
+    // everything below but the birds' own work is the same on all lanes
+    for (uint32_t s = g0; s < g1;) {
+      int r = 0;
+      uint32_t item = 0;
+      if (!tile_at(s, &r, &item)) {
+        ++s;
+        continue;
+      }
+      const RepDev& rp = reps[r];
+      const Geom& g = rp.g;
+      const FlockTile ft = flock_tile(reps, nreps, tile_prefix, item, *gstep);
+      uint32_t e = min(g1, max(s + 1u, offset[ft.tb1]));
+      if (!gflag[item]) {
+        s = e;
+        continue;
+      }
+      const FlockSinks lv{ob, tile_prefix[r], nullptr, nullptr, tile_sum};
+      const int32_t ca = cell_axis(g, R.x[s]);
+      int32_t cb = cell_axis(g, R.x[e - 1]);
+      bool lds = rp.near != 0 && cb >= ca;
+      FlockTile pt = ft;
+      for (int attempt = 0; lds; ++attempt) {
+        if (attempt > 0 && cb > ca) {  // the first column's birds alone
+          const int32_t lc = ca & (g.tx - 1);
+          e = min(e, max(s + 1u, offset[rp.bin_base + col_bin0(g, ft.tile, lc) + (uint32_t)g.tr]));
+          cb = ca;
+        } else if (attempt > 0) {  // half of them
+          e = s + (e - s + 1u) / 2u;
+        }
+        const int32_t r0 = ca == cb ? cell_axis(g, R.y[s]) : ft.y0;
+        const int32_t r1 = ca == cb ? cell_axis(g, R.y[e - 1]) : ft.y1 - 1;
+        pt = near_piece(rp, ft, ca, cb, r0, r1);
+        uint32_t L = 0;
+        if (pt.ncols <= cols) {
+          const uint32_t len =
+              t < pt.ncols ? flock_segments(rp, pt, t, offset, S.seg_start, S.seg_len) : 0u;
+          const uint32_t ex = block_exclusive_scan<kRun>(len, s_warp, &L);
+          if (t < pt.ncols) S.col_base[t] = ex;
+          if (t == 0) {
+            S.col_base[pt.ncols] = L;
+            s_bad = 0u;
+          }
+          __syncthreads();
+          if (L <= (uint32_t)kRunCap) {
+            for (uint32_t i = t; i < L; i += kRun)
+              if (!near_stage_piece(rp, pt, i, R, S)) s_bad = 1u;
+            if (t == 0) S.b.z[L] = ~0u;
+            __syncthreads();
+            lds = s_bad == 0u;
+            break;
+          }
+        }
+        // a neighbourhood this crowded: too few birds would share its staging
+        if (ca == cb && e - s < 64u) lds = false;
+      }
+      const uint32_t gi = s + (uint32_t)t;
+      if (gi < e) {
+        if (lds) near_agent_piece(rp, pt, gi, R, S, W, count_next, err, lv);
+        else flock_agent_global(rp, ft.step, gi, R, offset, W, count_next, err, lv);
+      }
+      __syncthreads();  // the next piece reuses the LDS
+      s = e;
+    }
+  };
+  if (kStride) {
+    const uint32_t nruns = (n + kRun - 1) / kRun;
+    for (uint32_t run = blockIdx.x; run < nruns; run += gridDim.x) one_run(run);
+  } else {
+    one_run(blockIdx.x);
+  }
+}
+
 // The birds of flagged tiles, one thread per read-buffer slot.  The read
 // buffer holds the replicas one after another (replica r at
 // app_prefix[r], its tiles one after another), each tile's bins in order.
@@ -793,6 +931,16 @@ hipError_t launch_flock(const WorkList& wl, Buf R, const uint32_t* offset, Buf W
                        wl.tile_prefix, R, offset, W, count_next, gstep, err, lds_cap, gflag, ob,
                        tile_sum);
   }
+  if (nagents && !inline_global && near.on) {
+    const uint32_t nruns = (nagents + kRun - 1) / kRun;
+    const bool stride = global_grid && global_grid < nruns;
+    hipLaunchKernelGGL(stride ? k_flock_runs<true> : k_flock_runs<false>,
+                       dim3(stride ? global_grid : nruns), dim3(kRun),
+                       near_piece_bytes(kRunCap, near.cols), s, wl.reps, wl.nreps, wl.tile_prefix,
+                       wl.app_prefix, R, offset, W, count_next, gstep, err, gflag, wl.ntiles,
+                       nagents, ob, tile_sum, near.cols);
+    return hipGetLastError();
+  }
   const uint32_t nruns = (nagents + kFlockThreads - 1) / kFlockThreads;
   if (nagents && !inline_global) {
     const bool stride = global_grid && global_grid < nruns;
@@ -812,10 +960,14 @@ hipError_t launch_flock(const WorkList& wl, Buf R, const uint32_t* offset, Buf W
 // round trip.  A bin of at most kSortSmall entries is sorted by its own lane
 // (sort_small_bin); a bin of up to 64 entries by a quarter wave, four bins
 // side by side (sort_seg_bins); a bin of up to four times a wave's width by
-// one wave -- all in registers, rewritten in place (every lane has loaded its
-// entries before any lane stores); larger bins are ranked by the whole
+// one wave (sort_wave_rows) -- all rewritten in place (every lane has loaded
+// its entries before any lane stores); larger bins are ranked by the whole
 // block against keys staged in LDS, written to the scratch buffer T at the
-// same indices and copied back.
+// same indices and copied back.  With a list, the bins past kSortSmall entries
+// are left to k_sort_list, which spreads them over the GPU, a wave each: in
+// crowded blobs one work-group's tile holds hundreds of them (8.4M birds in
+// 64 blobs: 1,073 us for the sort with all of a tile's bins in its own
+// work-group).
 
 constexpr int kSortThreads = 256;
 constexpr int kSortSlots = 4;                              // entries per lane on the wave path
@@ -911,15 +1063,34 @@ __device__ __forceinline__ void sort_seg_bins(const Geom& g, Buf R, uint32_t s, 
   }
 }
 
-// One wave ranks bin [s, s + m) (kSortSegMax < m <= kSortWaveMax): entry
-// lane + 64 u in slot u of the lane's registers.
-__device__ __forceinline__ void sort_wave_bin(const Geom& g, Buf R, uint32_t s, uint32_t m,
-                                              uint32_t lane) {
-  uint32_t idv[kSortSlots], rk[kSortSlots];
-  float xv[kSortSlots], yv[kSortSlots], hxv[kSortSlots], hyv[kSortSlots];
-  uint64_t kv[kSortSlots];
+// One wave sorts bin [s, s + m) (m <= 64 kSlots <= kSortWaveMax), entry lane
+// + 64 u in slot u of the lane's registers: counted by row in LDS, then
+// ranked among its own row's ids there, so an entry is compared with a bag's
+// birds and not with the bin's.  w: kSortWaveMax ids, then kSortRows + 1 row
+// starts; bins of more rows (a caller's bin height) take gather_rank over
+// whole keys.
+constexpr uint32_t kSortRows = 64;
+
+// LDS written by other lanes of the wave before this point is read after it
+// (one wave's LDS operations run in order; this keeps the compiler's too).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+struct SortWave {
+  uint64_t key[kSortWaveMax];  // ids (low words) or whole keys
+  uint32_t row[kSortRows];
+};
+
+template <int kSlots>
+__device__ __forceinline__ void sort_wave_rows(const Geom& g, Buf R, uint32_t s, uint32_t m,
+                                               uint32_t lane, SortWave* w) {
+  uint32_t idv[kSlots], rk[kSlots], rw[kSlots];
+  float xv[kSlots], yv[kSlots], hxv[kSlots], hyv[kSlots];
+  uint64_t kv[kSlots];
 #pragma unroll
-  for (int u = 0; u < kSortSlots; ++u) {
+  for (int u = 0; u < kSlots; ++u) {
     const uint32_t e = lane + (uint32_t)u * kWave;
     idv[u] = 0;
     yv[u] = 0.0f;
@@ -928,6 +1099,7 @@ __device__ __forceinline__ void sort_wave_bin(const Geom& g, Buf R, uint32_t s, 
       yv[u] = R.y[s + e];
     }
     kv[u] = e < m ? bin_key(g, yv[u], idv[u]) : ~0ull;
+    rw[u] = (uint32_t)(kv[u] >> 32) & (uint32_t)(g.hb - 1);
     rk[u] = 0;
   }
   // already in order (the scatter keeps most bins so): nothing to write.
@@ -936,7 +1108,7 @@ __device__ __forceinline__ void sort_wave_bin(const Geom& g, Buf R, uint32_t s, 
   // u - 1 for lane 0.
   bool inv = false;
 #pragma unroll
-  for (int u = 0; u < kSortSlots; ++u) {
+  for (int u = 0; u < kSlots; ++u) {
     const uint32_t e = lane + (uint32_t)u * kWave;
     const uint64_t up = __shfl_up(kv[u], 1, kWave);
     const uint64_t wrap = u > 0 ? readlane64(kv[u > 0 ? u - 1 : 0], kWave - 1) : 0ull;
@@ -945,7 +1117,7 @@ __device__ __forceinline__ void sort_wave_bin(const Geom& g, Buf R, uint32_t s, 
   }
   if (!__any(inv)) return;
 #pragma unroll
-  for (int u = 0; u < kSortSlots; ++u) {
+  for (int u = 0; u < kSlots; ++u) {
     const uint32_t e = lane + (uint32_t)u * kWave;
     xv[u] = hxv[u] = hyv[u] = 0.0f;
     if (e < m) {
@@ -954,20 +1126,50 @@ __device__ __forceinline__ void sort_wave_bin(const Geom& g, Buf R, uint32_t s, 
       hyv[u] = R.hy[s + e];
     }
   }
-  for (uint32_t j = 0; j < m; ++j) {
-    const uint32_t ju = j / kWave;  // the same on every lane
-    const uint64_t src = ju == 0 ? kv[0] : (ju == 1 ? kv[1] : (ju == 2 ? kv[2] : kv[3]));
-    const uint64_t kj = readlane64(src, j & (kWave - 1));
+  const bool rows = g.hb <= (int32_t)kSortRows;  // the same on every lane
+  if (rows) {
+    // row counts, then starts; an entry's place in its row is its turn at
+    // the counter
+    w->row[lane] = 0u;
+    wave_sync();
+    uint32_t turn[kSlots];
 #pragma unroll
-    for (int u = 0; u < kSortSlots; ++u) {
-      const uint32_t e = lane + (uint32_t)u * kWave;
-      rk[u] += (kj < kv[u]) || (kj == kv[u] && j < e);
+    for (int u = 0; u < kSlots; ++u)
+      turn[u] = lane + (uint32_t)u * kWave < m ? atomicAdd(&w->row[rw[u]], 1u) : 0u;
+    wave_sync();
+    const uint32_t cnt = w->row[lane];
+    uint32_t incl = cnt;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint32_t v = __shfl_up(incl, off, kWave);
+      if ((int)lane >= off) incl += v;
     }
+    wave_sync();
+    uint32_t lo[kSlots], hi[kSlots];
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+      hi[u] = __shfl(incl, (int)rw[u], kWave);
+      lo[u] = hi[u] - __shfl(cnt, (int)rw[u], kWave);
+      if (lane + (uint32_t)u * kWave < m) w->key[lo[u] + turn[u]] = idv[u];
+    }
+    wave_sync();
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u)
+      if (lane + (uint32_t)u * kWave < m)
+        rk[u] = lo[u] + gather_rank(w->key, lo[u], hi[u], lo[u] + turn[u], idv[u]);
+  } else {
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u)
+      if (lane + (uint32_t)u * kWave < m) w->key[lane + (uint32_t)u * kWave] = kv[u];
+    wave_sync();
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u)
+      if (lane + (uint32_t)u * kWave < m)
+        rk[u] = gather_rank(w->key, 0u, m, lane + (uint32_t)u * kWave, kv[u]);
   }
 #pragma unroll
-  for (int u = 0; u < kSortSlots; ++u) {
-    const uint32_t e = lane + (uint32_t)u * kWave;
-    if (e < m) {
+  for (int u = 0; u < kSlots; ++u) {
+    if (lane + (uint32_t)u * kWave < m) {
       R.id[s + rk[u]] = idv[u];
       R.x[s + rk[u]] = xv[u];
       R.y[s + rk[u]] = yv[u];
@@ -977,22 +1179,82 @@ __device__ __forceinline__ void sort_wave_bin(const Geom& g, Buf R, uint32_t s, 
   }
 }
 
+// A bin [s, s + m) of any size by the whole work-group, keys in s_key
+// (kSortChunk), T as scratch.
+__device__ __forceinline__ void sort_block_bin(const Geom& g, Buf R, uint32_t s, uint32_t m, Buf T,
+                                               uint64_t* s_key) {
+  const int t = threadIdx.x;
+  const bool staged_once = m <= kSortChunk;
+  if (staged_once) {
+    for (uint32_t j = t; j < m; j += kSortThreads) s_key[j] = bin_key(g, R.y[s + j], R.id[s + j]);
+    __syncthreads();
+  }
+  for (uint32_t e0 = 0; e0 < m; e0 += kSortThreads) {
+    const uint32_t e = e0 + (uint32_t)t;
+    const bool act = e < m;
+    const uint64_t key = act ? bin_key(g, R.y[s + e], R.id[s + e]) : 0ull;
+    uint32_t rank = 0;
+    for (uint32_t c0 = 0; c0 < m; c0 += kSortChunk) {
+      const uint32_t n = m - c0 < kSortChunk ? m - c0 : kSortChunk;
+      if (!staged_once) {
+        __syncthreads();
+        for (uint32_t j = t; j < n; j += kSortThreads)
+          s_key[j] = bin_key(g, R.y[s + c0 + j], R.id[s + c0 + j]);
+        __syncthreads();
+      }
+      if (act)
+        for (uint32_t j = 0; j < n; ++j) {
+          const uint64_t kj = s_key[j];
+          rank += (kj < key) || (kj == key && c0 + j < e);
+        }
+    }
+    if (act) {
+      T.id[s + rank] = R.id[s + e];
+      T.x[s + rank] = R.x[s + e];
+      T.y[s + rank] = R.y[s + e];
+      T.hx[s + rank] = R.hx[s + e];
+      T.hy[s + rank] = R.hy[s + e];
+    }
+  }
+  __syncthreads();
+  for (uint32_t j = t; j < m; j += kSortThreads) {
+    R.id[s + j] = T.id[s + j];
+    R.x[s + j] = T.x[s + j];
+    R.y[s + j] = T.y[s + j];
+    R.hx[s + j] = T.hx[s + j];
+    R.hy[s + j] = T.hy[s + j];
+  }
+  __syncthreads();
+}
+
+// Bins past kSortSmall entries, left to k_sort_list: n[0] of up to
+// kSortWaveMax entries from the front
+// of bin[], n[1] larger ones from its back (size entries, one per bin).
+struct SortList {
+  uint32_t* bin = nullptr;
+  uint32_t* n = nullptr;
+  uint32_t size = 0;
+};
+
 __device__ __forceinline__ void sort_bins_tiles(const RepDev* __restrict__ reps, int nreps,
                                                 const uint32_t* __restrict__ tile_prefix, Buf R,
                                                 const uint32_t* __restrict__ offset, Buf T,
-                                                uint32_t nitems) {
+                                                uint32_t nitems, const SortList& list) {
   __shared__ uint64_t s_key[kSortChunk];
   __shared__ uint32_t s_seg[kSortThreads];
   __shared__ uint32_t s_mid[kSortThreads];
   __shared__ uint32_t s_big[kSortThreads];
   __shared__ uint32_t s_nseg, s_nmid, s_nbig;
+  // the waves' sorting space and the block's keys are used one after the other
+  static_assert(sizeof(SortWave) * (kSortThreads / kWave) <= sizeof(uint64_t) * kSortChunk, "");
   const int t = threadIdx.x;
   const uint32_t lane = (uint32_t)t & (kWave - 1);
   const uint32_t wid = (uint32_t)t / kWave;
+  SortWave* const sw = (SortWave*)s_key + wid;
   for (uint32_t bi = blockIdx.x; bi < nitems; bi += gridDim.x) {
     const uint32_t item = xcd_remap(bi, nitems);
     const int r = find_rep(tile_prefix, nreps, item);
-    const Geom g = reps[r].g;
+    const Geom& g = reps[r].g;
     const uint32_t nb = 1u << (g.tx_log2 + g.tr_log2);
     const uint32_t b0 = reps[r].bin_base + ((item - tile_prefix[r]) << (g.tx_log2 + g.tr_log2));
 
@@ -1007,8 +1269,9 @@ __device__ __forceinline__ void sort_bins_tiles(const RepDev* __restrict__ reps,
         const uint32_t b = b0 + k0 + (uint32_t)t;
         const uint32_t s = offset[b], m = offset[b + 1] - s;
         if (m >= 2u && m <= kSortSmall) sort_small_bin(g, R, s, m);
-        else if (m > kSortSmall && m <= kSortSegMax) s_seg[atomicAdd(&s_nseg, 1u)] = b;
-        else if (m > kSortSegMax && m <= kSortWaveMax) s_mid[atomicAdd(&s_nmid, 1u)] = b;
+        else if (m > kSortSmall && m <= kSortSegMax && !list.bin)
+          s_seg[atomicAdd(&s_nseg, 1u)] = b;
+        else if (m > kSortSmall && m <= kSortWaveMax) s_mid[atomicAdd(&s_nmid, 1u)] = b;
         else if (m > kSortWaveMax) s_big[atomicAdd(&s_nbig, 1u)] = b;
       }
       __syncthreads();
@@ -1024,58 +1287,29 @@ __device__ __forceinline__ void sort_bins_tiles(const RepDev* __restrict__ reps,
         }
         sort_seg_bins(g, R, s, m, lane);
       }
-      // middle bins: one wave each
-      const uint32_t nmid = s_nmid;
-      for (uint32_t i = wid; i < nmid; i += kSortThreads / kWave) {
-        const uint32_t s = offset[s_mid[i]];
-        sort_wave_bin(g, R, s, offset[s_mid[i] + 1] - s, lane);
-      }
-      // larger bins: the whole block
-      const uint32_t nbig = s_nbig;
-      for (uint32_t i = 0; i < nbig; ++i) {
-        const uint32_t s = offset[s_big[i]];
-        const uint32_t m = offset[s_big[i] + 1] - s;
-        const bool staged_once = m <= kSortChunk;
-        if (staged_once) {
-          for (uint32_t j = t; j < m; j += kSortThreads) s_key[j] = bin_key(g, R.y[s + j], R.id[s + j]);
-          __syncthreads();
-        }
-        for (uint32_t e0 = 0; e0 < m; e0 += kSortThreads) {
-          const uint32_t e = e0 + (uint32_t)t;
-          const bool act = e < m;
-          const uint64_t key = act ? bin_key(g, R.y[s + e], R.id[s + e]) : 0ull;
-          uint32_t rank = 0;
-          for (uint32_t c0 = 0; c0 < m; c0 += kSortChunk) {
-            const uint32_t n = m - c0 < kSortChunk ? m - c0 : kSortChunk;
-            if (!staged_once) {
-              __syncthreads();
-              for (uint32_t j = t; j < n; j += kSortThreads)
-                s_key[j] = bin_key(g, R.y[s + c0 + j], R.id[s + c0 + j]);
-              __syncthreads();
-            }
-            if (act)
-              for (uint32_t j = 0; j < n; ++j) {
-                const uint64_t kj = s_key[j];
-                rank += (kj < key) || (kj == key && c0 + j < e);
-              }
-          }
-          if (act) {
-            T.id[s + rank] = R.id[s + e];
-            T.x[s + rank] = R.x[s + e];
-            T.y[s + rank] = R.y[s + e];
-            T.hx[s + rank] = R.hx[s + e];
-            T.hy[s + rank] = R.hy[s + e];
-          }
+      const uint32_t nmid = s_nmid, nbig = s_nbig;
+      if (list.bin) {
+        __shared__ uint32_t s_at[2];
+        if (t == 0) {
+          s_at[0] = nmid ? atomicAdd(&list.n[0], nmid) : 0u;
+          s_at[1] = nbig ? atomicAdd(&list.n[1], nbig) : 0u;
         }
         __syncthreads();
-        for (uint32_t j = t; j < m; j += kSortThreads) {
-          R.id[s + j] = T.id[s + j];
-          R.x[s + j] = T.x[s + j];
-          R.y[s + j] = T.y[s + j];
-          R.hx[s + j] = T.hx[s + j];
-          R.hy[s + j] = T.hy[s + j];
+        for (uint32_t i = t; i < nmid; i += kSortThreads) list.bin[s_at[0] + i] = s_mid[i];
+        for (uint32_t i = t; i < nbig; i += kSortThreads)
+          list.bin[list.size - 1u - (s_at[1] + i)] = s_big[i];
+      } else {
+        // middle bins: one wave each
+        for (uint32_t i = wid; i < nmid; i += kSortThreads / kWave) {
+          const uint32_t s = offset[s_mid[i]];
+          sort_wave_rows<kSortSlots>(g, R, s, offset[s_mid[i] + 1] - s, lane, sw);
         }
         __syncthreads();
+        // larger bins: the whole block
+        for (uint32_t i = 0; i < nbig; ++i) {
+          const uint32_t s = offset[s_big[i]];
+          sort_block_bin(g, R, s, offset[s_big[i] + 1] - s, T, s_key);
+        }
       }
       __syncthreads();
     }
@@ -1084,8 +1318,40 @@ __device__ __forceinline__ void sort_bins_tiles(const RepDev* __restrict__ reps,
 
 __global__ __launch_bounds__(kSortThreads) void k_sort_bins(
     const RepDev* __restrict__ reps, int nreps, const uint32_t* __restrict__ tile_prefix, Buf R,
-    const uint32_t* __restrict__ offset, Buf T, uint32_t nitems) {
-  sort_bins_tiles(reps, nreps, tile_prefix, R, offset, T, nitems);
+    const uint32_t* __restrict__ offset, Buf T, uint32_t nitems, SortList list) {
+  sort_bins_tiles(reps, nreps, tile_prefix, R, offset, T, nitems, list);
+}
+
+// The listed bins, a wave or (past kSortWaveMax entries) a work-group each.
+__global__ __launch_bounds__(kSortThreads) void k_sort_list(const RepDev* __restrict__ reps,
+                                                            int nreps, Buf R,
+                                                            const uint32_t* __restrict__ offset,
+                                                            Buf T, SortList list) {
+  __shared__ uint64_t s_key[kSortChunk];
+  const uint32_t lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  SortWave* const sw = (SortWave*)s_key + wid;
+  const uint32_t nmid = list.n[0], nbig = list.n[1];
+  auto geom_of = [&](uint32_t b) -> const Geom& {
+    int lo = 0, hi = nreps;  // last replica whose bins start at or before b
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (reps[mid].bin_base <= b) lo = mid;
+      else hi = mid;
+    }
+    return reps[lo].g;
+  };
+  constexpr uint32_t kWaves = kSortThreads / kWave;
+  for (uint32_t i = blockIdx.x * kWaves + wid; i < nmid; i += gridDim.x * kWaves) {
+    const uint32_t b = list.bin[i], s = offset[b];
+    const uint32_t m = offset[b + 1] - s;
+    if (m <= (uint32_t)kWave) sort_wave_rows<1>(geom_of(b), R, s, m, lane, sw);
+    else sort_wave_rows<kSortSlots>(geom_of(b), R, s, m, lane, sw);
+  }
+  __syncthreads();
+  for (uint32_t i = blockIdx.x; i < nbig; i += gridDim.x) {
+    const uint32_t b = list.bin[list.size - 1u - i], s = offset[b];
+    sort_block_bin(geom_of(b), R, s, offset[b + 1] - s, T, s_key);
+  }
 }
 
 // Waits until all `nblocks` work-groups of the grid have arrived at `bar`
@@ -1124,19 +1390,20 @@ __device__ bool grid_wait(uint32_t* bar, uint32_t nblocks) {
 // summed steps' gather writes no cursors).  A wait that times out sets bit
 // 2 of err and leaves the bins unsorted.
 __global__ __launch_bounds__(256) void k_rebin_fallback(
-    const RepDev* __restrict__ reps, int nreps, const uint32_t* __restrict__ tile_prefix, Buf R,
-    Buf W, const uint32_t* __restrict__ offset_cur, uint32_t* __restrict__ cursor, Buf R2,
+    const RepDev* __restrict__ reps, int nreps, const uint32_t* __restrict__ tile_prefix,
+    const uint32_t* __restrict__ app_prefix, Buf R, Buf W,
+    const uint32_t* __restrict__ offset_cur, uint32_t* __restrict__ cursor, Buf R2,
     const uint32_t* __restrict__ offset_new, Buf T, Gate gate, uint32_t* __restrict__ err,
     int count_down, uint32_t nitems) {
   if (*gate.flag == 0u) return;  // the gather rebinned this step
   if (blockIdx.x == 0 && threadIdx.x == 0) *gate.redone += 1u;  // steps redone
-  scatter_aligned_tiles(reps, nreps, tile_prefix, R, W, offset_cur, cursor, R2,
-                        count_down ? offset_new : nullptr, nitems);
+  scatter_aligned_runs(reps, nreps, app_prefix, R, W, offset_cur, cursor, R2,
+                       count_down ? offset_new : nullptr);
   if (!grid_wait(gate.bar, gridDim.x)) {
     if (threadIdx.x == 0) atomicOr(err, 2u);
     return;
   }
-  sort_bins_tiles(reps, nreps, tile_prefix, R2, offset_new, T, nitems);
+  sort_bins_tiles(reps, nreps, tile_prefix, R2, offset_new, T, nitems, SortList{});
 }
 
 hipError_t launch_rebin_fallback(const WorkList& wl, Buf R, Buf W, const uint32_t* offset_cur,
@@ -1147,16 +1414,28 @@ hipError_t launch_rebin_fallback(const WorkList& wl, Buf R, Buf W, const uint32_
   if (!gate.flag || !gate.redone || !gate.bar || !err) return hipErrorInvalidValue;
   const uint32_t grid = wl.ntiles > kGatedGrid ? kGatedGrid : wl.ntiles;
   hipLaunchKernelGGL(k_rebin_fallback, dim3(grid), dim3(256), 0, s, wl.reps, wl.nreps,
-                     wl.tile_prefix, R, W, offset_cur, cursor, R2, offset_new, T, gate, err,
-                     count_down ? 1 : 0, wl.ntiles);
+                     wl.tile_prefix, wl.app_prefix, R, W, offset_cur, cursor, R2, offset_new, T,
+                     gate, err, count_down ? 1 : 0, wl.ntiles);
   return hipGetLastError();
 }
 
+// Work-groups of k_sort_list: enough to fill the GPU (about 8 per CU).
+constexpr uint32_t kSortListGrid = 2048;
+
 hipError_t launch_sort_bins(const WorkList& wl, Buf R, const uint32_t* offset, Buf T,
-                            hipStream_t s) {
+                            hipStream_t s, uint32_t* bins, uint32_t nbins, uint32_t* nlist) {
   if (wl.ntiles == 0) return hipSuccess;
+  SortList list;
+  if (bins) {
+    list.bin = bins;
+    list.n = nlist;
+    list.size = nbins;
+  }
   hipLaunchKernelGGL(k_sort_bins, dim3(wl.ntiles), dim3(kSortThreads), 0, s, wl.reps, wl.nreps,
-                     wl.tile_prefix, R, offset, T, wl.ntiles);
+                     wl.tile_prefix, R, offset, T, wl.ntiles, list);
+  if (bins)
+    hipLaunchKernelGGL(k_sort_list, dim3(kSortListGrid), dim3(kSortThreads), 0, s, wl.reps,
+                       wl.nreps, R, offset, T, list);
   return hipGetLastError();
 }
 

@@ -22,9 +22,11 @@ hipError_t launch_scan(uint32_t* count, uint32_t* offset, uint32_t* cursor, uint
                        const ScanState& ss, uint64_t* gstep, hipStream_t s,
                        uint32_t* gate = nullptr);
 
-// Moves every agent of W (aligned with R) to its new bin's cursor in R2.
+// Moves every agent of W (aligned with R, nagents of them) to its new bin's
+// cursor in R2; nlist (or null): launch_sort_bins' counters, cleared here.
 hipError_t launch_scatter_aligned(const WorkList& wl, Buf R, Buf W, const uint32_t* offset_cur,
-                                  uint32_t* cursor, Buf R2, hipStream_t s);
+                                  uint32_t* cursor, Buf R2, uint32_t nagents, uint32_t* nlist,
+                                  hipStream_t s);
 // The gather rebinning (one work-group per tile; tiles of at most
 // kGatherMaxBins bins) of the flock step that filled the outboxes: R2 in
 // bin order with every bin sorted, or gate.flag set for
@@ -36,9 +38,13 @@ hipError_t launch_rebin_gather(const WorkList& wl, Buf R, Buf W, const uint32_t*
 hipError_t launch_scatter_append(const WorkList& wl, Buf A, uint32_t* cursor, Buf R2,
                                  hipStream_t s);
 // Sorts every bin of R (offsets `offset`) by (cell y, id); T is scratch of
-// R's capacity whose contents are lost.
+// R's capacity whose contents are lost.  bins (nbins words) and nlist (two
+// words, cleared): the bins of more than 8 birds are listed there and sorted
+// by a second launch over the whole GPU (worth its launch where a rebinning
+// by scatter has left crowded tiles); or none.
 hipError_t launch_sort_bins(const WorkList& wl, Buf R, const uint32_t* offset, Buf T,
-                            hipStream_t s);
+                            hipStream_t s, uint32_t* bins = nullptr, uint32_t nbins = 0,
+                            uint32_t* nlist = nullptr);
 // The scatter and the bin sort of a gathered step in one launch, run only if
 // gate.flag is set (gate.redone counts such steps, gate.bar is the grid
 // wait's counter, zeroed by the gather): the scatter as

@@ -129,11 +129,12 @@ KG_HD void near_candidate(const RepDev& rp, int32_t col0, float qx, float qy, ui
                           NearAcc* acc) {
   const float dx = qx - c.x, dy = qy - c.y;
   const float s = dx * dx + dy * dy;
-  bool ok = s <= rp.sq_thresh;
-  if (s > rp.sq_sure && s <= rp.sq_near) {  // rare: the corners decide
+  bool ok = s <= rp.sq_sure;
+  if (!ok && s <= rp.sq_near) {  // rare: the corners decide
     const int32_t bx = col0 + (int32_t)(B.z[e] >> kNearRowBits);
     const int32_t by = (int32_t)(B.z[e] & ((1u << kNearRowBits) - 1u));
-    if (near_corners(rp.g, bx, by, qx, qy, rp.sq_thresh, ok ? -1 : 1)) ok = !ok;
+    const bool in = s <= rp.sq_thresh;
+    ok = near_corners(rp.g, bx, by, qx, qy, rp.sq_thresh, in ? -1 : 1) != in;
   }
   if (ok && cid != qid) acc->add(dx, dy, s, c.hx, c.hy);
 }
@@ -355,43 +356,55 @@ KG_HD uint32_t near_at(uint32_t k, uint32_t n0, uint32_t n1, uint32_t o0, uint32
   return k + o;
 }
 
-// The neighbour sums of the bird `qid` at (qx, qy) over window w.
-template <class Find>
+// The neighbour sums of the bird `qid` at (qx, qy) over window w.  kFlat: one
+// loop over the runs of three columns, else a loop per column (cheaper per
+// candidate where every run is long).  Two candidates to a trip, the next one
+// loaded while one is worked on.
+template <bool kFlat, class Find>
 KG_HD void near_walk(const RepDev& rp, int32_t col0, const NearWindow& w, float qx, float qy,
                      uint32_t qid, const Find& find, const NearBirds& B, NearAcc* acc) {
   if (w.cols < 0 || w.rows < 0) return;
   const uint32_t rows = (uint32_t)w.rows;
-  if (rp.disc_dist == 1) {
-    // one loop over the three columns' runs: a wave's trips are those of its
-    // busiest lane, not of each column's.  The next candidate is loaded while
-    // this one is worked on.
+  if (kFlat && rp.disc_dist == 1) {
+    // a wave's trips are those of its busiest lane, not of each column's
     uint32_t lo[3], hi[3];
     find.three(w.c, w.cols, w.row, rows, lo, hi);
     const uint32_t n0 = hi[0] - lo[0], n1 = n0 + hi[1] - lo[1], n = n1 + hi[2] - lo[2];
     const uint32_t o1 = lo[1] - n0, o2 = lo[2] - n1;
     const uint32_t o0 = lo[0];
     if (n == 0u) return;
-    uint32_t e = near_at(0u, n0, n1, o0, o1, o2);
+    uint32_t e = near_at(0u, n0, n1, o0, o1, o2), k = 0;
     NearRec c = B.rec[e];
     uint32_t id = B.id[e];
-    for (uint32_t k = 1;; ++k) {
-      // past the last candidate this is at most the sentinel
-      const uint32_t en = near_at(k, n0, n1, o0, o1, o2);
-      const NearRec cn = B.rec[en];
-      const uint32_t idn = B.id[en];
+    for (; k + 1u < n; k += 2) {
+      const uint32_t e1 = near_at(k + 1u, n0, n1, o0, o1, o2);
+      const NearRec c1 = B.rec[e1];
+      const uint32_t id1 = B.id[e1];
       near_candidate(rp, col0, qx, qy, qid, B, e, c, id, acc);
-      if (k == n) break;
-      e = en;
-      c = cn;
-      id = idn;
+      // past the last candidate this is at most the sentinel
+      e = near_at(k + 2u, n0, n1, o0, o1, o2);
+      c = B.rec[e];
+      id = B.id[e];
+      near_candidate(rp, col0, qx, qy, qid, B, e1, c1, id1, acc);
     }
+    if (k < n) near_candidate(rp, col0, qx, qy, qid, B, e, c, id, acc);
     return;
   }
   for (int32_t q = 0; q <= w.cols; ++q) {
     uint32_t lo, hi;
     find.one(w.c + q, w.row, rows, &lo, &hi);
-    for (uint32_t e = lo; e < hi; ++e)
-      near_candidate(rp, col0, qx, qy, qid, B, e, B.rec[e], B.id[e], acc);
+    if (lo >= hi) continue;
+    NearRec c = B.rec[lo];
+    uint32_t id = B.id[lo], e = lo;
+    for (; e + 1u < hi; e += 2) {
+      const NearRec c1 = B.rec[e + 1u];
+      const uint32_t id1 = B.id[e + 1u];
+      near_candidate(rp, col0, qx, qy, qid, B, e, c, id, acc);
+      c = B.rec[e + 2u];  // at most the sentinel
+      id = B.id[e + 2u];
+      near_candidate(rp, col0, qx, qy, qid, B, e + 1u, c1, id1, acc);
+    }
+    if (e < hi) near_candidate(rp, col0, qx, qy, qid, B, e, c, id, acc);
   }
 }
 
@@ -417,7 +430,7 @@ KG_HD bool near_any(const RepDev& rp, int32_t col0, const NearWindow& w, float q
 }
 
 // Bird::step of entry o.
-template <class Find>
+template <bool kFlat, class Find>
 KG_HD void near_step(const RepDev& rp, int32_t col0, uint64_t step, uint32_t o, const Find& find,
                      const NearBirds& B, NearRec* next) {
   const NearRec b = B.rec[o];
@@ -426,7 +439,7 @@ KG_HD void near_step(const RepDev& rp, int32_t col0, uint64_t step, uint32_t o, 
   const int32_t cy = (int32_t)(z & ((1u << kNearRowBits) - 1u));
   const NearWindow w = near_window(rp, col0, c, cy);
   NearAcc acc;
-  near_walk(rp, col0, w, b.x, b.y, id, find, B, &acc);
+  near_walk<kFlat>(rp, col0, w, b.x, b.y, id, find, B, &acc);
   bool found = acc.n != 0 || near_self(rp, b.x, b.y, col0 + c, cy);
   if (!found) found = near_any(rp, col0, w, b.x, b.y, find, B);
   near_finish(acc, found, rp.p, id, step, b.x, b.y, b.hx, b.hy, rp.g.w, &next->x, &next->y,
@@ -555,9 +568,68 @@ KG_HD void near_agent(const RepDev& rp, const FlockTile& ft, const NearChunk& k,
                       const NearSmem& S, Buf W, uint32_t* count_next, uint32_t* err,
                       const FlockSinks& lv) {
   NearRec r;
-  near_step(rp, ft.sc_lo, ft.step, S.own[o], TileFind{S.b.z, S.col_base, k.base}, S.b, &r);
+  near_step<true>(rp, ft.sc_lo, ft.step, S.own[o], TileFind{S.b.z, S.col_base, k.base}, S.b, &r);
   flock_emit(rp.g, rp.bin_base, W, k.own_lo + o, r.x, r.y, r.hx, r.hy, count_next, err, ft.tile,
              lv);
+}
+
+// ---- staging a run of birds ---------------------------------------------------
+//
+// A tile too full for LDS is stepped by runs of its birds, each with only its
+// own neighbourhood staged: the columns the run's windows reach, whole tile
+// height if the run spans columns, else the rows around its own.  A run of a
+// dense column is a dozen rows, so three short column pieces hold its
+// neighbours.
+
+// LDS of a piece (a tile's without the own list).
+KG_HD size_t near_piece_bytes(int cap, int cols) {
+  return near_birds_bytes((uint32_t)cap) + (size_t)(7 * cols + 1) * sizeof(uint32_t);
+}
+
+// The staged rectangle of birds that lie in columns [ca, cb], rows [r0, r1] of
+// tile ft: ft with its staged columns and rows replaced.
+KG_HD FlockTile near_piece(const RepDev& rp, FlockTile ft, int32_t ca, int32_t cb, int32_t r0,
+                           int32_t r1) {
+  const Geom& g = rp.g;
+  const int32_t dd = rp.disc_dist;
+  ft.sc_lo = imax(0, ca - dd);
+  ft.ncols = imax(cb, imin(g.max_x - 1, cb + dd)) - ft.sc_lo + 1;
+  ft.ry_lo = imax(0, r0 - dd);
+  ft.ry_hi = imax(r1, imin(g.max_y - 1, r1 + dd));
+  return ft;
+}
+
+// Stages item i (< col_base[ncols]) of a piece at slot i; false if it is not
+// near.
+KG_HD bool near_stage_piece(const RepDev& rp, const FlockTile& pt, uint32_t i, Buf R,
+                            const NearSmem& S) {
+  int32_t lo = 0, hi = pt.ncols;  // column c with col_base[c] <= i < col_base[c + 1]
+  while (hi - lo > 1) {
+    const int32_t mid = (lo + hi) >> 1;
+    if (S.col_base[mid] <= i) lo = mid;
+    else hi = mid;
+  }
+  uint32_t off = i - S.col_base[lo];
+  const uint32_t l0 = S.seg_len[3 * lo], l1 = S.seg_len[3 * lo + 1];
+  uint32_t gi = S.seg_start[3 * lo] + off;
+  if (off >= l0 + l1) gi = S.seg_start[3 * lo + 2] + (off - l0 - l1);
+  else if (off >= l0) gi = S.seg_start[3 * lo + 1] + (off - l0);
+  const NearRec r{R.x[gi], R.y[gi], R.hx[gi], R.hy[gi]};
+  S.b.rec[i] = r;
+  S.b.z[i] = ((uint32_t)lo << kNearRowBits) | (uint32_t)cell_axis(rp.g, r.y);
+  S.b.id[i] = R.id[gi];
+  return !near_bad(rp.g, r.x, r.y, r.hx, r.hy);
+}
+
+// Bird::step of read-buffer bird gi of a staged piece.
+KG_HD void near_agent_piece(const RepDev& rp, const FlockTile& pt, uint32_t gi, Buf R,
+                            const NearSmem& S, Buf W, uint32_t* count_next, uint32_t* err,
+                            const FlockSinks& lv) {
+  const int32_t c = cell_axis(rp.g, R.x[gi]) - pt.sc_lo;
+  const uint32_t slot = S.col_base[c] + S.seg_len[3 * c] + (gi - S.seg_start[3 * c + 1]);
+  NearRec r;
+  near_step<false>(rp, pt.sc_lo, pt.step, slot, TileFind{S.b.z, S.col_base, 0u}, S.b, &r);
+  flock_emit(rp.g, rp.bin_base, W, gi, r.x, r.y, r.hx, r.hy, count_next, err, pt.tile, lv);
 }
 
 }  // namespace kg

@@ -118,7 +118,7 @@ __global__ __launch_bounds__(kT) void k_resident(const RepDev* __restrict__ reps
       uint32_t id = 0;
       if (i < n) {
         id = S.b.id[i];
-        if (near) near_step(rp, 0, step0 + k, i, find, S.b, &r);
+        if (near) near_step<true>(rp, 0, step0 + k, i, find, S.b, &r);
         else full_step(rp, step0 + k, i, find, S.b, &r);
       }
       // j is the same on every lane: the birds stay in registers

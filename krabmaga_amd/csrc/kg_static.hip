@@ -211,7 +211,7 @@ extern "C" int kg_schedule_step_static(const kg_field_desc* desc, const kg_flock
   KG_HIP(launch_flock(wl, c.R, c.offset, c.W, c.count, c.gstep, c.err, lds_cap, c.gflag, n, s,
                       Outbox{}, false, nullptr, 0, near));
   KG_HIP(launch_scan(c.count, c.offset2, c.cursor, g.nbins, ss, nullptr, s));
-  KG_HIP(launch_scatter_aligned(wl, c.R, c.W, c.offset, c.cursor, out, s));
+  KG_HIP(launch_scatter_aligned(wl, c.R, c.W, c.offset, c.cursor, out, n, nullptr, s));
   KG_HIP(launch_sort_bins(wl, out, c.offset2, c.W, s));
   KG_HIP(hipMemcpyAsync(&e, c.err, sizeof(e), hipMemcpyDeviceToHost, s));
   KG_HIP(hipStreamSynchronize(s));

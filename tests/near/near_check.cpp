@@ -181,6 +181,55 @@ static int run(const Case& c, uint64_t seed) {
     std::printf("%s: bin counts differ\n", c.name);
     return 1;
   }
+  // runs of birds of one tile, staged with their neighbourhood only
+  // (k_flock_runs): whole tile height across columns, else the run's rows
+  uint32_t pieces = 0;
+  std::vector<uint64_t> big((near_smem_bytes((int)c.n, cols) + 7) / 8 + 2);
+  const NearSmem P = near_carve((uint8_t*)(((uintptr_t)big.data() + 15) & ~(uintptr_t)15),
+                                (int)c.n, cols);
+  for (int k = 0; k < 60; ++k) {
+    uint32_t s = (uint32_t)(rng() % c.n), e = s + 1u + (uint32_t)(rng() % 200u);
+    int32_t cx, cy;
+    discretize(g, R.x[s], R.y[s], &cx, &cy);
+    const FlockTile ft = flock_tile(&rp, 1, prefix, tile_of(g, cx, cy), 0);
+    e = std::min(e, offset[ft.tb1]);
+    if (k % 2) e = std::min(e, offset[rp.bin_base + col_bin0(g, ft.tile, cx & (g.tx - 1)) +
+                                      (uint32_t)g.tr]);
+    const int32_t ca = cell_axis(g, R.x[s]), cb = cell_axis(g, R.x[e - 1]);
+    const int32_t r0 = ca == cb ? cell_axis(g, R.y[s]) : ft.y0;
+    const int32_t r1 = ca == cb ? cell_axis(g, R.y[e - 1]) : ft.y1 - 1;
+    const FlockTile pt = near_piece(rp, ft, ca, cb, r0, r1);
+    if (pt.ncols > cols) {
+      std::printf("%s: a piece of %d columns\n", c.name, pt.ncols);
+      return 1;
+    }
+    uint32_t L = 0;
+    for (int t = 0; t < pt.ncols; ++t) {
+      P.col_base[t] = L;
+      L += flock_segments(rp, pt, t, offset.data(), P.seg_start, P.seg_len);
+    }
+    P.col_base[pt.ncols] = L;
+    bool ok = true;
+    for (uint32_t i = 0; i < L; ++i) ok = near_stage_piece(rp, pt, i, R.view(), P) && ok;
+    if (!ok) continue;
+    P.b.z[L] = ~0u;
+    const FlockSinks lv{Outbox{}, 0u, nullptr, nullptr, nullptr};
+    for (uint32_t gi = s; gi < e; ++gi) {
+      near_agent_piece(rp, pt, gi, R.view(), P, W.view(), cnt.data(), &err, lv);
+      flock_agent_global(rp, ft.step, gi, R.view(), offset.data(), V.view(), want.data(), &err2,
+                         lv);
+      if (!same(W.x[gi], V.x[gi]) || !same(W.y[gi], V.y[gi]) || !same(W.hx[gi], V.hx[gi]) ||
+          !same(W.hy[gi], V.hy[gi])) {
+        std::printf("%s: bird %u of a run differs\n", c.name, R.id[gi]);
+        return 1;
+      }
+    }
+    ++pieces;
+  }
+  if (pieces < 10 && c.headings != 2) {
+    std::printf("%s: %u runs\n", c.name, pieces);
+    return 1;
+  }
   std::printf("%s: %u of %u birds in %u chunks, %u tiles left to the general form\n", c.name,
               stepped, c.n, chunks, bad_tiles);
   return stepped * 4 < c.n ? 1 : 0;  // a scenario that skips most birds shows nothing

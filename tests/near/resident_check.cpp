@@ -155,7 +155,7 @@ static int run(const Case& c, uint64_t seed) {
       ResBird& q = b[i];
       NearRec r;
       if (bad) full_step(rp, k, i, find, S.b, &r);
-      else near_step(rp, 0, k, i, find, S.b, &r);
+      else near_step<true>(rp, 0, k, i, find, S.b, &r);
       q.x = r.x;
       q.y = r.y;
       q.hx = r.hx;
