@@ -7,6 +7,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
 #include <string>
 
 #include "../../include/krabgpu.h"
@@ -42,5 +43,42 @@ template <class T>
 hipError_t dmalloc(T** p, size_t n) {
   return hipMalloc((void**)p, (n ? n : 1) * sizeof(T));
 }
+
+// Pinned host memory of one object for reading small buffers (launch_pack),
+// allocated at the first read and given back with the object.  Larger buffers
+// are copied straight to the caller (past about 32,000 agents the copies'
+// bandwidth outweighs their calls).
+constexpr size_t kStageAgents = 32768;
+
+struct HostStage {
+  uint32_t* p = nullptr;
+  size_t words = 0;
+
+  static bool fits(size_t n) { return n <= kStageAgents; }
+  // Room for n agents (fits(n)); false if the allocation fails.
+  bool reserve(size_t n) {
+    const size_t want = kPackHead + 5 * n;
+    if (want <= words) return true;
+    release();
+    if (hipHostMalloc((void**)&p, want * sizeof(uint32_t)) != hipSuccess) {
+      p = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+    words = want;
+    return true;
+  }
+  // The n packed agents to the caller's arrays (any may be null).
+  void unpack(size_t n, uint32_t* ids, float* x, float* y, float* hx, float* hy) const {
+    void* const dst[5] = {x, y, hx, hy, ids};
+    for (size_t k = 0; k < 5; ++k)
+      if (dst[k] && n) std::memcpy(dst[k], p + kPackHead + k * n, n * sizeof(uint32_t));
+  }
+  void release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    words = 0;
+  }
+};
 
 }  // namespace kg

@@ -130,6 +130,7 @@ struct kg_ensemble {
   uint64_t* gstep = nullptr;
   int lds_cap = 1024;
   NearPlan near{};  // off unless every run is near
+  HostStage stage;
   int parity = 0;  // bin-grouped steps taken since the build, mod 2
   // two-step graphs by parity + 2 * gather
   std::vector<std::pair<int, hipGraphExec_t>> bgraphs;
@@ -836,6 +837,7 @@ void kg_ensemble_destroy(kg_ensemble* e) {
   if (!e) return;
   if (e->stream) (void)hipStreamSynchronize(e->stream);
   e->drop_bgraphs();
+  e->stage.release();
   e->rt.release();
   e->A.release();
   e->A2.release();
@@ -954,6 +956,16 @@ int kg_ensemble_read(kg_ensemble* e, uint32_t id, uint32_t* ids, float* x, float
   const Buf src = e->binned ? e->R.b : e->A.b;
   const size_t m = r->desc.agents;
   const uint32_t b = r->app_base;
+  if (HostStage::fits(m) && e->stage.reserve(kStageAgents)) {
+    KG_HIP(launch_pack(src, b, (uint32_t)m, e->binned ? nullptr : e->rep_cursor + idx, e->stage.p,
+                       e->stream));
+    KG_HIP(hipStreamSynchronize(e->stream));
+    if (!e->binned && e->stage.p[0] != r->desc.agents)
+      return set_error(KG_E_STATE, "run %u holds %u agents, expected %u", id, e->stage.p[0],
+                       r->desc.agents);
+    e->stage.unpack(m, ids, x, y, hx, hy);
+    return KG_OK;
+  }
   if (ids) KG_HIP(hipMemcpyAsync(ids, src.id + b, m * 4, hipMemcpyDeviceToHost, e->stream));
   if (x) KG_HIP(hipMemcpyAsync(x, src.x + b, m * 4, hipMemcpyDeviceToHost, e->stream));
   if (y) KG_HIP(hipMemcpyAsync(y, src.y + b, m * 4, hipMemcpyDeviceToHost, e->stream));

@@ -74,6 +74,7 @@ struct kg_field {
   // tiles; the first gather step of a field is checked on its own
   uint64_t gather_steps = 0, gather_steps_copied = 0;
   uint32_t* seen = nullptr;
+  HostStage stage;
   bool gather_probed = false;
   // no tile has taken the global path since the probe: k_flock steps such a
   // tile itself and k_flock_global is not launched
@@ -611,6 +612,7 @@ void kg_field_destroy(kg_field* f) {
   (void)hipFree(f->tsum[1]);
   (void)hipFree(f->count2);
   if (f->seen) (void)hipHostFree(f->seen);
+  f->stage.release();
   if (f->stream) (void)hipStreamDestroy(f->stream);
   delete f;
 }
@@ -1165,11 +1167,13 @@ int kg_read_agents(kg_field* f, int buffer, uint32_t* ids, float* x, float* y, f
                    float* hy, size_t cap, size_t* n) {
   clear_error();
   if (!f || !n) return set_error(KG_E_INVALID, "field and n must not be NULL");
-  if (int rc = sync_and_check(f)) return rc;
+  if (int rc = ensure_atomic(f)) return rc;
+  // unless a location left the grid (which the error flag tells), the read
+  // buffer holds every agent
   Buf src;
   uint32_t cnt;
   if (buffer == 0) {
-    KG_HIP(hipMemcpy(&cnt, f->offset + f->g.nbins, 4, hipMemcpyDeviceToHost));
+    cnt = f->nR;
     src = f->R.b;
   } else if (f->w_aligned) {
     cnt = f->nW;
@@ -1179,6 +1183,19 @@ int kg_read_agents(kg_field* f, int buffer, uint32_t* ids, float* x, float* y, f
     cnt = f->nA;
     src = f->A.b;
   }
+  if (cnt <= cap && HostStage::fits(cnt) && f->stage.reserve(cnt)) {
+    KG_HIP(launch_pack(src, 0, cnt, f->err, f->stage.p, f->stream));
+    KG_HIP(hipStreamSynchronize(f->stream));
+    if (f->stage.p[0]) {
+      f->poisoned = true;
+      f->poison_bits |= f->stage.p[0];
+    }
+    if (int rc = check_poison(f)) return rc;
+    f->stage.unpack(cnt, ids, x, y, hx, hy);
+    *n = cnt;
+    return KG_OK;
+  }
+  if (int rc = sync_only(f)) return rc;
   *n = cnt;
   if (cnt > cap) return set_error(KG_E_CAPACITY, "%u agents do not fit in %zu", cnt, cap);
   const size_t fb = (size_t)cnt * sizeof(float);

@@ -344,6 +344,26 @@ __global__ void k_materialize(Buf R, Buf W, uint32_t n, Buf A) {
   A.id[i] = R.id[i];
 }
 
+__global__ void k_pack(Buf src, uint32_t base, uint32_t n, const uint32_t* __restrict__ word,
+                       uint32_t* __restrict__ dst) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) dst[0] = word ? *word : 0u;
+  if (i >= n) return;
+  float* const f = (float*)(dst + kPackHead);
+  f[i] = src.x[base + i];
+  f[(size_t)n + i] = src.y[base + i];
+  f[2 * (size_t)n + i] = src.hx[base + i];
+  f[3 * (size_t)n + i] = src.hy[base + i];
+  dst[kPackHead + 4 * (size_t)n + i] = src.id[base + i];
+}
+
+hipError_t launch_pack(Buf src, uint32_t base, uint32_t n, const uint32_t* word, uint32_t* dst,
+                       hipStream_t s) {
+  hipLaunchKernelGGL(k_pack, dim3(n ? (n + 255) / 256 : 1), dim3(256), 0, s, src, base, n, word,
+                     dst);
+  return hipGetLastError();
+}
+
 hipError_t launch_materialize(Buf R, Buf W, uint32_t n, Buf A, hipStream_t s) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_materialize, dim3((n + 255) / 256), dim3(256), 0, s, R, W, n, A);

@@ -82,6 +82,14 @@ hipError_t launch_flock(const WorkList& wl, Buf R, const uint32_t* offset, Buf W
                         const Outbox& ob = Outbox{}, bool inline_global = false,
                         uint32_t* tile_sum = nullptr, uint32_t global_grid = 0,
                         const NearPlan& near = NearPlan{});
+// Agents [base, base + n) of src to dst, pinned host memory (x, y, hx, hy, id,
+// n words each), after kPackHead words of which the first is *word (0 without
+// one): one launch and one wait bring a small buffer to the host, where
+// copies array by array cost about 12 us each.
+constexpr uint32_t kPackHead = 16;
+hipError_t launch_pack(Buf src, uint32_t base, uint32_t n, const uint32_t* word, uint32_t* dst,
+                       hipStream_t s);
+
 hipError_t launch_materialize(Buf R, Buf W, uint32_t n, Buf A, hipStream_t s);
 
 // nsteps (<= kResidentSteps) schedule steps of runs list[0 .. nruns) (or runs

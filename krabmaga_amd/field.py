@@ -207,19 +207,23 @@ class Field2D:
         check(self._L.kg_schedule_run(self._h, ctypes.byref(p), first_step, nsteps, flags))
 
     def read_agents(self, buffer=0):
+        # a buffer never holds more than the capacity: one call does for all
+        # but very large fields, which are asked for their count first
         n = ctypes.c_size_t()
-        rc = self._L.kg_read_agents(self._h, buffer, None, None, None, None, None, 0,
-                                    ctypes.byref(n))
-        if rc not in (_abi.KG_OK, _abi.KG_E_CAPACITY):
+        m = min(self.capacity, 1 << 20)
+        while True:
+            out = {"id": np.empty(m, np.uint32)}
+            for k in ("x", "y", "hx", "hy"):
+                out[k] = np.empty(m, np.float32)
+            rc = self._L.kg_read_agents(self._h, buffer, u32p(out["id"]), f32p(out["x"]),
+                                        f32p(out["y"]), f32p(out["hx"]), f32p(out["hy"]), m,
+                                        ctypes.byref(n))
+            if rc == _abi.KG_E_CAPACITY:
+                m = int(n.value)
+                continue
             check(rc)
-        m = int(n.value)
-        out = {"id": np.zeros(m, np.uint32), "x": np.zeros(m, np.float32),
-               "y": np.zeros(m, np.float32), "hx": np.zeros(m, np.float32),
-               "hy": np.zeros(m, np.float32)}
-        check(self._L.kg_read_agents(self._h, buffer, u32p(out["id"]), f32p(out["x"]),
-                                     f32p(out["y"]), f32p(out["hx"]), f32p(out["hy"]), m,
-                                     ctypes.byref(n)))
-        return out
+            break
+        return out if n.value == m else {k: v[: n.value].copy() for k, v in out.items()}
 
     def state_by_id(self, buffer=0):
         """Read buffer as a (4, n) array [x, y, hx, hy] indexed by id 0..n-1."""
