@@ -8,9 +8,8 @@ from the seeded Philox stream.  One step = one Schedule::step of the
 flockers model: neighbour query + Bird::step for every agent and the
 rebinning of the field (lazy_update).  State is resident in HBM before the
 timed region starts.  The headline runs the field's default path (at this
-size the three-kernel path: k_flock, then k_rebin_gather, which also does
-the bin-count scan, then k_rebin_fallback, the scatter and bin sort that
-run only in a step the gather could not rebin); the tile-resident step
+size the three-kernel path: k_flock_near, then k_rebin_gather, which also
+does the bin-count scan); the tile-resident step
 (one k_rt_step launch per tile class) is timed beside it from the same
 initial state.
 
@@ -527,9 +526,8 @@ def main():
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": ("schedule step: k_flock + k_rebin_gather (which does the bin-count "
-                       "scan in this run) + k_rebin_fallback (scatter and bin sort; returns "
-                       "at once unless the gather could not rebin the step)"
+            "kernel": ("schedule step: k_flock_near + k_rebin_gather (which does the "
+                       "bin-count scan in this run)"
                        if three else "schedule step: all k_rt_step launches of the step"),
             "launch_us": step_us,
             "unit_of_launch": "one schedule step",

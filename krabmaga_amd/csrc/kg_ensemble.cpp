@@ -135,9 +135,9 @@ struct kg_ensemble {
   // two-step graphs by parity + 2 * gather
   std::vector<std::pair<int, hipGraphExec_t>> bgraphs;
   // gather rebinning (every run's tiles of at most kGatherMaxBins bins): the
-  // lists of leavers, the gate words (a flag per step parity, steps redone,
-  // the fallback's grid-wait counter) and the redone
-  // count at the last check; a layout whose steps fail it drops it
+  // lists of leavers, the gate words (a flag per step parity, the steps with
+  // a tile rebinned the slow way) and that count at the last check; a layout
+  // with such steps drops it
   bool gather = false;
   Outbox outbox{};
   size_t cap_outbox = 0;
@@ -367,7 +367,7 @@ int reserve_binned(kg_ensemble* e, size_t agents, size_t tiles) {
       return set_error(KG_E_NOMEM, "ensemble outboxes: %s", hipGetErrorString(err));
     e->cap_outbox = n;
   }
-  if (!e->gate && (err = dmalloc(&e->gate, 4)) != hipSuccess)
+  if (!e->gate && (err = dmalloc(&e->gate, 3)) != hipSuccess)
     return set_error(KG_E_NOMEM, "ensemble gate: %s", hipGetErrorString(err));
   return KG_OK;
 }
@@ -569,8 +569,9 @@ int ready_binned(kg_ensemble* e) {
   e->near = near ? near_plan(cap, cols, e->ntiles) : NearPlan{};
   e->gather = rebin_gather_enabled();
   for (const RepDev& rp : e->h_reps)
-    if ((uint32_t)(rp.g.tx * rp.g.tr) > kGatherMaxBins) e->gather = false;
-  KG_HIP(hipMemsetAsync(e->gate, 0, 4 * sizeof(uint32_t), e->stream));
+    if ((uint32_t)(rp.g.tx * rp.g.tr) > kGatherMaxBins || !gather_reaches(rp.g, rp.p.jump))
+      e->gather = false;
+  KG_HIP(hipMemsetAsync(e->gate, 0, 3 * sizeof(uint32_t), e->stream));
   e->redone_seen = 0;
   e->binned_ready = true;
   return KG_OK;
@@ -593,8 +594,8 @@ int resident_steps(kg_ensemble* e, uint32_t n) {
 }
 
 // One bin-grouped schedule step of every replica: k_flock over all tiles,
-// the scan over all bins (it advances the step counter), the gather (the
-// scatter and the bin sort only if it cannot), then the buffers swap.
+// the scan over all bins (it advances the step counter), the gather (or the
+// scatter and the bin sort), then the buffers swap.
 // k_flock_global's work-groups in an ensemble step: a layout of many runs
 // seldom has a global-path tile, and a grid of one work-group per run of
 // birds costs about 20 us at 23M birds just to launch and leave.
@@ -617,7 +618,7 @@ hipError_t binned_step(kg_ensemble* e, const WorkList& w) {
   else err = launch_scan(e->count, e->offset2, e->cursor, e->nbins, e->ss, e->gstep, e->stream, gate);
   if (err != hipSuccess) return err;
   const Gate gt{gate, gate ? e->gate + 2 : nullptr, summed ? e->gate + (p ^ 1) : nullptr,
-                gate ? e->gate + 3 : nullptr};
+                e->err};
   if (gate) {
     GatherScan sc;
     if (summed) {
@@ -632,12 +633,6 @@ hipError_t binned_step(kg_ensemble* e, const WorkList& w) {
     }
     if ((err = launch_rebin_gather(w, e->R.b, e->W.b, e->offset, e->offset2, e->outbox, e->R2.b,
                                    gt, sc, e->stream)) != hipSuccess)
-      return err;
-    // what the gather could not rebin, in one launch (the write buffer,
-    // consumed by the scatter, is the sort's scratch)
-    if ((err = launch_rebin_fallback(w, e->R.b, e->W.b, e->offset,
-                                     summed ? e->counts(p) : e->cursor, e->R2.b, e->offset2,
-                                     e->W.b, gt, e->err, summed, e->stream)) != hipSuccess)
       return err;
   } else {
     if ((err = launch_scatter_aligned(w, e->R.b, e->W.b, e->offset, e->cursor, e->R2.b,
@@ -757,14 +752,13 @@ int check_flags(kg_ensemble* e) {
   if (e->binned) {
     uint32_t errflag = 0;
     KG_HIP(hipMemcpy(&errflag, e->err, sizeof(errflag), hipMemcpyDeviceToHost));
-    if (errflag & 2u)
-      return set_error(KG_E_HIP, "the rebinning fallback's grid-wide wait timed out");
+    if (errflag & 2u) return set_error(KG_E_STATE, "a rebinning lost agents");
     if (errflag & 4u)
       return set_error(KG_E_STATE, "the resident step found more birds than it was planned for");
     if (errflag) return set_error(KG_E_RANGE, "an agent left its run's bag grid");
     if (e->gather) {
-      // steps the gather could not rebin since the last check: a layout
-      // that keeps failing it pays for it and for the scatter and the sort
+      // steps with a tile rebinned the slow way since the last check: from
+      // then on the layout rebins by scatter and sort
       uint32_t redone = 0;
       KG_HIP(hipMemcpy(&redone, e->gate + 2, sizeof(redone), hipMemcpyDeviceToHost));
       if (redone != e->redone_seen) e->gather = false;

@@ -63,14 +63,15 @@ struct kg_field {
   uint32_t* gflag = nullptr;
   // gather rebinning (tiles of at most kGatherMaxBins bins): the flock
   // kernel's lists of leavers, the gate words (a flag per step parity, the
-  // steps redone, the fallback's grid-wait counter) and whether the last
-  // flock step filled the lists
+  // steps with a tile rebinned the slow way) and whether the last flock step
+  // filled the lists
   bool gather_ok = false;
+  bool gathers() const { return gather_ok && gather_reaches(g, h_rep.p.jump); }
   Outbox outbox{};
   uint32_t* gate = nullptr;
   bool outbox_filled = false;
   // steps run with the gather; the counts the host last saw (pinned, copied
-  // after every run): [0] steps the gather could not rebin, [1] global-path
+  // after every run): [0] steps with a tile the gather took the slow way, [1] global-path
   // tiles; the first gather step of a field is checked on its own
   uint64_t gather_steps = 0, gather_steps_copied = 0;
   uint32_t* seen = nullptr;
@@ -177,9 +178,8 @@ int prof_collect(kg_field* f) {
 
 int check_poison(kg_field* f) {
   if (f->poisoned && (f->poison_bits & 2u))
-    return set_error(KG_E_HIP,
-                     "the rebinning fallback's grid-wide wait timed out in an earlier step; "
-                     "the field is unusable");
+    return set_error(KG_E_STATE, "a rebinning lost agents in an earlier step; the field is "
+                                 "unusable");
   if (f->poisoned && (f->poison_bits & 4u))
     return set_error(KG_E_STATE, "the resident step found more birds than it was planned for");
   if (f->poisoned)
@@ -229,8 +229,7 @@ int upload_rep(kg_field* f) {
 int lazy_update_impl(kg_field* f, uint64_t* step_gstep) {
   WorkList wl = f->worklist();
   // a flock step's output with its lists of leavers and nothing appended:
-  // the gather rebins it, the scatter and the bin sort run only if it
-  // sets the gate
+  // the gather rebins it
   const bool gather = f->w_aligned && f->outbox_filled && f->nA == 0;
   const int p = f->parity;
   uint32_t* gate = gather ? f->gate + p : nullptr;
@@ -247,7 +246,7 @@ int lazy_update_impl(kg_field* f, uint64_t* step_gstep) {
                        gate));
   }
   const Gate gt{gate, gather ? f->gate + 2 : nullptr, summed ? f->gate + (p ^ 1) : nullptr,
-                gather ? f->gate + 3 : nullptr};
+                f->err};
   if (f->w_aligned) {
     ProfScope ps(f, KG_KERNEL_SCATTER);
     if (gather) {
@@ -263,12 +262,6 @@ int lazy_update_impl(kg_field* f, uint64_t* step_gstep) {
       }
       KG_HIP(launch_rebin_gather(wl, f->R.b, f->W.b, f->offset, f->offset2, f->outbox,
                                  f->R2.b, gt, sc, f->stream));
-      // what the gather could not rebin: scatter and bin sort in one launch
-      // (no appended agents in a gathered step); the write buffer has been
-      // consumed by then and is the sort's scratch
-      KG_HIP(launch_rebin_fallback(wl, f->R.b, f->W.b, f->offset,
-                                   summed ? f->counts(p) : f->cursor, f->R2.b, f->offset2,
-                                   f->W.b, gt, f->err, summed, f->stream));
     } else {
       KG_HIP(launch_scatter_aligned(wl, f->R.b, f->W.b, f->offset, f->cursor, f->R2.b, f->nW,
                                     f->ss.partial, f->stream));
@@ -305,13 +298,14 @@ int lazy_update_impl(kg_field* f, uint64_t* step_gstep) {
 
 int flock_impl(kg_field* f, const uint64_t* gstep) {
   ProfScope ps(f, KG_KERNEL_FLOCK);
-  const bool summed = f->gather_ok && f->summed;
+  const bool gather = f->gathers();
+  const bool summed = gather && f->summed;
   KG_HIP(launch_flock(f->worklist(), f->R.b, f->offset, f->W.b,
                       summed ? f->counts(f->parity) : f->count, gstep, f->err,
                       f->lds_cap, f->gflag, (uint32_t)f->nR, f->stream,
-                      f->gather_ok ? f->outbox : Outbox{}, f->global_inline,
+                      gather ? f->outbox : Outbox{}, f->global_inline,
                       summed ? f->tsum[f->parity] : nullptr, 0, f->near));
-  f->outbox_filled = f->gather_ok;
+  f->outbox_filled = gather;
   f->nW = f->nR;
   f->w_aligned = true;
   return KG_OK;
@@ -549,8 +543,8 @@ int kg_field_create(const kg_field_desc* desc, kg_field** out) {
     if ((e = dmalloc(&f->outbox.n, f->g.ntiles)) != hipSuccess) return fail(e);
     if ((e = dmalloc(&f->outbox.slot, (size_t)f->g.ntiles * kOutboxCap)) != hipSuccess)
       return fail(e);
-    if ((e = dmalloc(&f->gate, 4)) != hipSuccess) return fail(e);
-    if ((e = hipMemset(f->gate, 0, 4 * sizeof(uint32_t))) != hipSuccess) return fail(e);
+    if ((e = dmalloc(&f->gate, 3)) != hipSuccess) return fail(e);
+    if ((e = hipMemset(f->gate, 0, 3 * sizeof(uint32_t))) != hipSuccess) return fail(e);
     if ((e = dmalloc(&f->count2, nb)) != hipSuccess) return fail(e);
     if ((e = hipMemset(f->count2, 0, nb * sizeof(uint32_t))) != hipSuccess) return fail(e);
     if ((e = hipHostMalloc((void**)&f->seen, 2 * sizeof(uint32_t))) != hipSuccess)
@@ -1071,9 +1065,8 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
   }
   if (int rc = ensure_atomic(f)) return rc;
   if (int rc = set_params(f, p, first_step)) return rc;
-  // a field whose steps fail the gather (tiles too full, long jumps) pays
-  // for it and for the scatter and the sort: it rebins by scatter and sort
-  // from then on.  The first gather step is checked at once (one
+  // a field whose steps take the gather's slow way (tiles too full) rebins by
+  // scatter and sort from then on.  The first gather step is checked at once (one
   // synchronisation per field), later ones from the count copied after each
   // run, which may lag a run behind: it is only a hint.
   // Likewise a field whose tiles took the global path (counted by k_flock)
@@ -1085,7 +1078,7 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
   if (f->global_inline && seen[1] != 0) f->global_inline = false;
   KG_HIP(hipMemsetAsync(f->gstep, 0, sizeof(uint64_t), f->stream));
   uint32_t left = nsteps;
-  if (f->gather_ok && !f->gather_probed) {
+  if (f->gathers() && !f->gather_probed) {
     if (int rc = run_direct_step(f)) return rc;
     --left;
     uint32_t counts[2] = {0, 0};
@@ -1103,7 +1096,7 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
   // one sum), whose tiles fit the LDS histogram and whole scan tiles
   const uint32_t nbt = (uint32_t)(f->g.tx * f->g.tr);
   const uint32_t nscan = (f->g.nbins + kScanTile - 1) / kScanTile;
-  f->summed = f->gather_ok && f->global_inline && nscan <= kScanInlineTiles &&
+  f->summed = f->gathers() && f->global_inline && nscan <= kScanInlineTiles &&
               nbt <= kGatherMaxBins && (uint32_t)kScanTile % nbt == 0;
   if (f->summed) {
     for (int k = 0; k < 2; ++k)
@@ -1114,7 +1107,7 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
     GraphKey key;
     std::memcpy(key.params, p, sizeof(kg_flock_params));
     key.parity = f->parity;
-    key.gather = f->gather_ok ? 1 : 0;
+    key.gather = f->gathers() ? 1 : 0;
     key.inline_global = f->global_inline ? 1 : 0;
     auto it = f->graphs.find(key);
     hipGraphExec_t exec = nullptr;
@@ -1145,7 +1138,7 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
     if (int rc = run_direct_step(f)) return rc;
     --left;
   }
-  if (f->gather_ok) {
+  if (f->gathers()) {
     f->gather_steps += nsteps;
     KG_HIP(hipMemcpyAsync(f->seen, f->gate + 2, sizeof(uint32_t), hipMemcpyDeviceToHost,
                           f->stream));

@@ -88,18 +88,16 @@ hipError_t launch_scatter_append(const WorkList& wl, Buf A, uint32_t* cursor, Bu
 // the current read buffer, whose slots are taken kScatterRun at a time, a run
 // to a work-group, so a crowded tile is spread over the GPU (one work-group
 // per tile took 270 us for 8.4M birds in blobs of up to 37k birds per tile,
-// most of it in a few hundred work-groups).  fill_base null:
-// cursor[b] is bin b's next free slot; else cursor[b] is bin b's count of
-// agents still to place, and they go to fill_base[b] + count - 1 downwards
-// (the count ends at zero).
+// most of it in a few hundred work-groups). 
+// cursor[b] is bin b's next free slot.
 constexpr uint32_t kScatterRun = 1024;
 
 __device__ __forceinline__ void scatter_aligned_runs(const RepDev* __restrict__ reps, int nreps,
                                                      const uint32_t* __restrict__ app_prefix,
                                                      Buf R, Buf W,
                                                      const uint32_t* __restrict__ offset_cur,
-                                                     uint32_t* __restrict__ cursor, Buf R2,
-                                                     const uint32_t* __restrict__ fill_base) {
+                                                     uint32_t* __restrict__ cursor,
+                                                     Buf R2) {
   const RepDev& end = reps[nreps - 1];
   const uint32_t n = offset_cur[end.bin_base + end.g.nbins];
   const uint32_t nruns = (n + kScatterRun - 1) / kScatterRun;
@@ -144,8 +142,7 @@ __device__ __forceinline__ void scatter_aligned_runs(const RepDev* __restrict__ 
       uint32_t base = 0;
       if (head) {
         const uint32_t len = (uint32_t)__popcll(vmask & from_h & to_nh);
-        base = fill_base ? fill_base[bin] + atomicSub(&cursor[bin], len) - len
-                         : atomicAdd(&cursor[bin], len);
+        base = atomicAdd(&cursor[bin], len);
       }
       base = __shfl(base, h, kWave);
       if (valid) {
@@ -168,13 +165,8 @@ __global__ __launch_bounds__(256) void k_scatter_aligned(const RepDev* __restric
                                                          uint32_t* __restrict__ cursor, Buf R2,
                                                          uint32_t* __restrict__ nlist) {
   if (nlist && blockIdx.x == 0 && threadIdx.x < 2) nlist[threadIdx.x] = 0u;  // for the sort
-  scatter_aligned_runs(reps, nreps, app_prefix, R, W, offset_cur, cursor, R2, nullptr);
+  scatter_aligned_runs(reps, nreps, app_prefix, R, W, offset_cur, cursor, R2);
 }
-
-// Work-groups of the gated fallback: in most steps they only read the gate
-// (a launch costs in proportion to its work-groups), and in a step they redo
-// they loop over the tiles.
-constexpr uint32_t kGatedGrid = 256;
 
 hipError_t launch_scatter_aligned(const WorkList& wl, Buf R, Buf W, const uint32_t* offset_cur,
                                   uint32_t* cursor, Buf R2, uint32_t nagents, uint32_t* nlist,
@@ -183,154 +175,6 @@ hipError_t launch_scatter_aligned(const WorkList& wl, Buf R, Buf W, const uint32
   hipLaunchKernelGGL(k_scatter_aligned, dim3((nagents + kScatterRun - 1) / kScatterRun),
                      dim3(256), 0, s, wl.reps, wl.nreps, wl.app_prefix, R, W, offset_cur, cursor,
                      R2, nlist);
-  return hipGetLastError();
-}
-
-// The gather rebinning: one work-group per tile, phases in kg_phases.hpp.
-// Each thread keeps its candidates in registers from load to store, so a
-// bird is read once and written once; a tile with more candidates (or new
-// birds) than kGatherCap sends the step to the scatter and the bin sort.
-// With sc.count the work-group also does the scan's part for its tile: its
-// bins' new offsets follow from the earlier scan tiles' sums and the counts
-// of the earlier bins of its own scan tile (read from this step's counts,
-// which nothing clears in this step), and it writes them to offset_new.
-__global__ __launch_bounds__(kGatherThreads) void k_rebin_gather(
-    const RepDev* __restrict__ reps, int nreps, const uint32_t* __restrict__ tile_prefix, Buf R,
-    Buf W, const uint32_t* __restrict__ offset_cur, uint32_t* __restrict__ offset_new, Outbox ob,
-    Buf R2, Gate gate, GatherScan sc) {
-  __shared__ uint32_t s_warp[kGatherThreads / kWave];
-  __shared__ uint32_t s_bstart[kGatherMaxBins + 1];
-  __shared__ uint32_t s_fill[kGatherMaxBins];
-  __shared__ uint64_t s_key[kGatherCap];
-  __shared__ uint32_t s_sitem[kGatherSources], s_scnt[kGatherSources];
-  __shared__ uint32_t s_fail;
-  const uint32_t t = threadIdx.x;
-  const uint32_t item = xcd_remap(blockIdx.x, gridDim.x);
-  const int r = find_rep(tile_prefix, nreps, item);
-  const RepDev& rp = reps[r];
-  const Geom& g = rp.g;
-  const uint32_t tile = item - tile_prefix[r];
-  const uint32_t nbt = 1u << (g.tx_log2 + g.tr_log2);
-  const uint32_t tb0 = rp.bin_base + tile * nbt;
-  const uint32_t lo = offset_cur[tb0], nown = offset_cur[tb0 + nbt] - lo;
-  if (gate.bar && item == 0 && t == 0) *gate.bar = 0u;  // for the fallback's grid wait
-  uint32_t nlo;
-  if (sc.count) {
-    // before the tile: the earlier scan tiles' sums and the earlier bins of
-    // its own scan tile; one bin per thread (nbt <= kGatherThreads)
-    const uint32_t q = tb0 / (uint32_t)kScanTile;
-    uint32_t part = 0;
-    if (!sc.prefixed)
-      for (uint32_t i = t; i < q; i += kGatherThreads) part += sc.tile_sum[i];
-    else if (t == 0)
-      part = sc.tile_sum[q];
-    for (uint32_t b = q * (uint32_t)kScanTile + t; b < tb0; b += kGatherThreads)
-      part += sc.count[b];
-    block_exclusive_scan<kGatherThreads>(part, s_warp, &nlo);
-    const uint32_t c = t < nbt ? sc.count[tb0 + t] : 0u;
-    uint32_t tot;
-    const uint32_t ex = block_exclusive_scan<kGatherThreads>(c, s_warp, &tot);
-    if (t < nbt) {
-      s_bstart[t] = ex;
-      offset_new[tb0 + t] = nlo + ex;
-      if (sc.cursor) sc.cursor[tb0 + t] = nlo + ex;
-      sc.count_next[tb0 + t] = 0u;
-    }
-    if (tile == (uint32_t)g.ntiles - 1u) {
-      // bins between this replica's last and the next replica's first (on
-      // the next scan tile) hold nobody: they start where this tile ends
-      const uint32_t pad_end = min(sc.nbins, (tb0 + nbt + (uint32_t)kScanTile - 1u) /
-                                                 (uint32_t)kScanTile * (uint32_t)kScanTile);
-      for (uint32_t b = tb0 + nbt + t; b < pad_end; b += kGatherThreads) offset_new[b] = nlo + tot;
-    }
-    if (t == 0) {
-      s_bstart[nbt] = tot;
-      if (item == sc.last_item) offset_new[sc.nbins] = nlo + tot;
-      if (tb0 % (uint32_t)kScanTile == 0) sc.tile_sum_next[q] = 0u;
-      if (item == 0) {
-        *sc.gstep += 1;
-        if (gate.clear) *gate.clear = 0u;
-      }
-    }
-  } else {
-    nlo = offset_new[tb0];
-    for (uint32_t b = t; b <= nbt; b += kGatherThreads) s_bstart[b] = offset_new[tb0 + b] - nlo;
-  }
-  if (t < kGatherSources) {
-    const int32_t sl = gather_source(g, tile, t);
-    const uint32_t it = sl >= 0 ? tile_prefix[r] + (uint32_t)sl : 0u;
-    s_sitem[t] = it;
-    s_scnt[t] = sl >= 0 ? ob.n[it] : 0u;
-  }
-  if (t == 0) s_fail = 0u;
-  __syncthreads();
-  uint32_t ncand = nown;
-  for (uint32_t q = 0; q < kGatherSources; ++q) ncand += s_scnt[q];
-  if (t == 0 && (ncand > kGatherCap || s_bstart[nbt] > kGatherCap)) s_fail = 1u;
-  if (t < kGatherSources && s_scnt[t] > kOutboxCap) s_fail = 1u;
-  for (uint32_t b = t; b < nbt; b += kGatherThreads) {
-    if (s_bstart[b + 1] - s_bstart[b] > kGatherBinMax) s_fail = 1u;
-    s_fill[b] = 0u;
-  }
-  __syncthreads();
-  // s_fail is read only between barriers, so every thread takes the same path
-  if (!s_fail) {
-    // per candidate: (bin << 16 | slot in the bin) or ~0, and the bird
-    uint32_t cbs[kGatherRegs], cid[kGatherRegs];
-    float cx[kGatherRegs], cy[kGatherRegs], chx[kGatherRegs], chy[kGatherRegs];
-#pragma unroll
-    for (uint32_t u = 0; u < kGatherRegs; ++u) {
-      cbs[u] = ~0u;
-      const uint32_t k = t + u * kGatherThreads;
-      if (k < ncand) {
-        const uint32_t src = gather_src(ob, s_sitem, s_scnt, lo, nown, k);
-        cx[u] = W.x[src];
-        cy[u] = W.y[src];
-        chx[u] = W.hx[src];
-        chy[u] = W.hy[src];
-        cid[u] = R.id[src];
-        int32_t row;
-        const uint32_t b = gather_bin(g, tile, cx[u], cy[u], &row);
-        if (b < nbt) {
-          const uint32_t slot = atom_add(&s_fill[b], 1u);
-          if (slot < s_bstart[b + 1] - s_bstart[b]) {
-            s_key[s_bstart[b] + slot] = ((uint64_t)(uint32_t)row << 32) | cid[u];
-            cbs[u] = (b << 16) | slot;
-          } else {
-            s_fail = 1u;
-          }
-        }
-      }
-    }
-    __syncthreads();
-    for (uint32_t b = t; b < nbt; b += kGatherThreads)
-      if (s_fill[b] != s_bstart[b + 1] - s_bstart[b]) s_fail = 1u;
-    __syncthreads();
-    if (!s_fail) {
-#pragma unroll
-      for (uint32_t u = 0; u < kGatherRegs; ++u) {
-        if (cbs[u] == ~0u) continue;
-        const uint32_t b = cbs[u] >> 16;
-        const uint32_t e = s_bstart[b] + (cbs[u] & 0xFFFFu);
-        const uint32_t pos = nlo + s_bstart[b] + gather_rank(s_key, s_bstart[b], s_bstart[b + 1], e,
-                                                             s_key[e]);
-        R2.x[pos] = cx[u];
-        R2.y[pos] = cy[u];
-        R2.hx[pos] = chx[u];
-        R2.hy[pos] = chy[u];
-        R2.id[pos] = cid[u];
-      }
-    }
-  }
-  if (t == 0 && s_fail) *gate.flag = 1u;
-}
-
-hipError_t launch_rebin_gather(const WorkList& wl, Buf R, Buf W, const uint32_t* offset_cur,
-                               uint32_t* offset_new, const Outbox& ob, Buf R2, const Gate& gate,
-                               const GatherScan& sc, hipStream_t s) {
-  if (wl.ntiles == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_rebin_gather, dim3(wl.ntiles), dim3(kGatherThreads), 0, s, wl.reps,
-                     wl.nreps, wl.tile_prefix, R, W, offset_cur, offset_new, ob, R2, gate, sc);
   return hipGetLastError();
 }
 
@@ -1374,68 +1218,373 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_list(const RepDev* __rest
   }
 }
 
-// Waits until all `nblocks` work-groups of the grid have arrived at `bar`
-// (zeroed before the launch), with every write the grid made before it
-// visible to every work-group after it.  The fallback's 256 work-groups are
-// all resident at once on this GPU; the wait still ends after kGridWaitTicks
-// of the 100 MHz wall clock, returning false, so no launch can hang on it.
-constexpr uint64_t kGridWaitTicks = 10000000;  // 100 ms
-
-__device__ bool grid_wait(uint32_t* bar, uint32_t nblocks) {
-  __shared__ uint32_t s_ok;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __threadfence();
-    __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    const uint64_t t0 = wall_clock64();
-    uint32_t ok = 1u;
-    while (__hip_atomic_load(bar, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < nblocks) {
-      if (wall_clock64() - t0 > kGridWaitTicks) {
-        ok = 0u;
-        break;
+// A bin [s, s + m) of R by the whole work-group in place: up to kGatherCap
+// entries held in registers and ranked against the keys in s_key, more by a
+// bitonic network over memory (every comparator puts the smaller key at the
+// lower index, so entries past the end need not exist).
+__device__ __forceinline__ void sort_bin_in_place(const Geom& g, Buf R, uint32_t s, uint32_t m,
+                                                  uint64_t* s_key) {
+  constexpr uint32_t kT = kGatherThreads, kRegs = kGatherRegs;
+  const uint32_t t = threadIdx.x;
+  if (m <= kGatherCap) {
+    float x[kRegs], y[kRegs], hx[kRegs], hy[kRegs];
+    uint32_t id[kRegs];
+#pragma unroll
+    for (uint32_t u = 0; u < kRegs; ++u) {
+      const uint32_t e = t + u * kT;
+      if (e < m) {
+        x[u] = R.x[s + e];
+        y[u] = R.y[s + e];
+        hx[u] = R.hx[s + e];
+        hy[u] = R.hy[s + e];
+        id[u] = R.id[s + e];
+        s_key[e] = bin_key(g, y[u], id[u]);
       }
-      __builtin_amdgcn_s_sleep(4);
     }
-    __threadfence();
-    s_ok = ok;
-  }
-  __syncthreads();
-  return s_ok != 0u;
-}
-
-// The rebinning a gathered step could not do, in one launch: the scatter of
-// every tile, a grid-wide wait, then the bin sort of every tile (T: the
-// sort's scratch).  Returns at once unless the gate is set.  count_down:
-// cursor holds this step's bin counts, counted down from offset_new (the
-// summed steps' gather writes no cursors).  A wait that times out sets bit
-// 2 of err and leaves the bins unsorted.
-__global__ __launch_bounds__(256) void k_rebin_fallback(
-    const RepDev* __restrict__ reps, int nreps, const uint32_t* __restrict__ tile_prefix,
-    const uint32_t* __restrict__ app_prefix, Buf R, Buf W,
-    const uint32_t* __restrict__ offset_cur, uint32_t* __restrict__ cursor, Buf R2,
-    const uint32_t* __restrict__ offset_new, Buf T, Gate gate, uint32_t* __restrict__ err,
-    int count_down, uint32_t nitems) {
-  if (*gate.flag == 0u) return;  // the gather rebinned this step
-  if (blockIdx.x == 0 && threadIdx.x == 0) *gate.redone += 1u;  // steps redone
-  scatter_aligned_runs(reps, nreps, app_prefix, R, W, offset_cur, cursor, R2,
-                       count_down ? offset_new : nullptr);
-  if (!grid_wait(gate.bar, gridDim.x)) {
-    if (threadIdx.x == 0) atomicOr(err, 2u);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t u = 0; u < kRegs; ++u) {
+      const uint32_t e = t + u * kT;
+      if (e < m) {
+        const uint32_t q = s + gather_rank(s_key, 0u, m, e, s_key[e]);
+        R.x[q] = x[u];
+        R.y[q] = y[u];
+        R.hx[q] = hx[u];
+        R.hy[q] = hy[u];
+        R.id[q] = id[u];
+      }
+    }
+    __syncthreads();
     return;
   }
-  sort_bins_tiles(reps, nreps, tile_prefix, R2, offset_new, T, nitems, SortList{});
+  auto order = [&](uint32_t i, uint32_t j) {  // i < j
+    const uint64_t ki = bin_key(g, R.y[s + i], R.id[s + i]);
+    const uint64_t kj = bin_key(g, R.y[s + j], R.id[s + j]);
+    if (ki <= kj) return;
+    auto swap = [&](auto* p) {
+      const auto v = p[s + i];
+      p[s + i] = p[s + j];
+      p[s + j] = v;
+    };
+    swap(R.x);
+    swap(R.y);
+    swap(R.hx);
+    swap(R.hy);
+    swap(R.id);
+  };
+  for (uint32_t k = 2; k < 2u * m; k *= 2) {
+    for (uint32_t i = t; i < m; i += kT) {
+      const uint32_t j = i ^ (k - 1u);
+      if (j > i && j < m) order(i, j);
+    }
+    __syncthreads();
+    for (uint32_t w = k / 4; w > 0; w /= 2) {
+      for (uint32_t i = t; i < m; i += kT) {
+        const uint32_t j = i ^ w;
+        if (j > i && j < m) order(i, j);
+      }
+      __syncthreads();
+    }
+  }
 }
 
-hipError_t launch_rebin_fallback(const WorkList& wl, Buf R, Buf W, const uint32_t* offset_cur,
-                                 uint32_t* cursor, Buf R2, const uint32_t* offset_new, Buf T,
-                                 const Gate& gate, uint32_t* err, bool count_down,
-                                 hipStream_t s) {
+// The slow way of a tile: its own birds and its sources', a source whose
+// outbox overflowed read whole, go to their bins as they come, and the bins
+// are sorted in place.  Nothing here reads what another work-group of the
+// launch writes, so no tile waits for another.
+//
+// A call that takes the kernel's arguments from where they lie and finds the
+// rest again, so that the fast way keeps its registers (inlined, or called
+// with what the kernel holds, it made the fast way spill the birds it holds
+// there).
+struct GatherArgs {  // k_rebin_gather's arguments
+  const RepDev* reps;
+  int nreps;
+  const uint32_t* tile_prefix;
+  Buf R, W;
+  const uint32_t* offset_cur;
+  uint32_t* offset_new;
+  Outbox ob;
+  Buf R2;
+  Gate gate;
+  GatherScan sc;
+};
+
+// The work-group's LDS, all of it dynamic: it starts at LDS address 0 in the
+// kernel and in the function it calls.
+struct GatherSmem {
+  uint64_t key[kGatherCap];
+  uint64_t wave[kGatherThreads / kWave];
+  uint32_t bstart[kGatherMaxBins + 1];
+  uint32_t fill[kGatherMaxBins];
+  uint32_t sitem[kGatherSources], scnt[kGatherSources];
+  uint32_t fail;
+};
+
+extern __shared__ __align__(16) uint8_t gather_smem[];
+
+__device__ __noinline__ void gather_slow(uint32_t item, uint32_t nlo, const GatherArgs* args) {
+  constexpr uint32_t kT = kGatherThreads;
+  constexpr uint32_t kWaves = kT / kWave;
+  const uint32_t t = threadIdx.x;
+  const uint32_t lane = t & (kWave - 1), wid = t / kWave;
+  const Buf R = args->R, W = args->W, R2 = args->R2;
+  const Outbox ob = args->ob;
+  const uint32_t* const offset_cur = args->offset_cur;
+  const int r = find_rep(args->tile_prefix, args->nreps, item);
+  const uint32_t item0 = args->tile_prefix[r];
+  const RepDev& rp = args->reps[r];
+  const Geom& g = rp.g;
+  const uint32_t tile = item - item0;
+  const uint32_t nbt = 1u << (g.tx_log2 + g.tr_log2);
+  const uint32_t lo = offset_cur[rp.bin_base + tile * nbt];
+  const uint32_t nown = offset_cur[rp.bin_base + (tile + 1u) * nbt] - lo;
+  if (t == 0 && atomicExch(args->gate.flag, 1u) == 0u) atomicAdd(args->gate.redone, 1u);
+  GatherSmem& S = *(GatherSmem*)gather_smem;
+  uint32_t* const s_bstart = S.bstart;
+  uint32_t* const s_fill = S.fill;
+  uint64_t* const s_key = S.key;
+  auto take = [&](uint32_t src) {
+    const float x = W.x[src], y = W.y[src];
+    int32_t row;
+    const uint32_t b = gather_bin(g, tile, x, y, &row);
+    if (b >= nbt) return;
+    const uint32_t slot = atom_add(&s_fill[b], 1u);
+    if (slot >= s_bstart[b + 1] - s_bstart[b]) return;
+    const uint32_t pos = nlo + s_bstart[b] + slot;
+    R2.x[pos] = x;
+    R2.y[pos] = y;
+    R2.hx[pos] = W.hx[src];
+    R2.hy[pos] = W.hy[src];
+    R2.id[pos] = R.id[src];
+  };
+  for (uint32_t i = t; i < nown; i += kT) take(lo + i);
+  for (uint32_t q = 0; q < kGatherSources; ++q) {
+    const uint32_t n = S.scnt[q];
+    if (n > kOutboxCap) {
+      const uint32_t sb = rp.bin_base + (S.sitem[q] - item0) * nbt;
+      const uint32_t hi = offset_cur[sb + nbt];
+      for (uint32_t i = offset_cur[sb] + t; i < hi; i += kT) take(i);
+    } else {
+      for (uint32_t i = t; i < n; i += kT) take(ob.slot[(size_t)S.sitem[q] * kOutboxCap + i]);
+    }
+  }
+  __syncthreads();
+  for (uint32_t b = t; b < nbt; b += kT)
+    if (s_fill[b] != s_bstart[b + 1] - s_bstart[b]) atomicOr(args->gate.err, 2u);
+  for (uint32_t b = wid; b < nbt; b += kWaves) {
+    const uint32_t m = s_bstart[b + 1] - s_bstart[b];
+    if (m > 1u && m <= kSortWaveMax)
+      sort_wave_rows<kSortSlots>(g, R2, nlo + s_bstart[b], m, lane, (SortWave*)s_key + wid);
+  }
+  __syncthreads();
+  for (uint32_t b = 0; b < nbt; ++b) {
+    const uint32_t m = s_bstart[b + 1] - s_bstart[b];
+    if (m > kSortWaveMax)
+      sort_bin_in_place(g, R2, nlo + s_bstart[b], m, s_key);
+  }
+}
+
+// The gather rebinning: one work-group per tile, phases in kg_phases.hpp.
+// Each thread keeps its candidates in registers from load to store, so a
+// bird is read once and written once; a tile with more candidates (or new
+// birds) than kGatherCap goes the slow way.
+// With sc.count the work-group also does the scan's part for its tile: its
+// bins' new offsets follow from the earlier scan tiles' sums and the counts
+// of the earlier bins of its own scan tile (read from this step's counts,
+// which nothing clears in this step), and it writes them to offset_new.
+//
+// What bounds it: a work-group's chain of dependent loads (8 us alone on the
+// GPU, times the generations of work-groups a large field runs).  So the
+// tile's own birds, the counts and the outboxes' sizes are loaded before the
+// first wait, and one scan does for the bins and the birds before the tile:
+// 17,000 tiles of 260 birds 77 -> 69 us, 2,509 of 420 19.9 -> 19.5.
+// (128 threads to a tile, 15 tiles to a CU: 61 and 17.8 us, but a tile of
+// more than 1,024 birds then goes the slow way, which a field that gathers in
+// flocks soon has in every step.)
+__global__ __launch_bounds__(kGatherThreads, 8) void k_rebin_gather(
+    const RepDev* __restrict__ reps, int nreps, const uint32_t* __restrict__ tile_prefix, Buf R,
+    Buf W, const uint32_t* __restrict__ offset_cur, uint32_t* __restrict__ offset_new, Outbox ob,
+    Buf R2, Gate gate, GatherScan sc) {
+  constexpr uint32_t kT = kGatherThreads;
+  constexpr uint32_t kPer = kGatherMaxBins / kT;  // bins per thread
+  constexpr uint32_t kWaves = kT / kWave;
+  constexpr uint32_t kEarly = 3;
+  static_assert(sizeof(SortWave) * kWaves <= sizeof(uint64_t) * kGatherCap, "");
+  GatherSmem& S = *(GatherSmem*)gather_smem;
+  uint64_t* const s_wave = S.wave;
+  uint32_t* const s_bstart = S.bstart;
+  uint32_t* const s_fill = S.fill;
+  uint64_t* const s_key = S.key;
+  uint32_t *const s_sitem = S.sitem, *const s_scnt = S.scnt;
+  const uint32_t t = threadIdx.x;
+  const uint32_t lane = t & (kWave - 1), wid = t / kWave;
+  const uint32_t item = xcd_remap(blockIdx.x, gridDim.x);
+  const int r = find_rep(tile_prefix, nreps, item);
+  const RepDev& rp = reps[r];
+  const Geom& g = rp.g;
+  const uint32_t tile = item - tile_prefix[r];
+  const uint32_t nbt = 1u << (g.tx_log2 + g.tr_log2);
+  const uint32_t tb0 = rp.bin_base + tile * nbt;
+  const uint32_t lo = offset_cur[tb0], nown = offset_cur[tb0 + nbt] - lo;
+
+  // the loads that need nothing else
+  uint32_t scnt = 0;
+  if (t < kGatherSources) {
+    const int32_t sl = gather_source(g, tile, t);
+    const uint32_t it = sl >= 0 ? tile_prefix[r] + (uint32_t)sl : 0u;
+    s_sitem[t] = it;
+    scnt = sl >= 0 ? ob.n[it] : 0u;
+  }
+  uint32_t c[kPer], part = 0;  // this thread's bins; the birds before the tile
+  if (sc.count) {
+    // the earlier scan tiles' sums and the earlier bins of its own scan tile
+    const uint32_t q = tb0 / (uint32_t)kScanTile;
+    if (!sc.prefixed)
+      for (uint32_t i = t; i < q; i += kT) part += sc.tile_sum[i];
+    else if (t == 0)
+      part = sc.tile_sum[q];
+    for (uint32_t b = q * (uint32_t)kScanTile + t; b < tb0; b += kT) part += sc.count[b];
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i)
+      c[i] = t * kPer + i < nbt ? sc.count[tb0 + t * kPer + i] : 0u;
+  } else {
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+      const uint32_t b = tb0 + t * kPer + i;
+      c[i] = t * kPer + i < nbt ? offset_new[b + 1] - offset_new[b] : 0u;
+    }
+    if (t == 0) part = offset_new[tb0];
+  }
+  // per candidate: (bin << 16 | slot in the bin) or ~0, and the bird; the
+  // tile's own first kEarly * kT before the scan
+  uint32_t cbs[kGatherRegs], cid[kGatherRegs];
+  float cx[kGatherRegs], cy[kGatherRegs], chx[kGatherRegs], chy[kGatherRegs];
+  auto load = [&](uint32_t u, uint32_t src) {
+    cx[u] = W.x[src];
+    cy[u] = W.y[src];
+    chx[u] = W.hx[src];
+    chy[u] = W.hy[src];
+    cid[u] = R.id[src];
+  };
+#pragma unroll
+  for (uint32_t u = 0; u < kEarly; ++u)
+    if (t + u * kT < nown) load(u, lo + t + u * kT);
+  if (t == 0) S.fail = 0u;
+  if (t < kGatherSources) s_scnt[t] = scnt;
+  for (uint32_t b = t; b < nbt; b += kT) s_fill[b] = 0u;
+  // one scan for the bins' starts (low words) and the sum before the tile
+  uint32_t sum = 0, biggest = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < kPer; ++i) {
+    sum += c[i];
+    biggest = max(biggest, c[i]);
+  }
+  const uint64_t mine = ((uint64_t)part << 32) | sum;
+  uint64_t incl = mine;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint64_t v = __shfl_up(incl, off, kWave);
+    if ((int)lane >= off) incl += v;
+  }
+  if (lane == kWave - 1) s_wave[wid] = incl;
+  __syncthreads();
+  uint64_t before = 0, all = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < kWaves; ++w) {
+    const uint64_t v = s_wave[w];
+    if (w < wid) before += v;
+    all += v;
+  }
+  const uint32_t nlo = (uint32_t)(all >> 32), tot = (uint32_t)all;
+  uint32_t at = (uint32_t)before + (uint32_t)incl - sum;
+#pragma unroll
+  for (uint32_t i = 0; i < kPer; ++i) {
+    const uint32_t b = t * kPer + i;
+    if (b < nbt) {
+      s_bstart[b] = at;
+      if (sc.count) {
+        offset_new[tb0 + b] = nlo + at;
+        sc.count_next[tb0 + b] = 0u;
+      }
+      at += c[i];
+    }
+  }
+  if (sc.count && tile == (uint32_t)g.ntiles - 1u) {
+    // bins between this replica's last and the next replica's first (on
+    // the next scan tile) hold nobody: they start where this tile ends
+    const uint32_t pad_end = min(sc.nbins, (tb0 + nbt + (uint32_t)kScanTile - 1u) /
+                                               (uint32_t)kScanTile * (uint32_t)kScanTile);
+    for (uint32_t b = tb0 + nbt + t; b < pad_end; b += kT) offset_new[b] = nlo + tot;
+  }
+  uint32_t ncand = nown;
+  for (uint32_t q = 0; q < kGatherSources; ++q) ncand += s_scnt[q];
+  if (t == 0) {
+    s_bstart[nbt] = tot;
+    if (sc.count) {
+      if (item == sc.last_item) offset_new[sc.nbins] = nlo + tot;
+      if (tb0 % (uint32_t)kScanTile == 0) sc.tile_sum_next[tb0 / (uint32_t)kScanTile] = 0u;
+      if (item == 0) {
+        *sc.gstep += 1;
+        if (gate.clear) *gate.clear = 0u;
+      }
+    }
+    if (ncand > kGatherCap || tot > kGatherCap) S.fail = 1u;
+  }
+  if (biggest > kGatherBinMax || scnt > kOutboxCap) S.fail = 1u;
+  __syncthreads();
+  // fail is set before the barrier only: every thread takes the same path,
+  // here and (a count the candidates do not reach) not at all later, so the
+  // slow way's registers do not add to the fast way's
+  if (__builtin_amdgcn_readfirstlane((int)S.fail) != 0) {
+    gather_slow(item, nlo, (const GatherArgs*)__builtin_amdgcn_kernarg_segment_ptr());
+    return;
+  }
+#pragma unroll
+  for (uint32_t u = 0; u < kGatherRegs; ++u) {
+    const uint32_t k = t + u * kT;
+    cbs[u] = ~0u;
+    if (k < ncand) {
+      if (u >= kEarly || k >= nown) load(u, gather_src(ob, s_sitem, s_scnt, lo, nown, k));
+      int32_t row;
+      const uint32_t b = gather_bin(g, tile, cx[u], cy[u], &row);
+      if (b < nbt) {
+        const uint32_t slot = atom_add(&s_fill[b], 1u);
+        if (slot < s_bstart[b + 1] - s_bstart[b]) {
+          s_key[s_bstart[b] + slot] = ((uint64_t)(uint32_t)row << 32) | cid[u];
+          cbs[u] = (b << 16) | slot;
+        }
+      }
+    }
+  }
+  __syncthreads();
+  // every bird of a step that gather_reaches comes from a source: a bin that
+  // is not full is an error of the plan
+  for (uint32_t b = t; b < nbt; b += kT)
+    if (s_fill[b] != s_bstart[b + 1] - s_bstart[b]) atomicOr(gate.err, 2u);
+#pragma unroll
+  for (uint32_t u = 0; u < kGatherRegs; ++u) {
+    if (cbs[u] == ~0u) continue;
+    const uint32_t b = cbs[u] >> 16;
+    const uint32_t e = s_bstart[b] + (cbs[u] & 0xFFFFu);
+    const uint32_t pos =
+        nlo + s_bstart[b] + gather_rank(s_key, s_bstart[b], s_bstart[b + 1], e, s_key[e]);
+    R2.x[pos] = cx[u];
+    R2.y[pos] = cy[u];
+    R2.hx[pos] = chx[u];
+    R2.hy[pos] = chy[u];
+    R2.id[pos] = cid[u];
+  }
+}
+
+hipError_t launch_rebin_gather(const WorkList& wl, Buf R, Buf W, const uint32_t* offset_cur,
+                               uint32_t* offset_new, const Outbox& ob, Buf R2, const Gate& gate,
+                               const GatherScan& sc, hipStream_t s) {
   if (wl.ntiles == 0) return hipSuccess;
-  if (!gate.flag || !gate.redone || !gate.bar || !err) return hipErrorInvalidValue;
-  const uint32_t grid = wl.ntiles > kGatedGrid ? kGatedGrid : wl.ntiles;
-  hipLaunchKernelGGL(k_rebin_fallback, dim3(grid), dim3(256), 0, s, wl.reps, wl.nreps,
-                     wl.tile_prefix, wl.app_prefix, R, W, offset_cur, cursor, R2, offset_new, T,
-                     gate, err, count_down ? 1 : 0, wl.ntiles);
+  if (!gate.flag || !gate.redone || !gate.err) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_rebin_gather, dim3(wl.ntiles), dim3(kGatherThreads), sizeof(GatherSmem), s,
+                     wl.reps, wl.nreps, wl.tile_prefix, R, W, offset_cur, offset_new, ob, R2, gate,
+                     sc);
   return hipGetLastError();
 }
 

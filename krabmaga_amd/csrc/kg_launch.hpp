@@ -28,10 +28,9 @@ hipError_t launch_scatter_aligned(const WorkList& wl, Buf R, Buf W, const uint32
                                   uint32_t* cursor, Buf R2, uint32_t nagents, uint32_t* nlist,
                                   hipStream_t s);
 // The gather rebinning (one work-group per tile; tiles of at most
-// kGatherMaxBins bins) of the flock step that filled the outboxes: R2 in
-// bin order with every bin sorted, or gate.flag set for
-// launch_rebin_fallback to redo it.  sc.count: the scan is done here too (offset_new is
-// written); else offset_new holds the scan's offsets.
+// kGatherMaxBins bins) of the flock step that filled the outboxes: R2 in bin
+// order with every bin sorted.  sc.count: the scan is done here too
+// (offset_new is written); else offset_new holds the scan's offsets.
 hipError_t launch_rebin_gather(const WorkList& wl, Buf R, Buf W, const uint32_t* offset_cur,
                                uint32_t* offset_new, const Outbox& ob, Buf R2, const Gate& gate,
                                const GatherScan& sc, hipStream_t s);
@@ -45,17 +44,6 @@ hipError_t launch_scatter_append(const WorkList& wl, Buf A, uint32_t* cursor, Bu
 hipError_t launch_sort_bins(const WorkList& wl, Buf R, const uint32_t* offset, Buf T,
                             hipStream_t s, uint32_t* bins = nullptr, uint32_t nbins = 0,
                             uint32_t* nlist = nullptr);
-// The scatter and the bin sort of a gathered step in one launch, run only if
-// gate.flag is set (gate.redone counts such steps, gate.bar is the grid
-// wait's counter, zeroed by the gather): the scatter as
-// launch_scatter_aligned (count_down: cursor holds the step's bin counts,
-// each counted down to zero from offset_new), then the sort of R2's bins by
-// offset_new with T as scratch.  A grid wait that times out sets bit 2 of
-// err.
-hipError_t launch_rebin_fallback(const WorkList& wl, Buf R, Buf W, const uint32_t* offset_cur,
-                                 uint32_t* cursor, Buf R2, const uint32_t* offset_new, Buf T,
-                                 const Gate& gate, uint32_t* err, bool count_down,
-                                 hipStream_t s);
 // Whether a launch of ntiles takes 512-thread work-groups.
 bool near_wide(uint32_t ntiles);
 // Bytes of dynamic LDS for `cap` birds and `cols` columns.

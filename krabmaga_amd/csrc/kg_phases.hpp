@@ -84,16 +84,14 @@ KG_HD void scatter_append_one(const RepDev* reps, int nreps, const uint32_t* app
 // work-group per tile collects its candidates, ranks each inside its new
 // bin by (cell row, id) -- the order the bin sort gives -- and writes it to
 // its final slot, so the scatter and the bin sort need not run.  A tile that
-// cannot (more than kGatherCap candidates or new birds, an outbox past
-// kOutboxCap, a bin past kGatherBinMax birds, or collected counts that
-// differ from the histogram's, as when a bird jumps past the neighbouring
-// tiles) sets the gate word, and then the scatter and the bin sort redo the
-// whole rebinning of that step.
+// cannot be done so (more than the work-group's candidates or new birds, an
+// outbox past kOutboxCap, a bin past kGatherBinMax birds) is rebinned by its
+// own work-group from whole tiles and its bins sorted in place.
 
 constexpr uint32_t kGatherThreads = 256;
 constexpr uint32_t kGatherCap = 2048;     // candidates and new birds of a tile, at most
 constexpr uint32_t kGatherRegs = kGatherCap / kGatherThreads;  // candidates per thread
-constexpr uint32_t kGatherBinMax = 512;   // a fuller bin sends the step to the bin sort
+constexpr uint32_t kGatherBinMax = 512;   // a fuller bin is sorted by the work-group
 constexpr uint32_t kGatherMaxBins = 256;  // bins per tile the gather handles
 constexpr uint32_t kOutboxCap = 256;      // birds listed per tile and step
 constexpr uint32_t kGatherSources = 16;   // neighbouring tiles read, at most
@@ -103,32 +101,28 @@ struct Outbox {
   uint32_t* slot = nullptr;  // per tile: kOutboxCap read-buffer indices
 };
 
-// The gate of a gathered step: the flag a tile that cannot rebin sets (the
-// scatter and the bin sort run only if it is set), the count of steps they
-// redid, the flag the gather clears for the next step (or none: the scan
-// clears this step's), and the arrival counter of the fallback's grid wait
-// (the gather zeroes it; or none).
+// The gate of a gathered step: the flag of a step with a tile that took the
+// slow way, the count of such steps, the flag the gather clears for the
+// next step (or none: the scan clears this step's), and the error word (bit
+// 1: a bin's birds were not all found).
 struct Gate {
   uint32_t* flag = nullptr;
   uint32_t* redone = nullptr;
   uint32_t* clear = nullptr;
-  uint32_t* bar = nullptr;
+  uint32_t* err = nullptr;
 };
 
 // The scan done inside the gather, for a layout whose flock step left the
 // sums of the scan tiles (whole tiles each; every replica's bins start on a
 // scan tile): this step's bin counts and sums (or, with prefixed, the sums'
-// exclusive prefixes), the next step's (cleared here), the scatter cursors
-// to fill (or none: the fallback counts this step's counts down instead),
-// the new offsets, the schedule-step counter to advance, the bin count and
-// the last tile.  count == null: the offsets come from the scan
-// kernels.
+// exclusive prefixes), the next step's (cleared here), the schedule-step
+// counter to advance, the bin count and the last tile.  count == null: the
+// offsets come from the scan kernels.
 struct GatherScan {
   uint32_t* count = nullptr;
   const uint32_t* tile_sum = nullptr;
   uint32_t* count_next = nullptr;
   uint32_t* tile_sum_next = nullptr;
-  uint32_t* cursor = nullptr;
   uint64_t* gstep = nullptr;
   uint32_t nbins = 0;
   uint32_t last_item = 0;
@@ -156,6 +150,15 @@ KG_HD int32_t gather_source(const Geom& g, uint32_t tile, uint32_t q) {
   const int32_t sy = gather_axis_at(tcy, g.nty, (int)(q >> 2));
   if (sx < 0 || sy < 0 || (sx == tcx && sy == tcy)) return -1;
   return sy * g.ntx + sx;
+}
+
+// Whether the sources hold every bird that can enter a tile in a step: none
+// moves further than one tile, and the step wraps both axes by the width
+// (bird.rs:147), which is a neighbouring tile only on a square field.  Other
+// fields rebin by scatter and sort.
+KG_HD bool gather_reaches(const Geom& g, float jump) {
+  // with room for the step's rounding; false for NaN
+  return g.w == g.h && fabsf(jump) <= 0.99f * (float)imin(g.tx, g.ty) * g.d;
 }
 
 // Candidate k of a tile: its old birds [lo, lo + nown), then the outbox

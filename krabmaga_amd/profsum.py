@@ -1,10 +1,10 @@
 """Summaries of rocprofv3 output for the flockers schedule step.
 
 Two device paths run a step.  The three-kernel path (the default for large
-fields) launches k_flock (plus k_flock_global for crowded tiles), the scan
-(k_scan_reduce and k_scan_down, or k_scan_partials, or none when the gather
-does it), then k_rebin_gather and k_rebin_fallback, or k_scatter_aligned and
-k_sort_bins, once each per step, one after another on one stream: with
+fields) launches k_flock or k_flock_near (plus k_flock_global or k_flock_runs
+for crowded tiles), the scan (k_scan_reduce and k_scan_down, or
+k_scan_partials, or none when the gather does it), then k_rebin_gather, or
+k_scatter_aligned, k_sort_bins and k_sort_list, once each per step, one after another on one stream: with
 --step-kernel kg::k_flock a
 step runs from one k_flock launch to the next, and --fetch / --write sum
 those kernels' bytes per step.  The tile-resident path is described next.
@@ -36,11 +36,11 @@ import csv
 import statistics
 
 KERNEL = "kg::k_rt_step"
-FLOCK = "kg::k_flock"
+FLOCK = ("kg::k_flock", "kg::k_flock_near")
 # the kernels of one three-kernel schedule step
-STEP_KERNELS = ("kg::k_flock", "kg::k_flock_global", "kg::k_scan_reduce", "kg::k_scan_down",
-                "kg::k_rebin_gather", "kg::k_rebin_fallback", "kg::k_scatter_aligned",
-                "kg::k_sort_bins")
+STEP_KERNELS = ("kg::k_flock", "kg::k_flock_near", "kg::k_flock_global", "kg::k_flock_runs",
+                "kg::k_scan_reduce", "kg::k_scan_down", "kg::k_rebin_gather",
+                "kg::k_scatter_aligned", "kg::k_sort_bins", "kg::k_sort_list")
 # launched within a three-kernel step on some layouts: the tile-sum prefix
 # pass of large scans, the device step counter
 STEP_AUX_KERNELS = ("kg::k_scan_partials", "kg::k_add_u64")
@@ -186,7 +186,7 @@ def summarize(a):
                      f"-> {alg / per_step / 1e3:.1f} GB/s = {alg / per_step / 1e3 / 8000 * 100:.2f} % "
                      f"of 8 TB/s{own}")
         if three:
-            fl = [(r["end"] - r["start"]) / 1000.0 for g in sel for r in g if r["name"] == FLOCK]
+            fl = [(r["end"] - r["start"]) / 1000.0 for g in sel for r in g if r["name"] in FLOCK]
             if fl:
                 fb = FLOCK_BYTES_PER_AGENT * a.agents
                 lines.append(f"- k_flock: mean {statistics.mean(fl):.1f} us per launch; its own "
