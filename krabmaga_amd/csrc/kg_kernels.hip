@@ -484,9 +484,14 @@ __global__ __launch_bounds__(kFlockThreads) void k_flock(
 
 // k_flock on a near field (kg_near.hpp): the same tiles, chunks, global path
 // and sinks, the birds staged as sorted records.  A tile with a bird outside
-// the near form takes the global path.  kT threads: the tile's own birds fit
-// one round of 512 where tiles are few.
+// the near form takes the global path.
+// What bounds it: with few tiles a round's chain of LDS reads and f64
+// quotients (6.6 us a round, whatever the lanes in it), with many tiles VALU
+// issue.  So up to two tiles per CU take kT = 1,024 threads and one round for
+// all but a tile twice as full as the average (450 birds): 16,384 boids 20.5
+// -> 16.4 us, 65,537 21.9 -> 17.8, 262,144 25.4 -> 23.9; up to four 512.
 // Eight waves per SIMD (64 VGPRs): only the inline global walk spills.
+constexpr uint32_t kNearOneRoundTiles = 512;
 constexpr uint32_t kNearWideTiles = 1024;
 
 template <int kT, bool kInlineGlobal>
@@ -772,7 +777,9 @@ __global__ __launch_bounds__(kFlockThreads) void k_flock_global(
   }
 }
 
-bool near_wide(uint32_t ntiles) { return ntiles <= kNearWideTiles; }
+int near_threads(uint32_t ntiles) {
+  return ntiles <= kNearOneRoundTiles ? 1024 : ntiles <= kNearWideTiles ? 512 : 256;
+}
 size_t near_lds_bytes(int cap, int cols) { return near_smem_bytes(cap, cols); }
 
 hipError_t launch_flock(const WorkList& wl, Buf R, const uint32_t* offset, Buf W,
@@ -782,10 +789,12 @@ hipError_t launch_flock(const WorkList& wl, Buf R, const uint32_t* offset, Buf W
                         const NearPlan& near) {
   if (wl.ntiles == 0) return hipSuccess;
   if (near.on) {
-    const bool wide = near_wide(wl.ntiles);
-    auto kern = wide ? (inline_global ? k_flock_near<512, true> : k_flock_near<512, false>)
-                     : (inline_global ? k_flock_near<256, true> : k_flock_near<256, false>);
-    hipLaunchKernelGGL(kern, dim3(wl.ntiles), dim3(wide ? 512 : 256),
+    const int threads = near_threads(wl.ntiles);
+    auto kern = inline_global ? k_flock_near<256, true> : k_flock_near<256, false>;
+    if (threads == 512) kern = inline_global ? k_flock_near<512, true> : k_flock_near<512, false>;
+    if (threads == 1024)
+      kern = inline_global ? k_flock_near<1024, true> : k_flock_near<1024, false>;
+    hipLaunchKernelGGL(kern, dim3(wl.ntiles), dim3(threads),
                        near_smem_bytes(near.cap, near.cols), s, wl.reps, wl.nreps,
                        wl.tile_prefix, R, offset, W, count_next, gstep, err, near.cap, near.cols,
                        gflag, ob, tile_sum);

@@ -44,8 +44,8 @@ hipError_t launch_scatter_append(const WorkList& wl, Buf A, uint32_t* cursor, Bu
 hipError_t launch_sort_bins(const WorkList& wl, Buf R, const uint32_t* offset, Buf T,
                             hipStream_t s, uint32_t* bins = nullptr, uint32_t nbins = 0,
                             uint32_t* nlist = nullptr);
-// Whether a launch of ntiles takes 512-thread work-groups.
-bool near_wide(uint32_t ntiles);
+// Threads per work-group of a near launch of ntiles.
+int near_threads(uint32_t ntiles);
 // Bytes of dynamic LDS for `cap` birds and `cols` columns.
 size_t near_lds_bytes(int cap, int cols);
 
