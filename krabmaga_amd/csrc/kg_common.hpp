@@ -28,6 +28,13 @@ int clamp_lds_cap(int cap);
 // stage `cap` birds (pick_lds_cap), `ntiles` work-groups in the launch.
 NearPlan near_plan(int cap, int cols, uint32_t ntiles);
 
+// Three-kernel steps per captured graph in a run of n: the GPU idles about
+// 8 us between graph launches, 4 us per step with two steps to a graph
+// (of 28 at 16,384 boids), while a graph of sixteen takes its capture and
+// instantiation before the first launch.  Even, so that the buffers are back
+// in place.
+inline int graph_steps(uint32_t n) { return n >= 64u ? 16 : 2; }
+
 // The gather rebinning after flock steps; KG_REBIN_GATHER=0 turns it off
 // (scatter and bin sort every step), for comparison.
 bool rebin_gather_enabled();

@@ -132,7 +132,7 @@ struct kg_ensemble {
   NearPlan near{};  // off unless every run is near
   HostStage stage;
   int parity = 0;  // bin-grouped steps taken since the build, mod 2
-  // two-step graphs by parity + 2 * gather
+  // graphs by parity + 2 * gather + 4 * steps
   std::vector<std::pair<int, hipGraphExec_t>> bgraphs;
   // gather rebinning (every run's tiles of at most kGatherMaxBins bins): the
   // lists of leavers, the gate words (a flag per step parity, the steps with
@@ -651,8 +651,7 @@ hipError_t binned_step(kg_ensemble* e, const WorkList& w) {
   return hipSuccess;
 }
 
-// `n` bin-grouped steps (graph replays of two steps when allowed: the
-// buffers are back in place after two).
+// `n` bin-grouped steps (graph replays of graph_steps when allowed).
 int binned_steps(kg_ensemble* e, uint32_t n, bool use_graph) {
   if (int rc = ready_binned(e)) return rc;
   const WorkList w = e->wl();
@@ -668,14 +667,15 @@ int binned_steps(kg_ensemble* e, uint32_t n, bool use_graph) {
   }
   if (use_graph && left >= 2) {
     hipGraphExec_t exec = nullptr;
-    const int key = e->parity + (e->gather ? 2 : 0);
+    const int steps = graph_steps(left);
+    const int key = e->parity + (e->gather ? 2 : 0) + 4 * steps;
     for (auto& g : e->bgraphs)
       if (g.first == key) exec = g.second;
     if (!exec) {
       hipGraph_t graph = nullptr;
       KG_HIP(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-      hipError_t err = binned_step(e, w);
-      if (err == hipSuccess) err = binned_step(e, w);
+      hipError_t err = hipSuccess;
+      for (int k = 0; k < steps && err == hipSuccess; ++k) err = binned_step(e, w);
       const hipError_t e2 = hipStreamEndCapture(e->stream, &graph);
       if (err != hipSuccess || e2 != hipSuccess)
         return set_error(KG_E_HIP, "graph capture: %s",
@@ -686,9 +686,9 @@ int binned_steps(kg_ensemble* e, uint32_t n, bool use_graph) {
         return set_error(KG_E_HIP, "graph instantiate: %s", hipGetErrorString(err));
       e->bgraphs.push_back({key, exec});
     }
-    while (left >= 2) {
+    while (left >= (uint32_t)steps) {
       KG_HIP(hipGraphLaunch(exec, e->stream));
-      left -= 2;
+      left -= (uint32_t)steps;
     }
   }
   for (; left > 0; --left) KG_HIP(binned_step(e, w));

@@ -29,10 +29,12 @@ struct GraphKey {
   int parity;
   int gather;         // the steps rebin by gather
   int inline_global;  // global-path tiles stepped inside k_flock
+  int steps;          // even: the read buffer returns to the same array pair
   bool operator<(const GraphKey& o) const {
     if (parity != o.parity) return parity < o.parity;
     if (gather != o.gather) return gather < o.gather;
     if (inline_global != o.inline_global) return inline_global < o.inline_global;
+    if (steps != o.steps) return steps < o.steps;
     return std::memcmp(params, o.params, sizeof(params)) < 0;
   }
 };
@@ -1109,15 +1111,15 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
     key.parity = f->parity;
     key.gather = f->gathers() ? 1 : 0;
     key.inline_global = f->global_inline ? 1 : 0;
+    key.steps = graph_steps(left);
     auto it = f->graphs.find(key);
     hipGraphExec_t exec = nullptr;
     if (it == f->graphs.end()) {
-      // capture two steps: the read buffer returns to the same array pair
       hipGraph_t graph = nullptr;
       KG_HIP(hipStreamBeginCapture(f->stream, hipStreamCaptureModeThreadLocal));
       f->capturing = true;
-      int rc = run_direct_step(f);
-      if (rc == KG_OK) rc = run_direct_step(f);
+      int rc = KG_OK;
+      for (int k = 0; k < key.steps && rc == KG_OK; ++k) rc = run_direct_step(f);
       f->capturing = false;
       hipError_t e = hipStreamEndCapture(f->stream, &graph);
       if (rc) return rc;
@@ -1129,9 +1131,9 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
     } else {
       exec = it->second;
     }
-    while (left >= 2) {
+    while (left >= (uint32_t)key.steps) {
       KG_HIP(hipGraphLaunch(exec, f->stream));
-      left -= 2;
+      left -= (uint32_t)key.steps;
     }
   }
   while (left > 0) {
