@@ -543,6 +543,10 @@ __global__ __launch_bounds__(kT, 8) void k_flock_near(
     }
   }
   const FlockSinks lv{ob, item - ft.tile, &s_outn, tile_sum ? s_hist : nullptr, tile_sum};
+  const NearStrips st = near_strips(rp);
+  if (use_lds)  // read after the first chunk's barrier
+    for (uint32_t i = t; i < (uint32_t)(ft.ncols * st.per); i += kT)
+      near_strip_fill(rp, ft, st, i, offset, S);
   for (int32_t oa = own_lo; use_lds && oa < own_hi;) {
     const int32_t ob2 =
         chunked ? flock_chunk_end(rp, ft, S.col_base, oa, own_hi, cap) : own_hi;
@@ -554,7 +558,7 @@ __global__ __launch_bounds__(kT, 8) void k_flock_near(
     use_lds = s_bad == 0u;
     if (use_lds)
       for (uint32_t o = t; o < k.nown; o += kT)
-        near_agent(rp, ft, k, o, S, W, count_next, err, lv);
+        near_agent(rp, ft, k, st, o, S, W, count_next, err, lv);
     oa = ob2;
     if (oa < own_hi) __syncthreads();  // the next chunk reuses the LDS
   }

@@ -248,10 +248,7 @@ KG_HD uint32_t near_lower(const uint32_t* z, uint32_t lo, uint32_t hi, uint32_t 
 // neighbouring ones (those past `cols` are empty).
 //
 // TileFind: the birds are the staged columns of a tile, column c from
-// col_base[c] - base; the starts of three columns bisected side by side
-// (three LDS reads in flight), the ends found by stepping from them (bisecting
-// the ends too cost more: a 1M-boid step 86.7 us against 77.6, on a field ten
-// times denser 103.8 against 96.6).
+// col_base[c] - base; both ends of a column's run bisected.
 struct TileFind {
   const uint32_t* z;
   const uint32_t* col_base;
@@ -263,37 +260,56 @@ struct TileFind {
     *lo = near_lower(z, col_base[c] - base, end, key);
     *hi = near_lower(z, *lo, end, key + rows + 1u);
   }
+};
+
+// StripFind: the same birds with the strips' starts (near_strips): a run's
+// ends are at most a strip from a table entry, and where strips are single
+// rows they are entries.  Bisecting and stepping were a fifth of the
+// instructions of a dense tile (a round of 512 birds 6.6 us, 2.9 of them
+// here).
+struct StripFind : TileFind {
+  const uint16_t* strip;
+  int32_t n, per, sh, y0;
+
   KG_HD void three(int32_t c, int32_t cols, int32_t row, uint32_t rows, uint32_t* lo,
                    uint32_t* hi) const {
-    uint32_t n[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      lo[q] = q <= cols ? col_base[c + q] - base : 0u;
-      n[q] = q <= cols ? col_base[c + q + 1] - base - lo[q] : 0u;
-    }
-    const uint32_t key = ((uint32_t)c << kNearRowBits) + (uint32_t)row;
-    // an empty range reads one entry at most past the last bird
-    while (n[0] | n[1] | n[2]) {
+    const int32_t r0 = row - y0, r1 = r0 + (int32_t)rows;
+    const int32_t j0 = imin(imax(r0 >> sh, -1), n) + 1, j1 = imin(imax(r1 >> sh, -1), n) + 1;
+    const uint16_t* const s0 = strip + c * per;
+    if (sh == 0) {  // single rows (and bands of one: three() is for disc_dist = 1)
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        const uint32_t hn = n[q] >> 1;
-        const bool un = n[q] != 0u && z[lo[q] + hn] < key + ((uint32_t)q << kNearRowBits);
-        lo[q] = un ? lo[q] + hn + 1u : lo[q];
-        n[q] = un ? n[q] - hn - 1u : hn;
+        lo[q] = q <= cols ? s0[q * per + j0] - base : 0u;
+        hi[q] = q <= cols ? s0[q * per + j1 + 1] - base : 0u;
       }
+      return;
     }
-    // the ends from there: a run is short
-    uint32_t last[3];
+    const uint32_t key = ((uint32_t)c << kNearRowBits) + (uint32_t)row;
+    uint32_t first[3], last[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      hi[q] = lo[q];
-      last[q] = q <= cols ? key + ((uint32_t)q << kNearRowBits) + rows : 0u;
+      lo[q] = q <= cols ? s0[q * per + j0] - base : 0u;
+      hi[q] = q <= cols ? s0[q * per + j1] - base : 0u;
+      first[q] = q <= cols ? key + ((uint32_t)q << kNearRowBits) : 0u;
+      last[q] = q <= cols ? first[q] + rows : 0u;
     }
+    // both sides of each condition: no branch; the sentinel ends every run
     for (bool more = true; more;) {
       more = false;
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        const bool in = (z[hi[q]] <= last[q]) & (q <= cols);  // both sides: no branch
+        const bool before = z[lo[q]] < first[q];
+        lo[q] += before ? 1u : 0u;
+        more |= before;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) hi[q] = hi[q] < lo[q] ? lo[q] : hi[q];
+    for (bool more = true; more;) {
+      more = false;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const bool in = (z[hi[q]] <= last[q]) & (q <= cols);
         hi[q] += in ? 1u : 0u;
         more |= in;
       }
@@ -365,30 +381,32 @@ KG_HD void near_walk(const RepDev& rp, int32_t col0, const NearWindow& w, float 
                      uint32_t qid, const Find& find, const NearBirds& B, NearAcc* acc) {
   if (w.cols < 0 || w.rows < 0) return;
   const uint32_t rows = (uint32_t)w.rows;
-  if (kFlat && rp.disc_dist == 1) {
-    // a wave's trips are those of its busiest lane, not of each column's
-    uint32_t lo[3], hi[3];
-    find.three(w.c, w.cols, w.row, rows, lo, hi);
-    const uint32_t n0 = hi[0] - lo[0], n1 = n0 + hi[1] - lo[1], n = n1 + hi[2] - lo[2];
-    const uint32_t o1 = lo[1] - n0, o2 = lo[2] - n1;
-    const uint32_t o0 = lo[0];
-    if (n == 0u) return;
-    uint32_t e = near_at(0u, n0, n1, o0, o1, o2), k = 0;
-    NearRec c = B.rec[e];
-    uint32_t id = B.id[e];
-    for (; k + 1u < n; k += 2) {
-      const uint32_t e1 = near_at(k + 1u, n0, n1, o0, o1, o2);
-      const NearRec c1 = B.rec[e1];
-      const uint32_t id1 = B.id[e1];
-      near_candidate(rp, col0, qx, qy, qid, B, e, c, id, acc);
-      // past the last candidate this is at most the sentinel
-      e = near_at(k + 2u, n0, n1, o0, o1, o2);
-      c = B.rec[e];
-      id = B.id[e];
-      near_candidate(rp, col0, qx, qy, qid, B, e1, c1, id1, acc);
+  if constexpr (kFlat) {
+    if (rp.disc_dist == 1) {
+      // a wave's trips are those of its busiest lane, not of each column's
+      uint32_t lo[3], hi[3];
+      find.three(w.c, w.cols, w.row, rows, lo, hi);
+      const uint32_t n0 = hi[0] - lo[0], n1 = n0 + hi[1] - lo[1], n = n1 + hi[2] - lo[2];
+      const uint32_t o1 = lo[1] - n0, o2 = lo[2] - n1;
+      const uint32_t o0 = lo[0];
+      if (n == 0u) return;
+      uint32_t e = near_at(0u, n0, n1, o0, o1, o2), k = 0;
+      NearRec c = B.rec[e];
+      uint32_t id = B.id[e];
+      for (; k + 1u < n; k += 2) {
+        const uint32_t e1 = near_at(k + 1u, n0, n1, o0, o1, o2);
+        const NearRec c1 = B.rec[e1];
+        const uint32_t id1 = B.id[e1];
+        near_candidate(rp, col0, qx, qy, qid, B, e, c, id, acc);
+        // past the last candidate this is at most the sentinel
+        e = near_at(k + 2u, n0, n1, o0, o1, o2);
+        c = B.rec[e];
+        id = B.id[e];
+        near_candidate(rp, col0, qx, qy, qid, B, e1, c1, id1, acc);
+      }
+      if (k < n) near_candidate(rp, col0, qx, qy, qid, B, e, c, id, acc);
+      return;
     }
-    if (k < n) near_candidate(rp, col0, qx, qy, qid, B, e, c, id, acc);
-    return;
   }
   for (int32_t q = 0; q <= w.cols; ++q) {
     uint32_t lo, hi;
@@ -453,6 +471,25 @@ KG_HD void near_step(const RepDev& rp, int32_t col0, uint64_t step, uint32_t o, 
 // columns, whole columns beside them) follow.  Both go to their place in the
 // z order.
 
+// Where the strips of a tile's staged columns start: a column's entries are
+// the band below the tile, its own rows in strips of 1 << sh rows (whole bins,
+// whose starts the read buffer's offsets give), the band above, and its end.
+// As many strips to a column as kNearStrips entries allow (one strip always
+// fits: kMaxStageCols columns of 4).
+constexpr int kNearStrips = 4 * kMaxStageCols;
+
+struct NearStrips {
+  int32_t n, per, sh;  // strips of a column, its entries (n + 3), rows of a strip (log2)
+};
+
+KG_HD NearStrips near_strips(const RepDev& rp) {
+  const Geom& g = rp.g;
+  const int32_t cols = imin(kMaxStageCols, g.tx + 2 * rp.disc_dist);
+  int32_t up = 0;
+  while ((g.tr >> up) > 1 && cols * ((g.tr >> up) + 3) > kNearStrips) ++up;
+  return NearStrips{g.tr >> up, (g.tr >> up) + 3, g.hb_log2 + up};
+}
+
 // LDS of a staged tile: `cap` birds and the per-column tables of `cols`
 // columns.
 struct NearSmem {
@@ -461,11 +498,12 @@ struct NearSmem {
   uint32_t* seg_len;    // 3 per column
   uint32_t* col_base;   // cols + 1
   uint16_t* own;        // cap: slots of the own birds, in read-buffer order
+  uint16_t* strip;      // kNearStrips (near_strips)
 };
 
 KG_HD size_t near_smem_bytes(int cap, int cols) {
   return near_birds_bytes((uint32_t)cap) + (size_t)(7 * cols + 1) * sizeof(uint32_t) +
-         (size_t)((cap + 1) & ~1) * sizeof(uint16_t);
+         (size_t)(((cap + 1) & ~1) + kNearStrips) * sizeof(uint16_t);
 }
 
 KG_HD NearSmem near_carve(uint8_t* p, int cap, int cols) {
@@ -475,6 +513,7 @@ KG_HD NearSmem near_carve(uint8_t* p, int cap, int cols) {
   s.seg_len = s.seg_start + 3 * cols;
   s.col_base = s.seg_len + 3 * cols;
   s.own = (uint16_t*)(s.col_base + cols + 1);
+  s.strip = s.own + ((cap + 1) & ~1);
   return s;
 }
 
@@ -563,12 +602,37 @@ KG_HD bool near_item_ok(const RepDev& rp, const NearChunk& k, uint32_t i, Buf R,
   return !near_bad(rp.g, R.x[gi], R.y[gi], R.hx[gi], R.hy[gi]);
 }
 
+// Entry i (< ft.ncols * near_strips().per) of the strips' table, counted from
+// the tile's first staged bird (col_base).
+KG_HD void near_strip_fill(const RepDev& rp, const FlockTile& ft, const NearStrips& st, uint32_t i,
+                           const uint32_t* offset, const NearSmem& S) {
+  const Geom& g = rp.g;
+  const int32_t c = (int32_t)(i / (uint32_t)st.per), j = (int32_t)(i % (uint32_t)st.per) - 1;
+  uint32_t v = S.col_base[c];
+  if (j > st.n) {
+    v = S.col_base[c + 1];
+  } else if (j >= 0) {
+    v += S.seg_len[3 * c];
+    if (j == st.n) {
+      v += S.seg_len[3 * c + 1];
+    } else if (S.seg_len[3 * c + 1] != 0u) {
+      const int32_t col = ft.sc_lo + c;
+      const uint32_t tt = (uint32_t)(ft.tcy * g.ntx + (col >> g.tx_log2));
+      const uint32_t b = rp.bin_base + col_bin0(g, tt, col & (g.tx - 1)) +
+                         ((uint32_t)j << (st.sh - g.hb_log2));
+      v += offset[b] - S.seg_start[3 * c + 1];
+    }
+  }
+  S.strip[i] = (uint16_t)v;
+}
+
 // Bird::step of own bird o of a staged chunk.
-KG_HD void near_agent(const RepDev& rp, const FlockTile& ft, const NearChunk& k, uint32_t o,
-                      const NearSmem& S, Buf W, uint32_t* count_next, uint32_t* err,
-                      const FlockSinks& lv) {
+KG_HD void near_agent(const RepDev& rp, const FlockTile& ft, const NearChunk& k,
+                      const NearStrips& st, uint32_t o, const NearSmem& S, Buf W,
+                      uint32_t* count_next, uint32_t* err, const FlockSinks& lv) {
   NearRec r;
-  near_step<true>(rp, ft.sc_lo, ft.step, S.own[o], TileFind{S.b.z, S.col_base, k.base}, S.b, &r);
+  const StripFind find{{S.b.z, S.col_base, k.base}, S.strip, st.n, st.per, st.sh, ft.y0};
+  near_step<true>(rp, ft.sc_lo, ft.step, S.own[o], find, S.b, &r);
   flock_emit(rp.g, rp.bin_base, W, k.own_lo + o, r.x, r.y, r.hx, r.hy, count_next, err, ft.tile,
              lv);
 }

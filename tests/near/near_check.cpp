@@ -132,6 +132,10 @@ static int run(const Case& c, uint64_t seed) {
       L += flock_segments(rp, ft, t, offset.data(), S.seg_start, S.seg_len);
     }
     S.col_base[ft.ncols] = L;
+    const NearStrips st = near_strips(rp);
+    if (ft.ncols * st.per > kNearStrips) return 1;
+    for (uint32_t i = 0; i < (uint32_t)(ft.ncols * st.per); ++i)
+      near_strip_fill(rp, ft, st, i, offset.data(), S);
     const int32_t lo = ft.c0 - ft.sc_lo, hi = ft.c1 - ft.sc_lo;
     const uint32_t cap = (uint32_t)c.cap;
     bool fits = true;
@@ -160,7 +164,7 @@ static int run(const Case& c, uint64_t seed) {
           return 1;
         }
       for (uint32_t o = 0; o < k.nown; ++o) {
-        near_agent(rp, ft, k, o, S, W.view(), cnt.data(), &err, lv);
+        near_agent(rp, ft, k, st, o, S, W.view(), cnt.data(), &err, lv);
         const uint32_t gi = k.own_lo + o;
         flock_agent_global(rp, ft.step, gi, R.view(), offset.data(), V.view(), want.data(),
                            &err2, lv);
@@ -242,6 +246,8 @@ int main() {
       {"sparse", 3000, 1100, 1100, d, 10, 0.7f, 0, 0, 0, 900, 0, 0, 1, true},
       {"dense", 6000, 300, 300, d, 10, 0.7f, 0, 0, 0, 1400, 0, 0, 1, true},
       {"dense, chunked", 6000, 300, 300, d, 10, 0.7f, 8, 32, 4, 300, 0, 0, 1, true},
+      {"rows for strips", 6000, 300, 300, d, 10, 0.7f, 16, 16, 1, 1400, 0, 0, 1, true},
+      {"two bins to a strip", 6000, 300, 300, d, 10, 0.7f, 16, 64, 1, 3000, 0, 0, 1, true},
       {"short tiles", 2000, 400, 380, d, 10, 0.7f, 4, 4, 1, 600, 0, 0, 1, true},
       {"one-cell tiles", 800, 250, 250, d, 10, 0.7f, 1, 1, 1, 600, 0, 0, 1, true},
       {"corners", 4000, 200, 200, 5, 10, 0.7f, 0, 0, 0, 3000, 1, 0, 1, true},
