@@ -61,7 +61,7 @@ int clamp_lds_cap(int cap) {
   return cap;
 }
 
-NearPlan near_plan(int cap, int cols, uint32_t ntiles) {
+NearPlan near_plan(int cap, int cols, uint32_t ntiles, bool full) {
   int dev = 0, max_lds = 65536, cu_lds = 160 * 1024;
   if (hipGetDevice(&dev) == hipSuccess) {
     int v = 0;
@@ -77,7 +77,8 @@ NearPlan near_plan(int cap, int cols, uint32_t ntiles) {
   // about 1.1 KB.  The capacity grows to the largest that keeps the
   // work-groups per CU, which its waves also bound.
   constexpr size_t kStatic = 1280, kStep = 1280;
-  const size_t waves = 2048u / (size_t)near_threads(ntiles);  // work-groups of a CU's 32 waves
+  const int threads = near_threads(ntiles, full);
+  const size_t waves = 2048u / (size_t)threads;  // work-groups of a CU's 32 waves
   const size_t per_wg = (near_lds_bytes(cap, cols) + kStatic + kStep - 1) / kStep * kStep;
   const size_t fit = std::max<size_t>(1, std::min(waves, (size_t)cu_lds / per_wg));
   const size_t share = std::min((size_t)cu_lds / fit / kStep * kStep, (size_t)max_lds) - kStatic;
@@ -87,6 +88,7 @@ NearPlan near_plan(int cap, int cols, uint32_t ntiles) {
   p.on = true;
   p.cap = std::min(cap, 4096);
   p.cols = cols;
+  p.threads = threads;
   return p;
 }
 

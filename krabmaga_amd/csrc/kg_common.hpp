@@ -25,8 +25,9 @@ void clear_error();
 int clamp_lds_cap(int cap);
 
 // The near flock kernel's staging for tiles of `cols` columns expected to
-// stage `cap` birds (pick_lds_cap), `ntiles` work-groups in the launch.
-NearPlan near_plan(int cap, int cols, uint32_t ntiles);
+// stage `cap` birds (pick_lds_cap), `ntiles` work-groups in the launch; full:
+// as near_threads.
+NearPlan near_plan(int cap, int cols, uint32_t ntiles, bool full);
 
 // Three-kernel steps per captured graph in a run of n: the GPU idles about
 // 8 us between graph launches, 4 us per step with two steps to a graph

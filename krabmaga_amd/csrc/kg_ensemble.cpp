@@ -566,7 +566,7 @@ int ready_binned(kg_ensemble* e) {
     cols = std::max(cols, std::min(kMaxStageCols, rp.g.tx + 2 * rp.disc_dist));
     near = near && rp.near;
   }
-  e->near = near ? near_plan(cap, cols, e->ntiles) : NearPlan{};
+  e->near = near ? near_plan(cap, cols, e->ntiles, false) : NearPlan{};
   e->gather = rebin_gather_enabled();
   for (const RepDev& rp : e->h_reps)
     if ((uint32_t)(rp.g.tx * rp.g.tr) > kGatherMaxBins || !gather_reaches(rp.g, rp.p.jump))

@@ -313,16 +313,25 @@ int flock_impl(kg_field* f, const uint64_t* gstep) {
   return KG_OK;
 }
 
+// The near kernel's staging for the current parameters.  Tiles of more than
+// 320 birds on average mostly hold more than 256, unless some are crowded
+// (global_inline is not set) and the rest near empty.
+void plan_near(kg_field* f) {
+  const int cols = std::min(kMaxStageCols, f->g.tx + 2 * std::max(0, f->h_rep.disc_dist));
+  const bool full = f->global_inline && f->cap / f->g.ntiles > 320u;
+  if (f->h_rep.near &&
+      (f->near.cols != cols || f->near.threads != near_threads(f->g.ntiles, full)))
+    f->near = near_plan(pick_lds_cap(f->g, f->cap), cols, f->g.ntiles, full);
+  f->near.on = f->h_rep.near != 0;
+}
+
 int set_params(kg_field* f, const kg_flock_params* p, uint64_t step_base) {
   std::string why;
   if (!p) return set_error(KG_E_INVALID, "params is NULL");
   if (!params_valid(*p, &why)) return set_error(KG_E_INVALID, "%s", why.c_str());
   set_rep_params(&f->h_rep, *p);
   f->h_rep.step_base = step_base;
-  const int cols = std::min(kMaxStageCols, f->g.tx + 2 * std::max(0, f->h_rep.disc_dist));
-  if (f->h_rep.near && f->near.cols != cols)
-    f->near = near_plan(pick_lds_cap(f->g, f->cap), cols, f->g.ntiles);
-  f->near.on = f->h_rep.near != 0;
+  plan_near(f);
   return upload_rep(f);
 }
 
@@ -1093,6 +1102,7 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
     if (counts[0]) f->gather_ok = false;
     f->global_inline = counts[1] == 0;
   }
+  plan_near(f);  // as global_inline now is
   // steps whose counts go straight into the scan's tile sums: gathered
   // steps on a field without global-path tiles (their atomics would crowd
   // one sum), whose tiles fit the LDS histogram and whole scan tiles

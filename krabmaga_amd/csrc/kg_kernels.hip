@@ -489,7 +489,10 @@ __global__ __launch_bounds__(kFlockThreads) void k_flock(
 // quotients (6.6 us a round, whatever the lanes in it), with many tiles VALU
 // issue.  So up to two tiles per CU take kT = 1,024 threads and one round for
 // all but a tile twice as full as the average (450 birds): 16,384 boids 20.5
-// -> 16.4 us, 65,537 21.9 -> 17.8, 262,144 25.4 -> 23.9; up to four 512.
+// -> 16.4 us, 65,537 21.9 -> 17.8, 262,144 25.4 -> 23.9; up to four 512, and
+// more than that too if most tiles hold more than 256 birds (`full`; 1M
+// sparse, 420 to a tile: 63.4 -> 56.8 us over 1,000 steps; 17,000 tiles of
+// 260 189 -> 238, blobs' near-empty background 205 -> 317).
 // Eight waves per SIMD (64 VGPRs): only the inline global walk spills.
 constexpr uint32_t kNearOneRoundTiles = 512;
 constexpr uint32_t kNearWideTiles = 1024;
@@ -781,8 +784,8 @@ __global__ __launch_bounds__(kFlockThreads) void k_flock_global(
   }
 }
 
-int near_threads(uint32_t ntiles) {
-  return ntiles <= kNearOneRoundTiles ? 1024 : ntiles <= kNearWideTiles ? 512 : 256;
+int near_threads(uint32_t ntiles, bool full) {
+  return ntiles <= kNearOneRoundTiles ? 1024 : ntiles <= kNearWideTiles || full ? 512 : 256;
 }
 size_t near_lds_bytes(int cap, int cols) { return near_smem_bytes(cap, cols); }
 
@@ -793,7 +796,7 @@ hipError_t launch_flock(const WorkList& wl, Buf R, const uint32_t* offset, Buf W
                         const NearPlan& near) {
   if (wl.ntiles == 0) return hipSuccess;
   if (near.on) {
-    const int threads = near_threads(wl.ntiles);
+    const int threads = near.threads;
     auto kern = inline_global ? k_flock_near<256, true> : k_flock_near<256, false>;
     if (threads == 512) kern = inline_global ? k_flock_near<512, true> : k_flock_near<512, false>;
     if (threads == 1024)

@@ -44,16 +44,17 @@ hipError_t launch_scatter_append(const WorkList& wl, Buf A, uint32_t* cursor, Bu
 hipError_t launch_sort_bins(const WorkList& wl, Buf R, const uint32_t* offset, Buf T,
                             hipStream_t s, uint32_t* bins = nullptr, uint32_t nbins = 0,
                             uint32_t* nlist = nullptr);
-// Threads per work-group of a near launch of ntiles.
-int near_threads(uint32_t ntiles);
+// Threads per work-group of a near launch of ntiles, most of them with more
+// than 256 birds if full.
+int near_threads(uint32_t ntiles, bool full);
 // Bytes of dynamic LDS for `cap` birds and `cols` columns.
 size_t near_lds_bytes(int cap, int cols);
 
 // How the flock step's tiles are staged on a near field (kg_near.hpp): birds
-// and columns of LDS per work-group; off: the general kernel.
+// and columns of LDS per work-group, its threads; off: the general kernel.
 struct NearPlan {
   bool on = false;
-  int cap = 0, cols = 0;
+  int cap = 0, cols = 0, threads = 0;
 };
 
 // gflag: one word per tile plus two (the last counts global-path tiles and

@@ -116,7 +116,9 @@ struct NearAcc {
 KG_HD bool near_corners(const Geom& g, int32_t bx, int32_t by, float lx, float ly, float T,
                         int want) {
   const float x0 = (float)bx * g.d, y0 = (float)by * g.d;
-  const float x1 = fminf(x0 + g.d, g.w), y1 = fminf(y0 + g.d, g.h);
+  // (no fminf: it would have the walk canonicalise g.w and g.h at every trip)
+  const float xd = x0 + g.d, yd = y0 + g.d;
+  const float x1 = xd < g.w ? xd : g.w, y1 = yd < g.h ? yd : g.h;
   const float ax = x0 - lx, bx2 = x1 - lx, ay = y0 - ly, by2 = y1 - ly;
   if (want == 1)
     return fmaxf(ax * ax, bx2 * bx2) + fmaxf(ay * ay, by2 * by2) <= T;
@@ -129,14 +131,14 @@ KG_HD void near_candidate(const RepDev& rp, int32_t col0, float qx, float qy, ui
                           NearAcc* acc) {
   const float dx = qx - c.x, dy = qy - c.y;
   const float s = dx * dx + dy * dy;
-  bool ok = s <= rp.sq_sure;
-  if (!ok && s <= rp.sq_near) {  // rare: the corners decide
+  if (!((s <= rp.sq_near) & (cid != qid))) return;  // sq_sure <= sq_near
+  if (!(s <= rp.sq_sure)) {  // rare: the corners decide
     const int32_t bx = col0 + (int32_t)(B.z[e] >> kNearRowBits);
     const int32_t by = (int32_t)(B.z[e] & ((1u << kNearRowBits) - 1u));
     const bool in = s <= rp.sq_thresh;
-    ok = near_corners(rp.g, bx, by, qx, qy, rp.sq_thresh, in ? -1 : 1) != in;
+    if (near_corners(rp.g, bx, by, qx, qy, rp.sq_thresh, in ? -1 : 1) == in) return;
   }
-  if (ok && cid != qid) acc->add(dx, dy, s, c.hx, c.hy);
+  acc->add(dx, dy, s, c.hx, c.hy);
 }
 
 // Whether the bird at (qx, qy) of cell (cx, cy) finds itself: its own bag is

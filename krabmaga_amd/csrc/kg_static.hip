@@ -207,7 +207,7 @@ extern "C" int kg_schedule_step_static(const kg_field_desc* desc, const kg_flock
   NearPlan near;
   if (h.near)
     near = near_plan(pick_lds_cap(g, desc->capacity),
-                     std::min(kMaxStageCols, g.tx + 2 * h.disc_dist), g.ntiles);
+                     std::min(kMaxStageCols, g.tx + 2 * h.disc_dist), g.ntiles, false);
   KG_HIP(launch_flock(wl, c.R, c.offset, c.W, c.count, c.gstep, c.err, lds_cap, c.gflag, n, s,
                       Outbox{}, false, nullptr, 0, near));
   KG_HIP(launch_scan(c.count, c.offset2, c.cursor, g.nbins, ss, nullptr, s));
