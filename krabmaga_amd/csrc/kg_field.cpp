@@ -945,40 +945,42 @@ int kg_neighbor_sets(kg_field* f, float dist, uint32_t* row_ptr, uint32_t* ids, 
   uint32_t nR = 0;
   KG_HIP(hipMemcpy(&nR, f->offset + f->g.nbins, 4, hipMemcpyDeviceToHost));
   const float T = sq_threshold(dist);
-  uint32_t* d_cnt = nullptr;
-  KG_HIP(dmalloc(&d_cnt, nR + 1));
-  std::vector<uint32_t> cnt(nR);
-  hipError_t e = launch_neighbor_count(f->d_rep, f->R.b, f->offset, nR, dist, T, d_cnt, f->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(f->stream);
-  if (e == hipSuccess && nR)
-    e = hipMemcpy(cnt.data(), d_cnt, nR * sizeof(uint32_t), hipMemcpyDeviceToHost);
-  if (e != hipSuccess) {
-    (void)hipFree(d_cnt);
-    return set_error(KG_E_HIP, "neighbour count failed: %s", hipGetErrorString(e));
-  }
+  // one buffer: the 64-bit total, counts, row starts, the scan's cursors and
+  // its tile sums.  (Counts summed on the host and sent back as row starts
+  // took a third of the call.)
+  const size_t row = (size_t)nR + 1, nscan = ((size_t)nR + kScanTile - 1) / kScanTile;
+  uint32_t* d_buf = nullptr;
+  KG_HIP(dmalloc(&d_buf, 2 + 3 * row + nscan + 1));
+  uint32_t* const d_cnt = d_buf + 2;
+  uint32_t* const d_row = d_cnt + row;
+  uint32_t* d_ids = nullptr;
   uint64_t run = 0;
-  for (uint32_t i = 0; i < nR; ++i) {
-    row_ptr[i] = (uint32_t)run;
-    run += cnt[i];
-  }
-  row_ptr[nR] = (uint32_t)run;
+  hipError_t e = launch_fill_u32(d_buf, 0u, 2, f->stream);
+  if (e == hipSuccess)
+    e = launch_neighbor_count(f->d_rep, f->R.b, f->offset, nR, dist, T, d_cnt, f->stream);
+  if (e == hipSuccess) e = launch_sum_u32(d_cnt, nR, (uint64_t*)d_buf, f->stream);
+  if (e == hipSuccess && nR)
+    e = launch_scan(d_cnt, d_row, d_row + row, nR, ScanState{d_row + 2 * row}, nullptr, f->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(f->stream);
+  if (e == hipSuccess) e = hipMemcpy(&run, d_buf, sizeof(run), hipMemcpyDeviceToHost);
   *total = run;
-  if (run > cap || run > 0xFFFFFFFFull) {
-    (void)hipFree(d_cnt);
+  const bool fits = run <= cap && run <= 0xFFFFFFFFull;
+  row_ptr[nR] = (uint32_t)run;
+  if (e == hipSuccess && fits) e = dmalloc(&d_ids, run);
+  if (e == hipSuccess && fits)
+    e = launch_neighbor_fill(f->d_rep, f->R.b, f->offset, nR, dist, T, d_row, d_ids, f->stream);
+  // the row starts are complete: they come over while the ids are found
+  if (e == hipSuccess && nR)
+    e = hipMemcpy(row_ptr, d_row, nR * sizeof(uint32_t), hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = hipStreamSynchronize(f->stream);
+  if (e == hipSuccess && fits && run)
+    e = hipMemcpy(ids, d_ids, run * sizeof(uint32_t), hipMemcpyDeviceToHost);
+  (void)hipFree(d_buf);
+  (void)hipFree(d_ids);
+  if (e != hipSuccess) return set_error(KG_E_HIP, "neighbour sets failed: %s", hipGetErrorString(e));
+  if (!fits)
     return set_error(KG_E_CAPACITY, "%llu neighbour ids do not fit in %zu",
                      (unsigned long long)run, cap);
-  }
-  uint32_t* d_ids = nullptr;
-  e = hipMemcpy(d_cnt, row_ptr, (nR + 1) * sizeof(uint32_t), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = dmalloc(&d_ids, run);
-  if (e == hipSuccess)
-    e = launch_neighbor_fill(f->d_rep, f->R.b, f->offset, nR, dist, T, d_cnt, d_ids, f->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(f->stream);
-  if (e == hipSuccess && run)
-    e = hipMemcpy(ids, d_ids, run * sizeof(uint32_t), hipMemcpyDeviceToHost);
-  (void)hipFree(d_cnt);
-  (void)hipFree(d_ids);
-  if (e != hipSuccess) return set_error(KG_E_HIP, "neighbour fill failed: %s", hipGetErrorString(e));
   return KG_OK;
 }
 

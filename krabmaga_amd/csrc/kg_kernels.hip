@@ -1668,6 +1668,26 @@ hipError_t launch_neighbor_count(const RepDev* rep, Buf R, const uint32_t* offse
   return hipGetLastError();
 }
 
+// *out += the sum of v[0, n), in 64 bits (the row starts wrap at 32).
+__global__ void k_sum_u32(const uint32_t* __restrict__ v, uint32_t n,
+                          unsigned long long* __restrict__ out) {
+  __shared__ unsigned long long s_wave[256 / kWave];
+  unsigned long long sum = 0;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    sum += v[i];
+  for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+  if ((threadIdx.x & (kWave - 1)) == 0) s_wave[threadIdx.x / kWave] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(out, s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3]);
+}
+
+hipError_t launch_sum_u32(const uint32_t* v, uint32_t n, uint64_t* out, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_sum_u32, dim3(min(256u, (n + 255) / 256)), dim3(256), 0, s, v, n,
+                     (unsigned long long*)out);
+  return hipGetLastError();
+}
+
 __global__ void k_neighbor_fill(const RepDev* __restrict__ rep, Buf R,
                                 const uint32_t* __restrict__ offset, uint32_t n, float dist,
                                 float T, const uint32_t* __restrict__ row_ptr, uint32_t* ids) {

@@ -112,6 +112,8 @@ hipError_t launch_query(const RepDev* rep, Buf R, const uint32_t* offset, float 
                         uint32_t* nout, hipStream_t s);
 hipError_t launch_neighbor_count(const RepDev* rep, Buf R, const uint32_t* offset, uint32_t n,
                                  float dist, float T, uint32_t* counts, hipStream_t s);
+// *out (device) += the sum of v[0, n).
+hipError_t launch_sum_u32(const uint32_t* v, uint32_t n, uint64_t* out, hipStream_t s);
 hipError_t launch_neighbor_fill(const RepDev* rep, Buf R, const uint32_t* offset, uint32_t n,
                                 float dist, float T, const uint32_t* row_ptr, uint32_t* ids,
                                 hipStream_t s);
