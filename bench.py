@@ -521,7 +521,7 @@ def main():
             "workload": "flockers plain GPU drop-in: 1,048,576 boids, 20,480 x 20,480 torus, "
                         "discretization 10/1.5, radius 10, weights 1, jump 0.7",
             "agents": n, "side": w["side"], "seed": w["seed"],
-            "path": "three-kernel (k_flock, scan, k_rebin_gather), the field's default at "
+            "path": "three-kernel (k_flock_near, k_rebin_gather), the field's default at "
                     "this size" if three else "tile-resident (k_rt_step)",
         },
         "roofline": {
@@ -540,7 +540,7 @@ def main():
             "traffic_source": traffic_src,
             # the flock phase: k_flock, plus its k_flock_global launch (tiles
             # that do not fit LDS) on fields that need one, timed as one
-            "dominant_kernel": "k_flock (+ k_flock_global)" if three else "k_rt_step",
+            "dominant_kernel": "k_flock_near" if three else "k_rt_step",
             "dominant_kernel_us": dom_us,
             "dominant_kernel_bytes_per_agent": dom_bytes,
             "dominant_kernel_frac": dom_bytes * n / (dom_us * 1e-6) / HBM_PEAK if dom_us else 0.0,
