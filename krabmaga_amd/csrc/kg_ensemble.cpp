@@ -621,8 +621,7 @@ hipError_t binned_step(kg_ensemble* e, const WorkList& w) {
   else if (!summed)
     err = launch_scan(e->count, e->offset2, e->cursor, e->nbins, e->ss, e->gstep, e->stream, gate);
   if (err != hipSuccess) return err;
-  const Gate gt{gate, gate ? e->gate + 2 : nullptr, summed ? e->gate + (p ^ 1) : nullptr,
-                e->err};
+  const Gate gt{gate, gate ? e->gate + 2 : nullptr, summed ? e->gate + (p ^ 1) : nullptr};
   if (gate) {
     GatherScan sc;
     if (summed) {
@@ -756,7 +755,6 @@ int check_flags(kg_ensemble* e) {
   if (e->binned) {
     uint32_t errflag = 0;
     KG_HIP(hipMemcpy(&errflag, e->err, sizeof(errflag), hipMemcpyDeviceToHost));
-    if (errflag & 2u) return set_error(KG_E_STATE, "a rebinning lost agents");
     if (errflag & 4u)
       return set_error(KG_E_STATE, "the resident step found more birds than it was planned for");
     if (errflag) return set_error(KG_E_RANGE, "an agent left its run's bag grid");

@@ -179,9 +179,6 @@ int prof_collect(kg_field* f) {
 }
 
 int check_poison(kg_field* f) {
-  if (f->poisoned && (f->poison_bits & 2u))
-    return set_error(KG_E_STATE, "a rebinning lost agents in an earlier step; the field is "
-                                 "unusable");
   if (f->poisoned && (f->poison_bits & 4u))
     return set_error(KG_E_STATE, "the resident step found more birds than it was planned for");
   if (f->poisoned)
@@ -247,8 +244,7 @@ int lazy_update_impl(kg_field* f, uint64_t* step_gstep) {
     KG_HIP(launch_scan(f->count, f->offset2, f->cursor, f->g.nbins, f->ss, step_gstep, f->stream,
                        gate));
   }
-  const Gate gt{gate, gather ? f->gate + 2 : nullptr, summed ? f->gate + (p ^ 1) : nullptr,
-                f->err};
+  const Gate gt{gate, gather ? f->gate + 2 : nullptr, summed ? f->gate + (p ^ 1) : nullptr};
   if (f->w_aligned) {
     ProfScope ps(f, KG_KERNEL_SCATTER);
     if (gather) {

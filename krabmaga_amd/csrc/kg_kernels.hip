@@ -1305,8 +1305,9 @@ __device__ __forceinline__ void sort_bin_in_place(const Geom& g, Buf R, uint32_t
 }
 
 // The slow way of a tile: its own birds and its sources', a source whose
-// outbox overflowed read whole, go to their bins as they come, and the bins
-// are sorted in place.  Nothing here reads what another work-group of the
+// outbox overflowed read whole, go to their bins as they come (every bird of
+// the replica does, if that leaves a bin short), and the bins are sorted in
+// place.  Nothing here reads what another work-group of the
 // launch writes, so no tile waits for another.
 //
 // A call that takes the kernel's arguments from where they lie and finds the
@@ -1374,20 +1375,33 @@ __device__ __noinline__ void gather_slow(uint32_t item, uint32_t nlo, const Gath
     R2.hy[pos] = W.hy[src];
     R2.id[pos] = R.id[src];
   };
-  for (uint32_t i = t; i < nown; i += kT) take(lo + i);
-  for (uint32_t q = 0; q < kGatherSources; ++q) {
-    const uint32_t n = S.scnt[q];
-    if (n > kOutboxCap) {
-      const uint32_t sb = rp.bin_base + (S.sitem[q] - item0) * nbt;
-      const uint32_t hi = offset_cur[sb + nbt];
-      for (uint32_t i = offset_cur[sb] + t; i < hi; i += kT) take(i);
+  for (int whole = 0; whole < 2; ++whole) {
+    __syncthreads();
+    for (uint32_t b = t; b < nbt; b += kT) s_fill[b] = 0u;
+    if (t == 0) S.fail = 0u;
+    __syncthreads();
+    if (whole) {
+      const uint32_t hi = offset_cur[rp.bin_base + g.nbins];
+      for (uint32_t i = offset_cur[rp.bin_base] + t; i < hi; i += kT) take(i);
     } else {
-      for (uint32_t i = t; i < n; i += kT) take(ob.slot[(size_t)S.sitem[q] * kOutboxCap + i]);
+      for (uint32_t i = t; i < nown; i += kT) take(lo + i);
+      for (uint32_t q = 0; q < kGatherSources; ++q) {
+        const uint32_t n = S.scnt[q];
+        if (n > kOutboxCap) {
+          const uint32_t sb = rp.bin_base + (S.sitem[q] - item0) * nbt;
+          const uint32_t hi = offset_cur[sb + nbt];
+          for (uint32_t i = offset_cur[sb] + t; i < hi; i += kT) take(i);
+        } else {
+          for (uint32_t i = t; i < n; i += kT) take(ob.slot[(size_t)S.sitem[q] * kOutboxCap + i]);
+        }
+      }
     }
+    __syncthreads();
+    for (uint32_t b = t; b < nbt; b += kT)
+      if (s_fill[b] != s_bstart[b + 1] - s_bstart[b]) S.fail = 1u;
+    __syncthreads();
+    if (!S.fail) break;
   }
-  __syncthreads();
-  for (uint32_t b = t; b < nbt; b += kT)
-    if (s_fill[b] != s_bstart[b + 1] - s_bstart[b]) atomicOr(args->gate.err, 2u);
   for (uint32_t b = wid; b < nbt; b += kWaves) {
     const uint32_t m = s_bstart[b + 1] - s_bstart[b];
     if (m > 1u && m <= kSortWaveMax)
@@ -1549,13 +1563,14 @@ __global__ __launch_bounds__(kGatherThreads, 8) void k_rebin_gather(
   }
   if (biggest > kGatherBinMax || scnt > kOutboxCap) S.fail = 1u;
   __syncthreads();
-  // fail is set before the barrier only: every thread takes the same path,
-  // here and (a count the candidates do not reach) not at all later, so the
-  // slow way's registers do not add to the fast way's
-  if (__builtin_amdgcn_readfirstlane((int)S.fail) != 0) {
+  // fail is read between barriers, so every thread takes the same path; the
+  // kernel ends at the call, so that nothing the fast way holds lives past it
+  auto slow_if_failed = [&] {
+    if (__builtin_amdgcn_readfirstlane((int)S.fail) == 0) return;
     gather_slow(item, nlo, (const GatherArgs*)__builtin_amdgcn_kernarg_segment_ptr());
-    return;
-  }
+    __builtin_amdgcn_endpgm();
+  };
+  slow_if_failed();
 #pragma unroll
   for (uint32_t u = 0; u < kGatherRegs; ++u) {
     const uint32_t k = t + u * kT;
@@ -1574,10 +1589,12 @@ __global__ __launch_bounds__(kGatherThreads, 8) void k_rebin_gather(
     }
   }
   __syncthreads();
-  // every bird of a step that gather_reaches comes from a source: a bin that
-  // is not full is an error of the plan
+  // a bin that is not full: a bird came from further than the sources (one
+  // whose position is no number any more goes to cell 0)
   for (uint32_t b = t; b < nbt; b += kT)
-    if (s_fill[b] != s_bstart[b + 1] - s_bstart[b]) atomicOr(gate.err, 2u);
+    if (s_fill[b] != s_bstart[b + 1] - s_bstart[b]) S.fail = 1u;
+  __syncthreads();
+  slow_if_failed();
 #pragma unroll
   for (uint32_t u = 0; u < kGatherRegs; ++u) {
     if (cbs[u] == ~0u) continue;
@@ -1597,7 +1614,7 @@ hipError_t launch_rebin_gather(const WorkList& wl, Buf R, Buf W, const uint32_t*
                                uint32_t* offset_new, const Outbox& ob, Buf R2, const Gate& gate,
                                const GatherScan& sc, hipStream_t s) {
   if (wl.ntiles == 0) return hipSuccess;
-  if (!gate.flag || !gate.redone || !gate.err) return hipErrorInvalidValue;
+  if (!gate.flag || !gate.redone) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_rebin_gather, dim3(wl.ntiles), dim3(kGatherThreads), sizeof(GatherSmem), s,
                      wl.reps, wl.nreps, wl.tile_prefix, R, W, offset_cur, offset_new, ob, R2, gate,
                      sc);

@@ -84,9 +84,11 @@ KG_HD void scatter_append_one(const RepDev* reps, int nreps, const uint32_t* app
 // work-group per tile collects its candidates, ranks each inside its new
 // bin by (cell row, id) -- the order the bin sort gives -- and writes it to
 // its final slot, so the scatter and the bin sort need not run.  A tile that
-// cannot be done so (more than the work-group's candidates or new birds, an
-// outbox past kOutboxCap, a bin past kGatherBinMax birds) is rebinned by its
-// own work-group from whole tiles and its bins sorted in place.
+// cannot be done so (more than kGatherCap candidates or new birds, an outbox
+// past kOutboxCap, a bin past kGatherBinMax birds, or a bird that came from
+// further, as one whose position became NaN does: it goes to cell 0) is
+// rebinned by its own work-group from whole tiles, or the whole replica, and
+// its bins sorted in place.
 
 constexpr uint32_t kGatherThreads = 256;
 constexpr uint32_t kGatherCap = 2048;     // candidates and new birds of a tile, at most
@@ -102,14 +104,12 @@ struct Outbox {
 };
 
 // The gate of a gathered step: the flag of a step with a tile that took the
-// slow way, the count of such steps, the flag the gather clears for the
-// next step (or none: the scan clears this step's), and the error word (bit
-// 1: a bin's birds were not all found).
+// slow way, the count of such steps, and the flag the gather clears for the
+// next step (or none: the scan clears this step's).
 struct Gate {
   uint32_t* flag = nullptr;
   uint32_t* redone = nullptr;
   uint32_t* clear = nullptr;
-  uint32_t* err = nullptr;
 };
 
 // The scan done inside the gather, for a layout whose flock step left the
@@ -152,7 +152,7 @@ KG_HD int32_t gather_source(const Geom& g, uint32_t tile, uint32_t q) {
   return sy * g.ntx + sx;
 }
 
-// Whether the sources hold every bird that can enter a tile in a step: none
+// Whether the sources hold every bird that enters a tile in a step: none
 // moves further than one tile, and the step wraps both axes by the width
 // (bird.rs:147), which is a neighbouring tile only on a square field.  Other
 // fields rebin by scatter and sort.

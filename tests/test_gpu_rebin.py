@@ -1,5 +1,6 @@
 """The gather rebinning's slow way (a tile of more candidates than its
-work-group holds, a bin past 512 birds, past 2,048, an overflowed outbox) and
+work-group holds, a bin past 512 birds, past 2,048, an overflowed outbox, birds
+from further than the neighbouring tiles) and
 the fields it leaves to the scatter (not square, jumps past a tile): after
 every step the read buffer equals the oracle's, bit for bit."""
 import numpy as np
@@ -48,3 +49,28 @@ def test_every_rebinning_equals_the_oracle(oracle, width, height, jump, spread, 
     fl.step(steps)
     assert np.array_equal(ids, np.arange(n))
     assert np.array_equal(got.view(np.uint32), fl.state().view(np.uint32))
+
+
+def test_birds_without_a_position_go_to_the_first_cell(oracle):
+    """An infinite heading makes a position NaN, which lies in cell 0 of its
+    axis: the gather finds such birds though they pass many tiles."""
+    rng = np.random.default_rng(3)
+    x, y, hx, hy = crowds(rng, 700.0, 700.0, 9000, ())
+    far = np.flatnonzero((x > 300.0) & (y > 300.0))[:4]
+    hx[far[:2]] = np.inf
+    hy[far[1:]] = -np.inf
+    n, steps = x.size, 3
+    p = FlockParams(seed=7)
+    f = Field2D(700.0, 700.0, D, True, n)
+    f.set_object_locations(np.arange(n, dtype=np.uint32), x, y, hx, hy)
+    f.lazy_update()
+    for s in range(steps):
+        f.flock_step(p, s)
+        f.lazy_update()
+    got, ids = f.state_by_id(0)
+    fl = oracle.Flocker(700.0, 700.0, D, True, x, y, hx, hy, oracle.params(seed=7))
+    fl.step(steps)
+    want = fl.state()
+    assert np.array_equal(ids, np.arange(n)) and np.isnan(want).any()
+    same = (got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))
+    assert same.all()
