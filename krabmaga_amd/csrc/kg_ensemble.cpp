@@ -324,16 +324,23 @@ bool shrink_crowded(kg_ensemble* e, const std::vector<uint32_t>& counts) {
 // (the single-field crossover of the two paths lies between 16k and 64k).
 constexpr uint64_t kBinnedMeanAgents = 32768;
 
-// Every live run fits the resident step, and no form was asked for.
-bool want_resident(const kg_ensemble* e) {
-  if (e->want >= 0) return false;
-  bool any = false;
+// The launch of the live runs' resident step; false if one of them does not
+// fit it.
+bool resident_group(const kg_ensemble* e, ResGroup* grp) {
+  *grp = ResGroup{};
   for (const EnsRun& r : e->runs) {
     if (r.dead) continue;
     if (!r.res_bins) return false;
-    any = true;
+    grp->add(r.desc.agents, r.res_bins);
   }
-  return any;
+  return true;
+}
+
+// The live runs fit one launch of the resident step, and no form was asked
+// for.
+bool want_resident(const kg_ensemble* e) {
+  ResGroup grp;
+  return e->want < 0 && resident_group(e, &grp) && grp.cap > 0 && grp.fits(e->lds_limit);
 }
 
 bool want_binned(const kg_ensemble* e) {
@@ -579,14 +586,11 @@ int ready_binned(kg_ensemble* e) {
 
 // `n` (<= kResidentSteps) steps of every run in its own work-group.
 int resident_steps(kg_ensemble* e, uint32_t n) {
-  uint32_t cap = 1, bins = 1;
-  for (const EnsRun& r : e->runs) {
-    if (r.dead) continue;
-    cap = std::max(cap, r.desc.agents);
-    bins = std::max(bins, r.res_bins);
-  }
+  ResGroup grp;
+  if (!resident_group(e, &grp) || !grp.fits(e->lds_limit))
+    return set_error(KG_E_STATE, "the runs do not fit the resident step");
   KG_HIP(launch_resident(e->d_reps, e->d_prefix + 2 * (e->nreps + 1), e->nreps, e->R.b,
-                         e->offset, e->gstep, 0, n, e->err, cap, bins, e->stream));
+                         e->offset, e->gstep, 0, n, e->err, grp.cap, grp.bins, e->stream));
   KG_HIP(launch_add_u64(e->gstep, n, e->stream));
   e->steps_run += n;
   for (EnsRun& r : e->runs) r.steps_done += n;

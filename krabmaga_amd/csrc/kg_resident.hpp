@@ -75,6 +75,20 @@ KG_HD bool res_fits(const RepDev& rp, uint32_t agents, size_t lds, uint32_t* bin
   return res_smem_bytes(agents, b) <= lds;
 }
 
+// The runs of one launch: every work-group has the LDS of the most birds and
+// of the largest bin table among them, which need not be one run's (4,096
+// birds beside 200 in 16,384 bins: 163,868 bytes of a work-group's 163,840,
+// where each alone takes less than 115,000).
+struct ResGroup {
+  uint32_t cap = 0, bins = 0;
+
+  KG_HD void add(uint32_t agents, uint32_t res_bins) {
+    cap = cap > agents ? cap : agents;
+    bins = bins > res_bins ? bins : res_bins;
+  }
+  KG_HD bool fits(size_t lds) const { return res_smem_bytes(cap, bins) <= lds; }
+};
+
 // A bird between its walk and its place in LDS.
 struct ResBird {
   float x, y, hx, hy;
