@@ -30,11 +30,15 @@ struct GraphKey {
   int gather;         // the steps rebin by gather
   int inline_global;  // global-path tiles stepped inside k_flock
   int steps;          // even: the read buffer returns to the same array pair
+  // the read buffer's count, which the captured launches hold as a grid or a
+  // bound; 0 for gathered steps without the global kernel, which hold none
+  uint32_t agents;
   bool operator<(const GraphKey& o) const {
     if (parity != o.parity) return parity < o.parity;
     if (gather != o.gather) return gather < o.gather;
     if (inline_global != o.inline_global) return inline_global < o.inline_global;
     if (steps != o.steps) return steps < o.steps;
+    if (agents != o.agents) return agents < o.agents;
     return std::memcmp(params, o.params, sizeof(params)) < 0;
   }
 };
@@ -991,6 +995,23 @@ int kg_flock_step(kg_field* f, const kg_flock_params* p, uint64_t step) {
   return flock_impl(f, f->zero64);
 }
 
+// Destroys the graphs captured for another count of agents, so that a field
+// filled anew again and again does not keep them all.
+static int drop_stale_graphs(kg_field* f) {
+  bool synced = false;
+  for (auto it = f->graphs.begin(); it != f->graphs.end();) {
+    if (it->first.agents == 0u || it->first.agents == f->nR) {
+      ++it;
+      continue;
+    }
+    if (!synced) KG_HIP(hipStreamSynchronize(f->stream));  // one may still run
+    synced = true;
+    (void)hipGraphExecDestroy(it->second);
+    it = f->graphs.erase(it);
+  }
+  return KG_OK;
+}
+
 static int run_direct_step(kg_field* f) {
   if (int rc = flock_impl(f, f->gstep)) return rc;
   return lazy_update_impl(f, f->gstep);
@@ -1120,9 +1141,11 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
     key.gather = f->gathers() ? 1 : 0;
     key.inline_global = f->global_inline ? 1 : 0;
     key.steps = graph_steps(left);
+    key.agents = key.gather && key.inline_global ? 0u : f->nR;
     auto it = f->graphs.find(key);
     hipGraphExec_t exec = nullptr;
     if (it == f->graphs.end()) {
+      if (int rc = drop_stale_graphs(f)) return rc;
       hipGraph_t graph = nullptr;
       KG_HIP(hipStreamBeginCapture(f->stream, hipStreamCaptureModeThreadLocal));
       f->capturing = true;
