@@ -9,6 +9,8 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <utility>
+#include <vector>
 
 #include "../../include/krabgpu.h"
 #include "kg_geom.hpp"
@@ -51,6 +53,48 @@ template <class T>
 hipError_t dmalloc(T** p, size_t n) {
   return hipMalloc((void**)p, (n ? n : 1) * sizeof(T));
 }
+
+// Device arrays that live and die together, in one allocation.  hipFree puts
+// off the release of more than about eight blocks at a time, and each
+// hipMalloc after that waits 200 us for one of them (MI355X, blocks past
+// 2 MiB).  An ensemble of 12 runs and 60 steps, admitted, run, read and closed:
+// 16.7 ms with its 75 arrays apart, 8.3 ms with them in eight blocks.
+class DevBlock {
+ public:
+  // n elements for *p, from the next alloc() on; p stays valid till release().
+  template <class T>
+  void add(T** p, size_t n) {
+    parts_.push_back({p, size_});
+    size_ += ((n ? n : 1) * sizeof(T) + kAlign - 1) / kAlign * kAlign;
+  }
+  hipError_t alloc() {
+    const hipError_t e = hipMalloc(&base_, size_ ? size_ : kAlign);
+    if (e != hipSuccess) base_ = nullptr;
+    set();
+    return e;
+  }
+  // Every array to zero (not for a captured graph).
+  hipError_t clear() { return hipMemset(base_, 0, size_); }
+  void release() {
+    if (base_) (void)hipFree(base_);
+    base_ = nullptr;
+    set();
+    parts_.clear();
+    size_ = 0;
+  }
+
+ private:
+  static constexpr size_t kAlign = 256;
+  void set() {
+    for (const auto& q : parts_) {
+      void* const v = base_ ? (uint8_t*)base_ + q.second : nullptr;
+      std::memcpy(q.first, &v, sizeof(v));  // a pointer of the array's own type
+    }
+  }
+  std::vector<std::pair<void*, size_t>> parts_;  // where the array's pointer is, its offset
+  void* base_ = nullptr;
+  size_t size_ = 0;
+};
 
 // Pinned host memory of one object for reading small buffers (launch_pack),
 // allocated at the first read and given back with the object.  Larger buffers

@@ -153,6 +153,9 @@ struct kg_ensemble {
   uint32_t* tsum[2] = {nullptr, nullptr};  // with the bin arrays (one per scan tile)
   uint32_t* counts(int p) const { return p ? count2 : count; }
 
+  // the bin arrays; the replica tables; the outboxes; err, gstep and gate
+  DevBlock bin_block, rep_block, outbox_block, word_block;
+
   // current layout
   std::vector<RepDev> h_reps;
   std::vector<uint32_t> h_prefix;
@@ -228,21 +231,18 @@ int reserve(kg_ensemble* e, size_t bins, size_t reps, size_t tiles) {
   if (bins > e->cap_bins) {
     KG_HIP(hipStreamSynchronize(e->stream));
     const size_t n = std::max(bins, e->cap_bins + e->cap_bins / 2);
-    for (uint32_t* p : {e->count, e->count2, e->offset, e->offset2, e->cursor, e->ss.partial,
-                        e->tsum[0], e->tsum[1]})
-      (void)hipFree(p);
-    e->count = e->count2 = e->offset = e->offset2 = e->cursor = e->ss.partial = nullptr;
-    e->tsum[0] = e->tsum[1] = nullptr;
+    e->bin_block.release();
     e->cap_bins = 0;
     const size_t nscan = (n + kScanTile - 1) / kScanTile + 1;
-    // offset and offset2 have the same size: the bin-grouped steps swap them
-    if ((err = dmalloc(&e->count, n)) != hipSuccess || (err = dmalloc(&e->offset, n + 1)) != hipSuccess ||
-        (err = dmalloc(&e->offset2, n + 1)) != hipSuccess ||
-        (err = dmalloc(&e->cursor, n)) != hipSuccess ||
-        (err = dmalloc(&e->ss.partial, nscan)) != hipSuccess ||
-        (err = dmalloc(&e->count2, n)) != hipSuccess ||
-        (err = dmalloc(&e->tsum[0], nscan)) != hipSuccess ||
-        (err = dmalloc(&e->tsum[1], nscan)) != hipSuccess)
+    DevBlock& bb = e->bin_block;
+    bb.add(&e->count, n);
+    bb.add(&e->count2, n);
+    // the same size: the bin-grouped steps swap them
+    bb.add(&e->offset, n + 1);
+    bb.add(&e->offset2, n + 1);
+    bb.add(&e->cursor, n);
+    for (uint32_t** p : {&e->ss.partial, &e->tsum[0], &e->tsum[1]}) bb.add(p, nscan);
+    if ((err = bb.alloc()) != hipSuccess)
       return set_error(KG_E_NOMEM, "ensemble bin arrays: %s", hipGetErrorString(err));
     // the scan leaves the counts at zero, and a summed run leaves both
     // arrays there; a fresh array starts there
@@ -253,15 +253,12 @@ int reserve(kg_ensemble* e, size_t bins, size_t reps, size_t tiles) {
   if (reps > e->cap_reps) {
     KG_HIP(hipStreamSynchronize(e->stream));
     const size_t n = std::max(reps, e->cap_reps + e->cap_reps / 2);
-    (void)hipFree(e->d_reps);
-    (void)hipFree(e->d_prefix);
-    (void)hipFree(e->rep_cursor);
-    e->d_reps = nullptr;
-    e->d_prefix = e->rep_cursor = nullptr;
+    e->rep_block.release();
     e->cap_reps = 0;
-    if ((err = dmalloc(&e->d_reps, n)) != hipSuccess ||
-        (err = dmalloc(&e->d_prefix, 3 * (n + 1))) != hipSuccess ||
-        (err = dmalloc(&e->rep_cursor, n)) != hipSuccess)
+    e->rep_block.add(&e->d_reps, n);
+    e->rep_block.add(&e->d_prefix, 3 * (n + 1));
+    e->rep_block.add(&e->rep_cursor, n);
+    if ((err = e->rep_block.alloc()) != hipSuccess)
       return set_error(KG_E_NOMEM, "ensemble replica tables: %s", hipGetErrorString(err));
     e->cap_reps = n;
   }
@@ -364,18 +361,14 @@ int reserve_binned(kg_ensemble* e, size_t agents, size_t tiles) {
   if ((err = regrow(&e->gflag, &e->cap_gflag, tiles + 2)) != hipSuccess)
     return set_error(KG_E_NOMEM, "ensemble bin-grouped buffers: %s", hipGetErrorString(err));
   if (tiles > e->cap_outbox) {
-    (void)hipFree(e->outbox.n);
-    (void)hipFree(e->outbox.slot);
-    e->outbox = Outbox{};
+    e->outbox_block.release();
     e->cap_outbox = 0;
-    const size_t n = std::max(tiles, e->cap_outbox + e->cap_outbox / 2);
-    if ((err = dmalloc(&e->outbox.n, n)) != hipSuccess ||
-        (err = dmalloc(&e->outbox.slot, n * kOutboxCap)) != hipSuccess)
+    e->outbox_block.add(&e->outbox.n, tiles);
+    e->outbox_block.add(&e->outbox.slot, tiles * kOutboxCap);
+    if ((err = e->outbox_block.alloc()) != hipSuccess)
       return set_error(KG_E_NOMEM, "ensemble outboxes: %s", hipGetErrorString(err));
-    e->cap_outbox = n;
+    e->cap_outbox = tiles;
   }
-  if (!e->gate && (err = dmalloc(&e->gate, 3)) != hipSuccess)
-    return set_error(KG_E_NOMEM, "ensemble gate: %s", hipGetErrorString(err));
   return KG_OK;
 }
 
@@ -536,11 +529,6 @@ int rebuild(kg_ensemble* e) {
   if (binned) {
     // every bin into (cell y, id) order, the consumed build buffer as scratch
     KG_HIP(launch_sort_bins(w, e->R.b, e->offset, e->A2.b, e->stream));
-    if (!e->gstep) {
-      const hipError_t err = dmalloc(&e->gstep, 1);
-      if (err != hipSuccess)
-        return set_error(KG_E_NOMEM, "ensemble step counter: %s", hipGetErrorString(err));
-    }
     KG_HIP(hipMemsetAsync(e->gstep, 0, sizeof(uint64_t), e->stream));
     e->binned_ready = false;
     e->gather = false;
@@ -821,8 +809,11 @@ int kg_ensemble_create(const kg_tuning* tuning, kg_ensemble** out) {
   if (tuning) e->tuning = *tuning;
   e->lds_limit = device_lds_limit();
   hipError_t err;
+  e->word_block.add(&e->err, 1);
+  e->word_block.add(&e->gstep, 1);
+  e->word_block.add(&e->gate, 3);
   if ((err = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking)) != hipSuccess ||
-      (err = dmalloc(&e->err, 1)) != hipSuccess ||
+      (err = e->word_block.alloc()) != hipSuccess ||
       (err = hipMemsetAsync(e->err, 0, sizeof(uint32_t), e->stream)) != hipSuccess ||
       (err = hipStreamSynchronize(e->stream)) != hipSuccess) {
     kg_ensemble_destroy(e);
@@ -844,12 +835,9 @@ void kg_ensemble_destroy(kg_ensemble* e) {
   e->R.release();
   e->R2.release();
   e->W.release();
-  for (void* p : {(void*)e->count, (void*)e->offset, (void*)e->offset2, (void*)e->cursor,
-                  (void*)e->ss.partial, (void*)e->d_reps, (void*)e->d_prefix,
-                  (void*)e->rep_cursor, (void*)e->tcount, (void*)e->err, (void*)e->gflag,
-                  (void*)e->gstep, (void*)e->outbox.n, (void*)e->outbox.slot, (void*)e->gate})
-    (void)hipFree(p);
-  for (void* p : {(void*)e->count2, (void*)e->tsum[0], (void*)e->tsum[1]}) (void)hipFree(p);
+  for (DevBlock* b : {&e->bin_block, &e->rep_block, &e->outbox_block, &e->word_block}) b->release();
+  (void)hipFree(e->tcount);
+  (void)hipFree(e->gflag);
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;
 }

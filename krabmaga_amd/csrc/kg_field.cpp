@@ -53,7 +53,10 @@ struct kg_field {
   NearPlan near{};  // of the current parameters' window
   hipStream_t stream = nullptr;
 
-  DevBuf R, R2, W, A;
+  // every device array but tcount and the tile-resident layout's; those that
+  // start at zero
+  DevBlock block, zeroed;
+  DevBuf R, R2, W, A;  // in block
   int parity = 0;  // flips with every rebinning (R <-> R2)
   uint32_t *count = nullptr, *offset = nullptr, *offset2 = nullptr, *cursor = nullptr;
   ScanState ss{};
@@ -531,49 +534,36 @@ int kg_field_create(const kg_field_desc* desc, kg_field** out) {
   };
   hipError_t e;
   if ((e = hipStreamCreateWithFlags(&f->stream, hipStreamNonBlocking)) != hipSuccess) return fail(e);
-  if ((e = f->R.alloc(f->cap)) != hipSuccess) return fail(e);
-  if ((e = f->R2.alloc(f->cap)) != hipSuccess) return fail(e);
-  if ((e = f->W.alloc(f->cap)) != hipSuccess) return fail(e);
-  if ((e = f->A.alloc(f->cap)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->gflag, f->g.ntiles + 2u)) != hipSuccess) return fail(e);
   const uint32_t nb = f->g.nbins;
   const uint32_t nscan = (nb + kScanTile - 1) / kScanTile;
-  if ((e = dmalloc(&f->count, nb)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->offset, nb + 1)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->offset2, nb + 1)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->cursor, nb)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->ss.partial, nscan + 1)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->err, 1)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->gstep, 1)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->zero64, 1)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->prefix, 4)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->d_rep, 1)) != hipSuccess) return fail(e);
-  if ((e = dmalloc(&f->scratch, 4)) != hipSuccess) return fail(e);
   f->gather_ok = rebin_gather_enabled() && (uint32_t)(f->g.tx * f->g.tr) <= kGatherMaxBins;
+  DevBlock &blk = f->block, &zero = f->zeroed;
+  for (DevBuf* d : {&f->R, &f->R2, &f->W, &f->A}) add_buf(&blk, &d->b, f->cap);
+  blk.add(&f->cursor, nb);
+  blk.add(&f->prefix, 4);
+  blk.add(&f->d_rep, 1);
+  blk.add(&f->scratch, 4);
+  zero.add(&f->gflag, f->g.ntiles + 2u);
+  zero.add(&f->count, nb);
+  zero.add(&f->offset, nb + 1);
+  zero.add(&f->offset2, nb + 1);
+  zero.add(&f->ss.partial, nscan + 1);
+  zero.add(&f->err, 1);
+  zero.add(&f->gstep, 1);
+  zero.add(&f->zero64, 1);
   if (f->gather_ok) {
-    if ((e = dmalloc(&f->outbox.n, f->g.ntiles)) != hipSuccess) return fail(e);
-    if ((e = dmalloc(&f->outbox.slot, (size_t)f->g.ntiles * kOutboxCap)) != hipSuccess)
-      return fail(e);
-    if ((e = dmalloc(&f->gate, 3)) != hipSuccess) return fail(e);
-    if ((e = hipMemset(f->gate, 0, 3 * sizeof(uint32_t))) != hipSuccess) return fail(e);
-    if ((e = dmalloc(&f->count2, nb)) != hipSuccess) return fail(e);
-    if ((e = hipMemset(f->count2, 0, nb * sizeof(uint32_t))) != hipSuccess) return fail(e);
+    blk.add(&f->outbox.n, f->g.ntiles);
+    blk.add(&f->outbox.slot, (size_t)f->g.ntiles * kOutboxCap);
+    for (int k = 0; k < 2; ++k) blk.add(&f->tsum[k], nscan);
+    zero.add(&f->gate, 3);
+    zero.add(&f->count2, nb);
     if ((e = hipHostMalloc((void**)&f->seen, 2 * sizeof(uint32_t))) != hipSuccess)
       return fail(e);
     f->seen[0] = f->seen[1] = 0;
-    const uint32_t nscan = (f->g.nbins + kScanTile - 1) / kScanTile;
-    for (int k = 0; k < 2; ++k)
-      if ((e = dmalloc(&f->tsum[k], nscan)) != hipSuccess) return fail(e);
   }
-  // one-time clears (never inside a captured graph)
-  const std::pair<void*, size_t> clears[] = {
-      {f->count, sizeof(uint32_t) * nb},          {f->offset, sizeof(uint32_t) * (nb + 1)},
-      {f->offset2, sizeof(uint32_t) * (nb + 1)},  {f->ss.partial, sizeof(uint32_t) * (nscan + 1)},
-      {f->err, sizeof(uint32_t)},                 {f->gstep, sizeof(uint64_t)},
-      {f->gflag, sizeof(uint32_t) * (f->g.ntiles + 2u)},
-      {f->zero64, sizeof(uint64_t)}};
-  for (const auto& c : clears)
-    if ((e = hipMemset(c.first, 0, c.second)) != hipSuccess) return fail(e);
+  if ((e = blk.alloc()) != hipSuccess) return fail(e);
+  if ((e = zero.alloc()) != hipSuccess) return fail(e);
+  if ((e = zero.clear()) != hipSuccess) return fail(e);
   const uint32_t pre[4] = {0u, f->g.ntiles, 0u, 0u};
   if ((e = hipMemcpy(f->prefix, pre, sizeof(pre), hipMemcpyHostToDevice)) != hipSuccess) return fail(e);
   if ((e = hipMemcpy(f->d_rep, &f->h_rep, sizeof(RepDev), hipMemcpyHostToDevice)) != hipSuccess)
@@ -593,29 +583,9 @@ void kg_field_destroy(kg_field* f) {
   }
   for (hipEvent_t e : f->ev_pool) (void)hipEventDestroy(e);
   f->rt.release();
-  f->R.release();
-  f->R2.release();
-  f->W.release();
-  f->A.release();
-  (void)hipFree(f->count);
-  (void)hipFree(f->offset);
-  (void)hipFree(f->offset2);
-  (void)hipFree(f->cursor);
-  (void)hipFree(f->ss.partial);
-  (void)hipFree(f->err);
-  (void)hipFree(f->gstep);
-  (void)hipFree(f->zero64);
-  (void)hipFree(f->prefix);
-  (void)hipFree(f->d_rep);
-  (void)hipFree(f->scratch);
+  f->block.release();
+  f->zeroed.release();
   (void)hipFree(f->tcount);
-  (void)hipFree(f->gflag);
-  (void)hipFree(f->outbox.n);
-  (void)hipFree(f->outbox.slot);
-  (void)hipFree(f->gate);
-  (void)hipFree(f->tsum[0]);
-  (void)hipFree(f->tsum[1]);
-  (void)hipFree(f->count2);
   if (f->seen) (void)hipHostFree(f->seen);
   f->stage.release();
   if (f->stream) (void)hipStreamDestroy(f->stream);

@@ -9,9 +9,9 @@ RtDev RtState::dev() const {
   for (int p = 0; p < 2; ++p) {
     D.cnt[p] = cnt[p];
     D.boff[p] = boff[p];
-    D.stay[p] = stay[p].b;
-    D.inbox[p] = inbox[p].b;
-    D.spill[p] = spill[p].b;
+    D.stay[p] = stay[p];
+    D.inbox[p] = inbox[p];
+    D.spill[p] = spill[p];
     D.spill_rep[p] = spill_rep[p];
   }
   for (int k = 0; k < 3; ++k) {
@@ -38,17 +38,7 @@ void RtState::release() {
     if (ev_done[k]) (void)hipEventDestroy(ev_done[k]);
   }
   if (ev_fork) (void)hipEventDestroy(ev_fork);
-  (void)hipFree(meta);
-  (void)hipFree(dense);
-  for (uint32_t* p : {cnt[0], cnt[1], boff[0], boff[1], icnt[0], icnt[1], icnt[2], scnt,
-                      spill_rep[0], spill_rep[1], flags, ovf})
-    (void)hipFree(p);
-  (void)hipFree(gstep);
-  for (int p = 0; p < 2; ++p) {
-    stay[p].release();
-    inbox[p].release();
-    spill[p].release();
-  }
+  block.release();
   *this = RtState();
 }
 
@@ -72,25 +62,22 @@ int RtState::setup(const RtPlan& pl, const RtClassPlan& cls, uint64_t spill_cap,
     boff_alloc = bo;
     spill_alloc = sp;
     tiles_alloc = ti;
-    hipError_t e = hipSuccess;
-    auto ok = [&](hipError_t r) {
-      if (e == hipSuccess) e = r;
-    };
-    ok(dmalloc(&meta, tiles_alloc));
-    ok(dmalloc(&dense, tiles_alloc));
+    block.add(&meta, tiles_alloc);
+    block.add(&dense, tiles_alloc);
     for (int p = 0; p < 2; ++p) {
-      ok(dmalloc(&cnt[p], tiles_alloc));
-      ok(dmalloc(&boff[p], boff_alloc));
-      ok(stay[p].alloc(stay_alloc));
-      ok(inbox[p].alloc(inbox_alloc));
-      ok(spill[p].alloc(spill_alloc));
-      ok(dmalloc(&spill_rep[p], spill_alloc));
+      block.add(&cnt[p], tiles_alloc);
+      block.add(&boff[p], boff_alloc);
+      add_buf(&block, &stay[p], stay_alloc);
+      add_buf(&block, &inbox[p], inbox_alloc);
+      add_buf(&block, &spill[p], spill_alloc);
+      block.add(&spill_rep[p], spill_alloc);
     }
-    for (int k = 0; k < 3; ++k) ok(dmalloc(&icnt[k], tiles_alloc));
-    ok(dmalloc(&scnt, 3));
-    ok(dmalloc(&flags, 2));
-    ok(dmalloc(&ovf, 2 * (kRtOvfMax + 1)));
-    ok(dmalloc(&gstep, 1));
+    for (int k = 0; k < 3; ++k) block.add(&icnt[k], tiles_alloc);
+    block.add(&scnt, 3);
+    block.add(&flags, 2);
+    block.add(&ovf, 2 * (kRtOvfMax + 1));
+    block.add(&gstep, 1);
+    const hipError_t e = block.alloc();
     if (e != hipSuccess) {
       release();
       return set_error(KG_E_NOMEM, "tile-resident layout allocation failed: %s",

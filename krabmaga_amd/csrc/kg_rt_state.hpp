@@ -7,25 +7,32 @@
 
 namespace kg {
 
+// An agent buffer, its five arrays in one allocation (that of x), or part of a
+// block that owns them.
 struct DevBuf {
   Buf b{};
   hipError_t alloc(size_t cap) {
-    hipError_t e;
-    if ((e = dmalloc(&b.x, cap)) != hipSuccess) return e;
-    if ((e = dmalloc(&b.y, cap)) != hipSuccess) return e;
-    if ((e = dmalloc(&b.hx, cap)) != hipSuccess) return e;
-    if ((e = dmalloc(&b.hy, cap)) != hipSuccess) return e;
-    return dmalloc(&b.id, cap);
+    const size_t stride = ((cap ? cap : 1) + 63) / 64 * 64;  // 256 bytes
+    float* p = nullptr;
+    const hipError_t e = dmalloc(&p, 5 * stride);
+    b = Buf{};
+    if (e == hipSuccess)
+      b = Buf{p, p + stride, p + 2 * stride, p + 3 * stride, (uint32_t*)(p + 4 * stride)};
+    return e;
   }
   void release() {
     (void)hipFree(b.x);
-    (void)hipFree(b.y);
-    (void)hipFree(b.hx);
-    (void)hipFree(b.hy);
-    (void)hipFree(b.id);
     b = Buf{};
   }
 };
+
+inline void add_buf(DevBlock* block, Buf* b, size_t cap) {
+  block->add(&b->x, cap);
+  block->add(&b->y, cap);
+  block->add(&b->hx, cap);
+  block->add(&b->hy, cap);
+  block->add(&b->id, cap);
+}
 
 struct RtState {
   bool allocated = false;
@@ -42,11 +49,12 @@ struct RtState {
   uint32_t *cnt[2] = {nullptr, nullptr}, *boff[2] = {nullptr, nullptr};
   uint32_t* icnt[3] = {nullptr, nullptr, nullptr};
   uint32_t* scnt = nullptr;  // 3 counters
-  DevBuf stay[2], inbox[2], spill[2];
+  Buf stay[2]{}, inbox[2]{}, spill[2]{};
   uint32_t* spill_rep[2] = {nullptr, nullptr};
   uint32_t* flags = nullptr;
   uint64_t* gstep = nullptr;
   uint32_t* ovf = nullptr;  // 2 x (kRtOvfMax + 1)
+  DevBlock block;  // every device array above
   uint64_t G = 0;  // value of *gstep once queued work has run
   std::vector<std::pair<int, hipGraphExec_t>> graphs;  // (steps, exec)
   // the class launches of a step run side by side on these streams
