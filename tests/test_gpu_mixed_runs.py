@@ -47,3 +47,30 @@ def test_many_birds_beside_many_bins(tuning, other):
         ref, rids = f.state_by_id(0)
         assert np.array_equal(order, rids)
         assert np.array_equal(state.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.gpu
+def test_a_short_tail_is_not_rebuilt_for_the_resident_step():
+    """When the last run past the resident step's size has retired, the layout
+    is kept for a few steps more: a rebuild costs more than they do.  (The
+    retired run is under a third of the tiles, so nothing else asks for one.)"""
+    specs = [_run(900 + 100 * i, 250.0, 3 + i) for i in range(16)] + [_run(6000, 490.0, 20)]
+    with Ensemble() as ens:
+        ids = ens.admit(specs)
+        ens.run(3)
+        ens.retire(ids[-1])
+        builds = ens.stats()["builds"]
+        ens.run(1)
+        ens.run(4)
+        assert ens.stats()["builds"] == builds
+        ens.run(40)
+        ens.run(2)
+        assert ens.stats()["builds"] == builds + 1
+        got = [ens.state_by_id(i) for i in ids[:-1]]
+    for s, (state, order) in zip(specs, got):
+        f = Field2D(s.width, s.height, s.discretization, True, s.agents)
+        f.init_uniform(s.agents, s.init_seed, s.heading_mode)
+        f.schedule_run(s.params, 0, 50)
+        ref, rids = f.state_by_id(0)
+        assert np.array_equal(order, rids)
+        assert np.array_equal(state.view(np.uint32), ref.view(np.uint32))
