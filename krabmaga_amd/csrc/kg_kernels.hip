@@ -493,7 +493,9 @@ __global__ __launch_bounds__(kFlockThreads) void k_flock(
 // more than that too if most tiles hold more than 256 birds (`full`; 1M
 // sparse, 420 to a tile: 63.4 -> 56.8 us over 1,000 steps; 17,000 tiles of
 // 260 189 -> 238, blobs' near-empty background 205 -> 317).
-// Eight waves per SIMD (64 VGPRs): only the inline global walk spills.
+// Eight waves per SIMD (64 VGPRs).  With the inline global walk 17 VGPRs are
+// spilled, most of them in that walk, but two on every lane's way (about 10 MB
+// of scratch writes in a 1M step); without it none.
 constexpr uint32_t kNearOneRoundTiles = 512;
 constexpr uint32_t kNearWideTiles = 1024;
 
@@ -1314,17 +1316,28 @@ __device__ __forceinline__ void sort_bin_in_place(const Geom& g, Buf R, uint32_t
 // rest again, so that the fast way keeps its registers (inlined, or called
 // with what the kernel holds, it made the fast way spill the birds it holds
 // there).
-struct GatherArgs {  // k_rebin_gather's arguments
-  const RepDev* reps;
-  int nreps;
-  const uint32_t* tile_prefix;
-  Buf R, W;
-  const uint32_t* offset_cur;
-  uint32_t* offset_new;
-  Outbox ob;
-  Buf R2;
-  Gate gate;
-  GatherScan sc;
+//
+// The arguments are listed once, for the kernel and for the struct that the
+// call reads them through (the kernel lays them out as a struct does).  (As
+// one struct passed by value they lose __restrict__: a field's step took
+// 2.5 % longer at 16,384, 65,537 and 1M boids.)
+#define KG_GATHER_ARGS(sep)                     \
+  const RepDev* __restrict__ reps sep()         \
+  int nreps sep()                               \
+  const uint32_t* __restrict__ tile_prefix sep() \
+  Buf R sep()                                   \
+  Buf W sep()                                   \
+  const uint32_t* __restrict__ offset_cur sep() \
+  uint32_t* __restrict__ offset_new sep()       \
+  Outbox ob sep()                               \
+  Buf R2 sep()                                  \
+  Gate gate sep()                               \
+  GatherScan sc
+#define KG_SEMICOLON() ;
+#define KG_COMMA() ,
+
+struct GatherArgs {
+  KG_GATHER_ARGS(KG_SEMICOLON);
 };
 
 // The work-group's LDS, all of it dynamic: it starts at LDS address 0 in the
@@ -1432,10 +1445,7 @@ __device__ __noinline__ void gather_slow(uint32_t item, uint32_t nlo, const Gath
 // (128 threads to a tile, 15 tiles to a CU: 61 and 17.8 us, but a tile of
 // more than 1,024 birds then goes the slow way, which a field that gathers in
 // flocks soon has in every step.)
-__global__ __launch_bounds__(kGatherThreads, 8) void k_rebin_gather(
-    const RepDev* __restrict__ reps, int nreps, const uint32_t* __restrict__ tile_prefix, Buf R,
-    Buf W, const uint32_t* __restrict__ offset_cur, uint32_t* __restrict__ offset_new, Outbox ob,
-    Buf R2, Gate gate, GatherScan sc) {
+__global__ __launch_bounds__(kGatherThreads, 8) void k_rebin_gather(KG_GATHER_ARGS(KG_COMMA)) {
   constexpr uint32_t kT = kGatherThreads;
   constexpr uint32_t kPer = kGatherMaxBins / kT;  // bins per thread
   constexpr uint32_t kWaves = kT / kWave;
