@@ -1275,35 +1275,13 @@ __device__ __forceinline__ void sort_bin_in_place(const Geom& g, Buf R, uint32_t
     __syncthreads();
     return;
   }
-  auto order = [&](uint32_t i, uint32_t j) {  // i < j
-    const uint64_t ki = bin_key(g, R.y[s + i], R.id[s + i]);
-    const uint64_t kj = bin_key(g, R.y[s + j], R.id[s + j]);
-    if (ki <= kj) return;
-    auto swap = [&](auto* p) {
-      const auto v = p[s + i];
-      p[s + i] = p[s + j];
-      p[s + j] = v;
-    };
-    swap(R.x);
-    swap(R.y);
-    swap(R.hx);
-    swap(R.hy);
-    swap(R.id);
-  };
-  for (uint32_t k = 2; k < 2u * m; k *= 2) {
+  bitonic_passes(m, [&](uint32_t x) {
     for (uint32_t i = t; i < m; i += kT) {
-      const uint32_t j = i ^ (k - 1u);
-      if (j > i && j < m) order(i, j);
+      const uint32_t j = i ^ x;
+      if (j > i && j < m) sort_exchange(g, R, s, i, j);
     }
     __syncthreads();
-    for (uint32_t w = k / 4; w > 0; w /= 2) {
-      for (uint32_t i = t; i < m; i += kT) {
-        const uint32_t j = i ^ w;
-        if (j > i && j < m) order(i, j);
-      }
-      __syncthreads();
-    }
-  }
+  });
 }
 
 // The slow way of a tile: its own birds and its sources', a source whose
@@ -1374,19 +1352,9 @@ __device__ __noinline__ void gather_slow(uint32_t item, uint32_t nlo, const Gath
   uint32_t* const s_bstart = S.bstart;
   uint32_t* const s_fill = S.fill;
   uint64_t* const s_key = S.key;
-  auto take = [&](uint32_t src) {
-    const float x = W.x[src], y = W.y[src];
-    int32_t row;
-    const uint32_t b = gather_bin(g, tile, x, y, &row);
-    if (b >= nbt) return;
-    const uint32_t slot = atom_add(&s_fill[b], 1u);
-    if (slot >= s_bstart[b + 1] - s_bstart[b]) return;
-    const uint32_t pos = nlo + s_bstart[b] + slot;
-    R2.x[pos] = x;
-    R2.y[pos] = y;
-    R2.hx[pos] = W.hx[src];
-    R2.hy[pos] = W.hy[src];
-    R2.id[pos] = R.id[src];
+  auto take = [&](const uint32_t* list, uint32_t base, uint32_t n) {
+    for (uint32_t i = t; i < n; i += kT)
+      gather_take(g, tile, nlo, s_bstart, s_fill, R, W, list ? list[i] : base + i, R2);
   };
   for (int whole = 0; whole < 2; ++whole) {
     __syncthreads();
@@ -1394,20 +1362,11 @@ __device__ __noinline__ void gather_slow(uint32_t item, uint32_t nlo, const Gath
     if (t == 0) S.fail = 0u;
     __syncthreads();
     if (whole) {
-      const uint32_t hi = offset_cur[rp.bin_base + g.nbins];
-      for (uint32_t i = offset_cur[rp.bin_base] + t; i < hi; i += kT) take(i);
+      const uint32_t r0 = offset_cur[rp.bin_base];
+      take(nullptr, r0, offset_cur[rp.bin_base + g.nbins] - r0);
     } else {
-      for (uint32_t i = t; i < nown; i += kT) take(lo + i);
-      for (uint32_t q = 0; q < kGatherSources; ++q) {
-        const uint32_t n = S.scnt[q];
-        if (n > kOutboxCap) {
-          const uint32_t sb = rp.bin_base + (S.sitem[q] - item0) * nbt;
-          const uint32_t hi = offset_cur[sb + nbt];
-          for (uint32_t i = offset_cur[sb] + t; i < hi; i += kT) take(i);
-        } else {
-          for (uint32_t i = t; i < n; i += kT) take(ob.slot[(size_t)S.sitem[q] * kOutboxCap + i]);
-        }
-      }
+      take(nullptr, lo, nown);
+      gather_slow_sources(ob, S.sitem, S.scnt, offset_cur, rp.bin_base, item0, nbt, take);
     }
     __syncthreads();
     for (uint32_t b = t; b < nbt; b += kT)

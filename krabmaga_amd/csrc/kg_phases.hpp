@@ -194,6 +194,41 @@ KG_HD uint32_t gather_rank(const uint64_t* key, uint32_t lo, uint32_t hi, uint32
   return rank;
 }
 
+// The slow way's candidate src: to its bin's next free slot, if it lies in
+// tile `tile` and the bin (bstart, from nlo on) has one left.
+KG_HD void gather_take(const Geom& g, uint32_t tile, uint32_t nlo, const uint32_t* bstart,
+                       uint32_t* fill, Buf R, Buf W, uint32_t src, Buf R2) {
+  const float x = W.x[src], y = W.y[src];
+  int32_t row;
+  const uint32_t b = gather_bin(g, tile, x, y, &row);
+  if (b >= (1u << (g.tx_log2 + g.tr_log2))) return;
+  const uint32_t slot = atom_add(&fill[b], 1u);
+  if (slot >= bstart[b + 1] - bstart[b]) return;
+  const uint32_t pos = nlo + bstart[b] + slot;
+  R2.x[pos] = x;
+  R2.y[pos] = y;
+  R2.hx[pos] = W.hx[src];
+  R2.hy[pos] = W.hy[src];
+  R2.id[pos] = R.id[src];
+}
+
+// The slow way's sources: take(list, base, n) for entries list[0, n), or
+// base + [0, n) without a list -- a source's outbox, or its whole tile if the
+// outbox overflowed.  item0: the replica's first work item.
+template <class Take>
+KG_HD void gather_slow_sources(const Outbox& ob, const uint32_t* sitem, const uint32_t* scnt,
+                               const uint32_t* offset_cur, uint32_t bin_base, uint32_t item0,
+                               uint32_t nbt, const Take& take) {
+  for (uint32_t q = 0; q < kGatherSources; ++q) {
+    if (scnt[q] > kOutboxCap) {
+      const uint32_t sb = bin_base + (sitem[q] - item0) * nbt;
+      take(nullptr, offset_cur[sb], offset_cur[sb + nbt] - offset_cur[sb]);
+    } else {
+      take(ob.slot + (size_t)sitem[q] * kOutboxCap, 0u, scnt[q]);
+    }
+  }
+}
+
 // ---- rebinning of the flock kernel's output (aligned with R) ---------------
 
 struct TileRange {
@@ -238,6 +273,34 @@ KG_HD void scatter_aligned_one(const RepDev& rp, Buf R, Buf W, uint32_t i, uint3
 
 KG_HD uint64_t bin_key(const Geom& g, float y, uint32_t id) {
   return ((uint64_t)(uint32_t)cell_axis(g, y) << 32) | id;
+}
+
+// Entries i < j of the bin at s into order.
+KG_HD void sort_exchange(const Geom& g, Buf R, uint32_t s, uint32_t i, uint32_t j) {
+  const uint64_t ki = bin_key(g, R.y[s + i], R.id[s + i]);
+  const uint64_t kj = bin_key(g, R.y[s + j], R.id[s + j]);
+  if (ki <= kj) return;
+  auto swap = [&](auto* p) {
+    const auto v = p[s + i];
+    p[s + i] = p[s + j];
+    p[s + j] = v;
+  };
+  swap(R.x);
+  swap(R.y);
+  swap(R.hx);
+  swap(R.hy);
+  swap(R.id);
+}
+
+// The bitonic network over m entries, any m: pass(x) puts every pair i, i ^ x
+// with both below m into order, the smaller key first, so entries past the end
+// need not exist.
+template <class Pass>
+KG_HD void bitonic_passes(uint32_t m, const Pass& pass) {
+  for (uint32_t k = 2; k < 2u * m; k *= 2) {
+    pass(k - 1u);
+    for (uint32_t w = k / 4; w > 0; w /= 2) pass(w);
+  }
 }
 
 // Bins of at most kSortSmall entries are sorted by one lane: keys in
