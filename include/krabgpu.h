@@ -168,12 +168,14 @@ int kg_flock_step(kg_field *f, const kg_flock_params *p, uint64_t step);
  * each = [lazy_update if the step is 0] + kg_flock_step + lazy_update
  * (schedule.rs:349-351, 395-412).  Asynchronous: call kg_field_sync to wait.
  *
- * Two device paths give identical results: the three-kernel path (flock +
- * scan + scatter and bin sort) and, for toroidal fields whose window
- * (floor(radius/d) cells) fits one tile of halo, a tile-resident layout that
- * runs each whole step as ONE kernel launch.  By default fields of fewer
- * than 32,768 agents take the tile-resident step and larger ones the
- * three-kernel path (the faster of the two at each size on MI355X).
+ * Three device paths give identical results: the three-kernel path (flock +
+ * scan + rebinning) and, for toroidal fields whose window (floor(radius/d)
+ * cells) fits one tile of halo, a tile-resident layout that runs each whole
+ * step as ONE kernel launch, and a resident step that runs up to 256 steps
+ * per launch in one work-group's LDS (up to 4,096 agents).  By default fields
+ * that fit it take the resident step, other fields the three-kernel path --
+ * but toroidal ones of fewer than 32,768 agents the tile-resident step if
+ * they are only a few cells wide, or a jump passes 0.3 of the width.
  * `flags`: KG_RUN_GRAPH replays launches from HIP graphs; KG_RUN_BINNED
  * forces the three-kernel path; KG_RUN_TILE_RESIDENT the tile-resident step
  * where the field suits it (the two exclude each other). */
@@ -256,7 +258,8 @@ int kg_field_stats(kg_field *f, uint64_t out[16]);
  * toroidal Field2D, parameters, Philox key and schedule step -- in one
  * device layout, the same launches per schedule step for all of them: a
  * tile-resident layout (one launch per tile class), or the bin-grouped read
- * buffer stepped by the three-kernel path over every run at once.  A run's
+ * buffer stepped by the three-kernel path over every run at once, or by the
+ * resident step with a work-group per run.  A run's
  * results are bit-identical to the same run on its own kg_field
  * (kg_schedule_run), whatever else shares the ensemble.  Runs can join and
  * leave between kg_ensemble_run calls; the layout is rebuilt then. */
@@ -302,7 +305,10 @@ int kg_ensemble_retire(kg_ensemble *e, uint32_t id);
  * src/lib.rs:1163-1173).  flags: KG_RUN_GRAPH; KG_RUN_BINNED or
  * KG_RUN_TILE_RESIDENT choose the layout's form (the layout is rebuilt when
  * the form changes); without either, ensembles whose live runs average
- * 32,768 agents or more take the bin-grouped form.  Asynchronous. */
+ * 32,768 agents or more take the bin-grouped form, and those whose live runs
+ * all fit the resident step (up to 4,096 agents each) take that on it -- from
+ * the sixteenth step on where a larger run has just been retired.
+ * Asynchronous. */
 int kg_ensemble_run(kg_ensemble *e, uint32_t nsteps, int flags);
 
 /* Schedule steps run so far by run `id`. */

@@ -18,9 +18,11 @@
 // the tile-resident plan above (one k_rt_step launch per tile class and
 // step), and the bin-grouped read buffer itself, stepped by the
 // three-kernel path over every replica at once (one k_flock launch over all
-// tiles, one scan over all bins, one scatter and one bin sort).  By default
-// ensembles whose runs average 32,768 agents or more take the bin-grouped
-// form; KG_RUN_BINNED and KG_RUN_TILE_RESIDENT choose either.
+// tiles, the scan and the rebinning over all bins).  By default ensembles
+// whose runs average 32,768 agents or more take the bin-grouped form, and so
+// do those whose runs fit one launch of the resident step (kg_resident.hpp: a
+// work-group per run, up to 256 steps to a launch); KG_RUN_BINNED and
+// KG_RUN_TILE_RESIDENT choose either.
 #include <algorithm>
 #include <cstring>
 #include <map>
@@ -318,8 +320,12 @@ bool shrink_crowded(kg_ensemble* e, const std::vector<uint32_t>& counts) {
   return any;
 }
 
-// The form of the next layout: the requested one, or by the runs' mean size
-// (the single-field crossover of the two paths lies between 16k and 64k).
+// The form of the next layout: the requested one, the bin-grouped one where
+// every run steps resident, or by the runs' mean size.  The line is where the
+// general kernels' paths cross on single fields (between 16k and 64k birds).
+// Near runs step faster bin-grouped below it too, us a step, tile-resident to
+// bin-grouped: 187 runs of 2,884 birds on average 197 to 61, 25 of 10,647 121
+// to 37, 12 of 15,708 84 to 30; KG_RUN_BINNED chooses it.
 constexpr uint64_t kBinnedMeanAgents = 32768;
 
 // The launch of the live runs' resident step; false if one of them does not

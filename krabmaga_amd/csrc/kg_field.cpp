@@ -1007,24 +1007,25 @@ int kg_schedule_run(kg_field* f, const kg_flock_params* p, uint64_t first_step, 
     RepDev probe = f->h_rep;
     set_rep_params(&probe, *p);
     // by default a field that fits one work-group's LDS steps there, many
-    // steps to a launch
+    // steps to a launch (kResidentMaxAgents)
     uint32_t bins = 0;
     if (!(use_graph & (KG_RUN_BINNED | KG_RUN_TILE_RESIDENT)) &&
         res_fits(probe, f->nR, f->lds_limit, &bins)) {
       if (int rc = ensure_atomic(f)) return rc;
       if (int rc = set_params(f, p, first_step)) return rc;
-      for (uint32_t k = 0; k < nsteps; k += kResidentSteps) {
+      for (uint32_t k = 0, m = 0; k < nsteps; k += m) {
+        m = std::min(kResidentSteps, nsteps - k);
         ProfScope ps(f, KG_KERNEL_RT_STEP);
-        KG_HIP(launch_resident(f->d_rep, nullptr, 1, f->R.b, f->offset, f->zero64, k,
-                               std::min(kResidentSteps, nsteps - k), f->err, f->nR, bins,
-                               f->stream));
+        KG_HIP(launch_resident(f->d_rep, nullptr, 1, f->R.b, f->offset, f->zero64, k, m, f->err,
+                               f->nR, bins, f->stream));
       }
       return KG_OK;
     }
-    // by default small fields take the one-launch tile-resident step (fewer
-    // launches per step) and large ones the three-kernel path (more of its
-    // work-groups fit a CU): measured at constant density on MI355X, the two
-    // cross between 16k and 64k birds
+    // larger near fields take the three-kernel path (8,000 birds, 150 steps:
+    // 3.4 ms against 13.0 tile-resident).  Other fields of fewer than 32,768
+    // take the tile-resident step, if their windows suit it (fewer launches
+    // per step; the three-kernel path fits more work-groups to a CU): with
+    // the general kernels the two cross between 16k and 64k birds
     constexpr uint32_t kRtDefaultMaxAgents = 32768;
     const bool want_rt = (use_graph & KG_RUN_TILE_RESIDENT) ||
                          (!(use_graph & KG_RUN_BINNED) && !probe.near &&

@@ -20,9 +20,16 @@
 
 namespace kg {
 
-// Steps per launch: a bound on how long one launch can run (a step of the
-// largest field takes about 30 us).
+// Steps per launch.  A step of 4,096 birds takes 30 us where they are uniform
+// at 0.025 per unit^2 and 1.5 ms in one blob of sigma 1 (a walk is linear in
+// its window's birds, a step quadratic in a crowd's); the paths with a
+// work-group per tile took 1.5 ms for that blob too.
 constexpr uint32_t kResidentSteps = 256;
+// What a work-group's registers and LDS hold.  Against the three-kernel path,
+// fields of 0.025 birds per unit^2, us: one step 49 to 77 at 2,048 birds, 67
+// to 75 at 4,096; 200 steps 2,999 to 3,942 at 2,048, 4,369 to 4,149 at 3,072,
+// 5,971 to 4,494 at 4,096: single steps are shorter here at every size, runs
+// of many up to about 2,900 birds.
 constexpr uint32_t kResidentMaxAgents = 4096;
 // z holds 12 bits of column here
 constexpr int32_t kResidentMaxCols = 4095;

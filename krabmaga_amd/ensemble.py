@@ -98,10 +98,11 @@ class Ensemble:
     def run(self, nsteps, use_graph=True, binned=False, tile_resident=False):
         """Every run advances nsteps schedule steps (asynchronous).
 
-        By default ensembles whose runs average 32,768 agents or more step
-        the bin-grouped layout with the three-kernel path, smaller ones the
-        tile-resident layout; binned / tile_resident choose either (same
-        results)."""
+        By default ensembles whose runs all have up to 4,096 agents step
+        each run in a work-group of its own, those whose runs average 32,768
+        agents or more the bin-grouped layout with the three-kernel path, the
+        others the tile-resident layout; binned / tile_resident choose either
+        of the latter two (same results)."""
         flags = (1 if use_graph else 0) | (2 if binned else 0) | (4 if tile_resident else 0)
         check(self._L.kg_ensemble_run(self._h, nsteps, flags))
 

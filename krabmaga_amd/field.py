@@ -198,10 +198,13 @@ class Field2D:
                      tile_resident=False):
         """`nsteps` Schedule::step calls from `first_step` (simulate!'s loop).
 
-        By default fields of fewer than 32,768 agents take the one-launch
-        tile-resident step and larger ones the three-kernel path; binned=True
-        forces the three-kernel path, tile_resident=True the tile-resident
-        step where the field suits it (same results either way)."""
+        By default fields of up to 4,096 agents step in one work-group's LDS
+        (up to 256 steps per launch) and larger ones on the three-kernel path
+        (toroidal fields of fewer than 32,768 agents that are only a few cells
+        wide, or whose jump passes 0.3 of the width, the one-launch
+        tile-resident step); binned=True forces the three-kernel path,
+        tile_resident=True the tile-resident step where the field suits it
+        (same results either way)."""
         p = params.c()
         flags = (1 if use_graph else 0) | (2 if binned else 0) | (4 if tile_resident else 0)
         check(self._L.kg_schedule_run(self._h, ctypes.byref(p), first_step, nsteps, flags))
