@@ -306,9 +306,8 @@ int kg_ensemble_retire(kg_ensemble *e, uint32_t id);
  * KG_RUN_TILE_RESIDENT choose the layout's form (the layout is rebuilt when
  * the form changes); without either, ensembles whose live runs average
  * 32,768 agents or more take the bin-grouped form, and those whose live runs
- * all fit the resident step (up to 4,096 agents each) take that on it -- from
- * the sixteenth step on where a larger run has just been retired.
- * Asynchronous. */
+ * all fit the resident step (up to 4,096 agents each) take that on it -- some
+ * steps later where a larger run has just been retired.  Asynchronous. */
 int kg_ensemble_run(kg_ensemble *e, uint32_t nsteps, int flags);
 
 /* Schedule steps run so far by run `id`. */

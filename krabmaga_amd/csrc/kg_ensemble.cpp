@@ -349,9 +349,11 @@ bool want_resident(const kg_ensemble* e) {
 
 // Steps that a tile-resident layout whose runs have come to fit the resident
 // step (its last large run retired) still takes before it is rebuilt for it:
-// the rebuild takes 0.2 to 1.9 ms (8 to 150 runs of 2,500 birds), a resident
-// step is 60 to 110 us shorter.
-constexpr uint32_t kFormSteps = 16;
+// about as many as the rebuild costs.  It takes 0.16, 0.58 and 1.86 ms for 8,
+// 40 and 150 runs of 2,500 birds, a resident step is 61, 63 and 109 us
+// shorter.  (Sixteen steps for every layout: a served queue of 30 runs 3 %
+// slower than without the wait.)
+uint32_t form_steps(const kg_ensemble* e) { return 2u + e->nreps / 8u; }
 
 bool want_binned(const kg_ensemble* e) {
   if (e->want >= 0) return e->want == 1;
@@ -906,8 +908,11 @@ int kg_ensemble_run(kg_ensemble* e, uint32_t nsteps, int flags) {
   if (nsteps == 0) return KG_OK;
   e->want = (flags & KG_RUN_BINNED) ? 1 : ((flags & KG_RUN_TILE_RESIDENT) ? 0 : -1);
   if (e->built && !e->dirty && e->nreps > 0 && want_binned(e) != e->binned) {
-    if (e->binned || !want_resident(e) || nsteps >= kFormSteps - e->late_steps) e->dirty = true;
-    else e->late_steps += nsteps;
+    const uint32_t due = form_steps(e);
+    if (e->binned || !want_resident(e) || e->late_steps >= due || nsteps >= due - e->late_steps)
+      e->dirty = true;
+    else
+      e->late_steps += nsteps;
   }
   if (e->dirty || !e->built)
     if (int rc = rebuild(e)) return rc;

