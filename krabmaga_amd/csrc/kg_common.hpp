@@ -54,46 +54,88 @@ hipError_t dmalloc(T** p, size_t n) {
   return hipMalloc((void**)p, (n ? n : 1) * sizeof(T));
 }
 
-// Device arrays that live and die together, in one allocation.  hipFree puts
-// off the release of more than about eight blocks at a time, and each
-// hipMalloc after that waits 200 us for one of them (MI355X, blocks past
-// 2 MiB).  An ensemble of 12 runs and 60 steps, admitted, run, read and closed:
-// 16.7 ms with its 75 arrays apart, 8.3 ms with them in eight blocks.
+// Device arrays that live and die together, in as few allocations as pay.
+// What an allocation costs depends on what else is allocated and freed
+// (MI355X, ROCm 7.2): arrays under 2 MiB come out of blocks that the runtime
+// keeps, about 1 us each; larger ones are mapped anew, 12 us, but once eight or
+// so have been freed in a row the frees are put off and every allocation after
+// them waits 0.2 to 1.2 ms.  So the arrays take one piece where they fit the
+// runtime's block or the object has little else (`whole`), pieces of their
+// own while all are small, pieces of the runtime's block size up to a total of
+// 64 MiB, and else one piece.  Ensembles admitted, run, read and closed, ms:
+// 12 runs up to 120,000 birds, 60 steps, 12.7 with 75 arrays apart, 8.2; 50 up
+// to 30,000, 100 steps, 28.0 and 17.9; 30 up to 5,000 served 10.0 and 10.1 (10.2
+// in one piece).
 class DevBlock {
  public:
   // n elements for *p, from the next alloc() on; p stays valid till release().
   template <class T>
   void add(T** p, size_t n) {
-    parts_.push_back({p, size_});
-    size_ += ((n ? n : 1) * sizeof(T) + kAlign - 1) / kAlign * kAlign;
+    parts_.push_back({p, ((n ? n : 1) * sizeof(T) + kAlign - 1) / kAlign * kAlign, 0, 0});
   }
-  hipError_t alloc() {
-    const hipError_t e = hipMalloc(&base_, size_ ? size_ : kAlign);
-    if (e != hipSuccess) base_ = nullptr;
+  hipError_t alloc(bool whole = false) {
+    size_t total = 0, largest = 0;
+    for (const Part& q : parts_) {
+      total += q.size;
+      largest = q.size > largest ? q.size : largest;
+    }
+    size_t cut = total;  // bytes of a piece, at most, or those of one array
+    if (!whole && total > kPiece && largest < kOwn) cut = 0;
+    else if (!whole && largest <= kPiece && total <= kSplit) cut = kPiece;
+    for (Part& q : parts_) {
+      if (pieces_.empty() || pieces_.back().size + q.size > cut) pieces_.push_back({nullptr, 0});
+      q.piece = pieces_.size() - 1;
+      q.at = pieces_.back().size;
+      pieces_.back().size += q.size;
+    }
+    hipError_t e = hipSuccess;
+    for (Piece& q : pieces_)
+      if (e == hipSuccess && (e = hipMalloc(&q.base, q.size)) != hipSuccess) q.base = nullptr;
+    if (e != hipSuccess) free_pieces();
     set();
     return e;
   }
   // Every array to zero (not for a captured graph).
-  hipError_t clear() { return hipMemset(base_, 0, size_); }
+  hipError_t clear() {
+    hipError_t e = hipSuccess;
+    for (const Piece& q : pieces_)
+      if (e == hipSuccess) e = hipMemset(q.base, 0, q.size);
+    return e;
+  }
   void release() {
-    if (base_) (void)hipFree(base_);
-    base_ = nullptr;
+    free_pieces();
     set();
     parts_.clear();
-    size_ = 0;
+    pieces_.clear();
   }
 
  private:
+  struct Piece {
+    void* base;
+    size_t size;
+  };
+  struct Part {
+    void* p;  // where the array's pointer is
+    size_t size;
+    size_t piece, at;
+  };
   static constexpr size_t kAlign = 256;
-  void set() {
-    for (const auto& q : parts_) {
-      void* const v = base_ ? (uint8_t*)base_ + q.second : nullptr;
-      std::memcpy(q.first, &v, sizeof(v));  // a pointer of the array's own type
+  static constexpr size_t kPiece = (2u << 20) - (64u << 10), kOwn = 1u << 20, kSplit = 64u << 20;
+  void free_pieces() {
+    for (Piece& q : pieces_) {
+      if (q.base) (void)hipFree(q.base);
+      q.base = nullptr;
     }
   }
-  std::vector<std::pair<void*, size_t>> parts_;  // where the array's pointer is, its offset
-  void* base_ = nullptr;
-  size_t size_ = 0;
+  void set() {
+    for (const Part& q : parts_) {
+      void* const b = pieces_.empty() ? nullptr : pieces_[q.piece].base;
+      void* const v = b ? (uint8_t*)b + q.at : nullptr;
+      std::memcpy(q.p, &v, sizeof(v));  // a pointer of the array's own type
+    }
+  }
+  std::vector<Part> parts_;
+  std::vector<Piece> pieces_;
 };
 
 // Pinned host memory of one object for reading small buffers (launch_pack),

@@ -105,8 +105,8 @@ struct kg_ensemble {
   bool built = false;
 
   // device memory, grown on demand
-  DevBuf A, A2, R;  // unload target, build input, binned read buffer
-  size_t cap_a = 0, cap_a2 = 0, cap_r = 0;
+  DevBuf A2, R;  // build input, binned read buffer (the unload target is rt's)
+  size_t cap_a2 = 0, cap_r = 0;
   uint32_t *count = nullptr, *offset = nullptr, *cursor = nullptr;
   ScanState ss{};
   size_t cap_bins = 0, cap_scan = 0;
@@ -124,11 +124,11 @@ struct kg_ensemble {
   bool binned = false;  // the layout's form
   bool binned_ready = false;  // the buffers of the three-kernel steps are there
   int want = -1;        // requested form: -1 by run size, 0 tile-resident, 1 bin-grouped
-  DevBuf R2, W;
+  DevBuf R2;
+  Buf W{};  // in step_block
   size_t cap_r2 = 0, cap_w = 0;
   uint32_t* offset2 = nullptr;  // with the bin arrays (cap_bins + 1)
   uint32_t* gflag = nullptr;
-  size_t cap_gflag = 0;
   uint64_t* gstep = nullptr;
   int lds_cap = 1024;
   NearPlan near{};  // off unless every run is near
@@ -142,7 +142,7 @@ struct kg_ensemble {
   // with such steps drops it
   bool gather = false;
   Outbox outbox{};
-  size_t cap_outbox = 0;
+  size_t cap_step_tiles = 0;
   uint32_t* gate = nullptr;
   uint32_t redone_seen = 0;
   // gathered steps whose counts go straight into the scan tiles' sums (every
@@ -155,8 +155,9 @@ struct kg_ensemble {
   uint32_t* tsum[2] = {nullptr, nullptr};  // with the bin arrays (one per scan tile)
   uint32_t* counts(int p) const { return p ? count2 : count; }
 
-  // the bin arrays; the replica tables; the outboxes; err, gstep and gate
-  DevBlock bin_block, rep_block, outbox_block, word_block;
+  // few blocks (see DevBlock): the bin arrays, replica tables, tile counts, err,
+  // gstep and gate; W, gflag and the outboxes
+  DevBlock tables, step_block;
 
   // current layout
   std::vector<RepDev> h_reps;
@@ -180,10 +181,9 @@ struct kg_ensemble {
   }
 
   size_t bytes_held() const {
-    return (cap_a + cap_a2 + cap_r + cap_r2 + cap_w) * 20 + cap_bins * 20 +
-           (cap_bins / kScanTile + 2) * 12 + cap_gflag * 4 +
-           cap_outbox * (kOutboxCap + 1) * 4 +
-           rt.stay_alloc * 40 + rt.inbox_alloc * 40 + rt.spill_alloc * 44 +
+    return (cap_a2 + cap_r + cap_r2 + cap_w) * 20 + cap_bins * 20 +
+           (cap_bins / kScanTile + 2) * 12 + cap_step_tiles * (kOutboxCap + 2) * 4 +
+           rt.stay_alloc * 40 + rt.inbox_alloc * 40 + rt.spill_alloc * 64 +
            rt.boff_alloc * 8 + cap_tiles * 48;
   }
 
@@ -201,18 +201,6 @@ uint64_t scan_tile_align(uint64_t bins) {
   return (bins + kScanTile - 1) / kScanTile * kScanTile;
 }
 
-template <class T>
-hipError_t regrow(T** p, size_t* cap, size_t want) {
-  if (want <= *cap) return hipSuccess;
-  (void)hipFree(*p);
-  *p = nullptr;
-  const size_t n = std::max(want, *cap + *cap / 2);
-  hipError_t e = dmalloc(p, n);
-  if (e == hipSuccess) *cap = n;
-  else *cap = 0;
-  return e;
-}
-
 // Grows one agent buffer (its contents are not kept).
 int reserve_buf(kg_ensemble* e, DevBuf* b, size_t* cap, size_t want) {
   if (want <= *cap) return KG_OK;
@@ -227,46 +215,45 @@ int reserve_buf(kg_ensemble* e, DevBuf* b, size_t* cap, size_t want) {
   return KG_OK;
 }
 
-// Grows the bin arrays, replica tables and per-tile counts (contents not
-// kept).
+// Grows the bin arrays, replica tables, per-tile counts and words, one block
+// (contents not kept but the error word).
 int reserve(kg_ensemble* e, size_t bins, size_t reps, size_t tiles) {
-  hipError_t err = hipSuccess;
-  if (bins > e->cap_bins) {
-    KG_HIP(hipStreamSynchronize(e->stream));
-    const size_t n = std::max(bins, e->cap_bins + e->cap_bins / 2);
-    e->bin_block.release();
-    e->cap_bins = 0;
-    const size_t nscan = (n + kScanTile - 1) / kScanTile + 1;
-    DevBlock& bb = e->bin_block;
-    bb.add(&e->count, n);
-    bb.add(&e->count2, n);
-    // the same size: the bin-grouped steps swap them
-    bb.add(&e->offset, n + 1);
-    bb.add(&e->offset2, n + 1);
-    bb.add(&e->cursor, n);
-    for (uint32_t** p : {&e->ss.partial, &e->tsum[0], &e->tsum[1]}) bb.add(p, nscan);
-    if ((err = bb.alloc()) != hipSuccess)
-      return set_error(KG_E_NOMEM, "ensemble bin arrays: %s", hipGetErrorString(err));
-    // the scan leaves the counts at zero, and a summed run leaves both
-    // arrays there; a fresh array starts there
-    KG_HIP(hipMemsetAsync(e->count, 0, n * sizeof(uint32_t), e->stream));
-    KG_HIP(hipMemsetAsync(e->count2, 0, n * sizeof(uint32_t), e->stream));
-    e->cap_bins = n;
-  }
-  if (reps > e->cap_reps) {
-    KG_HIP(hipStreamSynchronize(e->stream));
-    const size_t n = std::max(reps, e->cap_reps + e->cap_reps / 2);
-    e->rep_block.release();
-    e->cap_reps = 0;
-    e->rep_block.add(&e->d_reps, n);
-    e->rep_block.add(&e->d_prefix, 3 * (n + 1));
-    e->rep_block.add(&e->rep_cursor, n);
-    if ((err = e->rep_block.alloc()) != hipSuccess)
-      return set_error(KG_E_NOMEM, "ensemble replica tables: %s", hipGetErrorString(err));
-    e->cap_reps = n;
-  }
-  if ((err = regrow(&e->tcount, &e->cap_tiles, tiles)) != hipSuccess)
-    return set_error(KG_E_NOMEM, "ensemble tile counts: %s", hipGetErrorString(err));
+  if (bins <= e->cap_bins && reps <= e->cap_reps && tiles <= e->cap_tiles) return KG_OK;
+  KG_HIP(hipStreamSynchronize(e->stream));
+  auto grown = [](size_t need, size_t held) { return need <= held ? held : std::max(need, held + held / 2); };
+  const size_t nb = grown(bins, e->cap_bins), nr = grown(reps, e->cap_reps);
+  const size_t nt = grown(tiles, e->cap_tiles);
+  const size_t nscan = (nb + kScanTile - 1) / kScanTile + 1;
+  uint32_t errflag = 0;
+  if (e->err) KG_HIP(hipMemcpy(&errflag, e->err, sizeof(errflag), hipMemcpyDeviceToHost));
+  DevBlock& t = e->tables;
+  t.release();
+  e->cap_bins = e->cap_reps = e->cap_tiles = 0;
+  t.add(&e->count, nb);
+  t.add(&e->count2, nb);
+  // the same size: the bin-grouped steps swap them
+  t.add(&e->offset, nb + 1);
+  t.add(&e->offset2, nb + 1);
+  t.add(&e->cursor, nb);
+  for (uint32_t** p : {&e->ss.partial, &e->tsum[0], &e->tsum[1]}) t.add(p, nscan);
+  t.add(&e->d_reps, nr);
+  t.add(&e->d_prefix, 3 * (nr + 1));
+  t.add(&e->rep_cursor, nr);
+  t.add(&e->tcount, nt);
+  t.add(&e->err, 1);
+  t.add(&e->gstep, 1);
+  t.add(&e->gate, 3);
+  const hipError_t err = t.alloc();
+  if (err != hipSuccess)
+    return set_error(KG_E_NOMEM, "ensemble tables: %s", hipGetErrorString(err));
+  // the scan leaves the counts at zero, and a summed run leaves both arrays
+  // there; a fresh array starts there
+  KG_HIP(hipMemsetAsync(e->count, 0, nb * sizeof(uint32_t), e->stream));
+  KG_HIP(hipMemsetAsync(e->count2, 0, nb * sizeof(uint32_t), e->stream));
+  KG_HIP(launch_fill_u32(e->err, errflag, 1, e->stream));
+  e->cap_bins = nb;
+  e->cap_reps = nr;
+  e->cap_tiles = nt;
   return KG_OK;
 }
 
@@ -371,19 +358,22 @@ bool want_binned(const kg_ensemble* e) {
 // offset table comes with the bin arrays).
 int reserve_binned(kg_ensemble* e, size_t agents, size_t tiles) {
   if (int rc = reserve_buf(e, &e->R2, &e->cap_r2, agents)) return rc;
-  if (int rc = reserve_buf(e, &e->W, &e->cap_w, agents)) return rc;
-  hipError_t err;
-  if ((err = regrow(&e->gflag, &e->cap_gflag, tiles + 2)) != hipSuccess)
+  if (agents <= e->cap_w && tiles <= e->cap_step_tiles) return KG_OK;
+  KG_HIP(hipStreamSynchronize(e->stream));
+  const size_t na = agents <= e->cap_w ? e->cap_w : std::max(agents, e->cap_w + e->cap_w / 2);
+  const size_t nt = std::max(tiles, e->cap_step_tiles);
+  DevBlock& b = e->step_block;
+  b.release();
+  e->cap_w = e->cap_step_tiles = 0;
+  add_buf(&b, &e->W, na);
+  b.add(&e->gflag, nt + 2);
+  b.add(&e->outbox.n, nt);
+  b.add(&e->outbox.slot, nt * kOutboxCap);
+  const hipError_t err = b.alloc();
+  if (err != hipSuccess)
     return set_error(KG_E_NOMEM, "ensemble bin-grouped buffers: %s", hipGetErrorString(err));
-  if (tiles > e->cap_outbox) {
-    e->outbox_block.release();
-    e->cap_outbox = 0;
-    e->outbox_block.add(&e->outbox.n, tiles);
-    e->outbox_block.add(&e->outbox.slot, tiles * kOutboxCap);
-    if ((err = e->outbox_block.alloc()) != hipSuccess)
-      return set_error(KG_E_NOMEM, "ensemble outboxes: %s", hipGetErrorString(err));
-    e->cap_outbox = tiles;
-  }
+  e->cap_w = na;
+  e->cap_step_tiles = nt;
   return KG_OK;
 }
 
@@ -420,9 +410,9 @@ int rebuild(kg_ensemble* e) {
   // survivors of a bin-grouped layout are already together in the read
   // buffer, at their append slots
   if (have_old && !e->binned) {
-    if (int rc = unload(e, e->A.b, 0, e->ntiles)) return rc;
+    if (int rc = unload(e, e->rt.out, 0, e->ntiles)) return rc;
   }
-  const Buf old_src = e->binned ? e->R.b : e->A.b;
+  const Buf old_src = e->binned ? e->R.b : e->rt.out;
   const bool binned = want_binned(e);
   uint32_t base = 0;
   for (size_t i = 0; i < e->runs.size(); ++i) {
@@ -455,7 +445,6 @@ int rebuild(kg_ensemble* e) {
     if (int rc = reserve(e, std::max<uint64_t>(lbins, 1), std::max<size_t>(e->runs.size(), 1),
                          std::max<uint64_t>(ltiles, 1)))
       return rc;
-    if (int rc = reserve_buf(e, &e->A, &e->cap_a, std::max<uint64_t>(agents, 1))) return rc;
     // replica table
     const uint32_t nreps = (uint32_t)e->runs.size();
     e->h_reps.assign(nreps, RepDev{});
@@ -550,7 +539,7 @@ int rebuild(kg_ensemble* e) {
     e->gather = false;
     e->parity = 0;
   } else {
-    if (int rc = e->rt.setup(plan, cls, e->nagents, e->stream)) return rc;
+    if (int rc = e->rt.setup(plan, cls, e->nagents, e->stream, true)) return rc;
     if (int rc = e->rt.reset(G, e->stream)) return rc;
     const RtDev D = e->rt.dev();
     for (int c = 0; c < e->rt.ncls; ++c)
@@ -615,7 +604,7 @@ hipError_t binned_step(kg_ensemble* e, const WorkList& w) {
   const bool summed = e->summed;
   uint32_t* gate = e->gather ? e->gate + (summed ? p : 0) : nullptr;
   uint32_t* count = summed ? e->counts(p) : e->count;
-  if ((err = launch_flock(w, e->R.b, e->offset, e->W.b, count, e->gstep, e->err, e->lds_cap,
+  if ((err = launch_flock(w, e->R.b, e->offset, e->W, count, e->gstep, e->err, e->lds_cap,
                           e->gflag, e->nagents, e->stream,
                           e->gather ? e->outbox : Outbox{}, false,
                           summed ? e->tsum[p] : nullptr, kEnsGlobalGrid, e->near)) !=
@@ -642,16 +631,16 @@ hipError_t binned_step(kg_ensemble* e, const WorkList& w) {
       sc.last_item = e->ntiles - 1;
       sc.prefixed = prefixed ? 1 : 0;
     }
-    if ((err = launch_rebin_gather(w, e->R.b, e->W.b, e->offset, e->offset2, e->outbox, e->R2.b,
+    if ((err = launch_rebin_gather(w, e->R.b, e->W, e->offset, e->offset2, e->outbox, e->R2.b,
                                    gt, sc, e->stream)) != hipSuccess)
       return err;
   } else {
-    if ((err = launch_scatter_aligned(w, e->R.b, e->W.b, e->offset, e->cursor, e->R2.b,
+    if ((err = launch_scatter_aligned(w, e->R.b, e->W, e->offset, e->cursor, e->R2.b,
                                       e->nagents, e->ss.partial, e->stream)) != hipSuccess)
       return err;
     // the write buffer has been consumed: it is the sort's scratch
     // (the cursors and the scan's sums, used by then, list its crowded bins)
-    if ((err = launch_sort_bins(w, e->R2.b, e->offset2, e->W.b, e->stream, e->cursor, e->nbins,
+    if ((err = launch_sort_bins(w, e->R2.b, e->offset2, e->W, e->stream, e->cursor, e->nbins,
                                 e->ss.partial)) != hipSuccess)
       return err;
   }
@@ -825,13 +814,7 @@ int kg_ensemble_create(const kg_tuning* tuning, kg_ensemble** out) {
   if (tuning) e->tuning = *tuning;
   e->lds_limit = device_lds_limit();
   hipError_t err;
-  e->word_block.add(&e->err, 1);
-  e->word_block.add(&e->gstep, 1);
-  e->word_block.add(&e->gate, 3);
-  if ((err = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking)) != hipSuccess ||
-      (err = e->word_block.alloc()) != hipSuccess ||
-      (err = hipMemsetAsync(e->err, 0, sizeof(uint32_t), e->stream)) != hipSuccess ||
-      (err = hipStreamSynchronize(e->stream)) != hipSuccess) {
+  if ((err = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking)) != hipSuccess) {
     kg_ensemble_destroy(e);
     return set_error(KG_E_NOMEM, "ensemble setup: %s", hipGetErrorString(err));
   }
@@ -846,14 +829,10 @@ void kg_ensemble_destroy(kg_ensemble* e) {
   e->drop_bgraphs();
   e->stage.release();
   e->rt.release();
-  e->A.release();
   e->A2.release();
   e->R.release();
   e->R2.release();
-  e->W.release();
-  for (DevBlock* b : {&e->bin_block, &e->rep_block, &e->outbox_block, &e->word_block}) b->release();
-  (void)hipFree(e->tcount);
-  (void)hipFree(e->gflag);
+  for (DevBlock* b : {&e->tables, &e->step_block}) b->release();
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;
 }
@@ -962,8 +941,8 @@ int kg_ensemble_read(kg_ensemble* e, uint32_t id, uint32_t* ids, float* x, float
   // the bin-grouped read buffer holds every run at its append slots; the
   // tile-resident layout is unloaded there first
   if (!e->binned)
-    if (int rc = unload(e, e->A.b, r->tile0, r->ntiles)) return rc;
-  const Buf src = e->binned ? e->R.b : e->A.b;
+    if (int rc = unload(e, e->rt.out, r->tile0, r->ntiles)) return rc;
+  const Buf src = e->binned ? e->R.b : e->rt.out;
   const size_t m = r->desc.agents;
   const uint32_t b = r->app_base;
   if (HostStage::fits(m) && e->stage.reserve(kStageAgents)) {

@@ -561,8 +561,8 @@ int kg_field_create(const kg_field_desc* desc, kg_field** out) {
       return fail(e);
     f->seen[0] = f->seen[1] = 0;
   }
-  if ((e = blk.alloc()) != hipSuccess) return fail(e);
-  if ((e = zero.alloc()) != hipSuccess) return fail(e);
+  if ((e = blk.alloc(true)) != hipSuccess) return fail(e);
+  if ((e = zero.alloc(true)) != hipSuccess) return fail(e);
   if ((e = zero.clear()) != hipSuccess) return fail(e);
   const uint32_t pre[4] = {0u, f->g.ntiles, 0u, 0u};
   if ((e = hipMemcpy(f->prefix, pre, sizeof(pre), hipMemcpyHostToDevice)) != hipSuccess) return fail(e);

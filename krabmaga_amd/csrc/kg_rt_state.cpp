@@ -42,7 +42,8 @@ void RtState::release() {
   *this = RtState();
 }
 
-int RtState::setup(const RtPlan& pl, const RtClassPlan& cls, uint64_t spill_cap, hipStream_t s) {
+int RtState::setup(const RtPlan& pl, const RtClassPlan& cls, uint64_t spill_cap, hipStream_t s,
+                   bool with_out) {
   const uint64_t nt = pl.sbase.size();
   drop_graphs();
   if (!allocated || pl.stay_total > stay_alloc || pl.inbox_total > inbox_alloc ||
@@ -72,6 +73,7 @@ int RtState::setup(const RtPlan& pl, const RtClassPlan& cls, uint64_t spill_cap,
       add_buf(&block, &spill[p], spill_alloc);
       block.add(&spill_rep[p], spill_alloc);
     }
+    if (with_out) add_buf(&block, &out, spill_alloc);
     for (int k = 0; k < 3; ++k) block.add(&icnt[k], tiles_alloc);
     block.add(&scnt, 3);
     block.add(&flags, 2);

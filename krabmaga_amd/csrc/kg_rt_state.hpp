@@ -50,6 +50,7 @@ struct RtState {
   uint32_t* icnt[3] = {nullptr, nullptr, nullptr};
   uint32_t* scnt = nullptr;  // 3 counters
   Buf stay[2]{}, inbox[2]{}, spill[2]{};
+  Buf out{};  // unload target (if asked for), of the spill lists' capacity
   uint32_t* spill_rep[2] = {nullptr, nullptr};
   uint32_t* flags = nullptr;
   uint64_t* gstep = nullptr;
@@ -62,9 +63,11 @@ struct RtState {
   hipEvent_t ev_fork = nullptr, ev_done[kRtMaxClasses] = {};
 
   RtDev dev() const;
-  // (Re)allocates for `plan` (growing only) and uploads the plan tables and
-  // the class split.
-  int setup(const RtPlan& plan, const RtClassPlan& cls, uint64_t spill_cap, hipStream_t s);
+  // (Re)allocates for `plan` (growing only), with room for spill_cap agents
+  // in each spill list and in `out` (with_out), and uploads the plan tables
+  // and the class split.
+  int setup(const RtPlan& plan, const RtClassPlan& cls, uint64_t spill_cap, hipStream_t s,
+            bool with_out = false);
   // Zeroes the counters and flags and sets the step counter to G.
   int reset(uint64_t G, hipStream_t s);
   void drop_graphs();

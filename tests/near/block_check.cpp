@@ -1,24 +1,28 @@
 // block_check.cpp -- the device arrays that share an allocation (DevBlock in
 // kg_common.hpp, DevBuf in kg_rt_state.hpp) over an allocator of the test's
-// own: one allocation for all of them, aligned, apart from each other and
-// inside it, null when it fails or is released.  Exit status 0: all agree.
+// own: as few allocations as their sizes ask for, aligned, apart from each
+// other and inside them, null when one fails or is released.  Exit status 0:
+// all agree.
 #define __HIP_PLATFORM_AMD__ 1
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <vector>
 
 #include "kg_rt_state.hpp"
 
 static std::map<void*, size_t> live;
 static int mallocs = 0;
 static bool fail_next = false;
+static int fail_after = -1;  // allocations that still succeed
 
 extern "C" hipError_t hipMalloc(void** p, size_t n) {
   ++mallocs;
   *p = nullptr;
-  if (fail_next) return hipErrorOutOfMemory;
+  if (fail_next || fail_after == 0) return hipErrorOutOfMemory;
+  if (fail_after > 0) --fail_after;
   *p = std::aligned_alloc(4096, (n + 4095) / 4096 * 4096);
   live[*p] = n;
   return hipSuccess;
@@ -106,8 +110,43 @@ static int blocks(size_t n) {
   return 0;
 }
 
+// n arrays of `bytes`: the allocations they take, whole or not.
+static int pieces(size_t n, size_t bytes, bool whole, int want) {
+  std::vector<uint8_t*> p(n);
+  DevBlock b;
+  for (auto& v : p) b.add(&v, bytes);
+  mallocs = 0;
+  EXPECT(b.alloc(whole) == hipSuccess && mallocs == want && (int)live.size() == want);
+  for (size_t i = 0; i < n; ++i) std::memset(p[i], (int)i + 1, bytes);
+  for (size_t i = 0; i < n; ++i)
+    EXPECT((uintptr_t)p[i] % 256 == 0 && p[i][0] == i + 1 && p[i][bytes - 1] == i + 1);
+  b.release();
+  EXPECT(live.empty());
+  for (auto& v : p) EXPECT(v == nullptr);
+  // the second allocation fails: the first is given back
+  if (want > 1) {
+    for (auto& v : p) b.add(&v, bytes);
+    fail_after = 1;
+    EXPECT(b.alloc(whole) != hipSuccess && live.empty());
+    fail_after = -1;
+    for (auto& v : p) EXPECT(v == nullptr);
+    b.release();
+  }
+  return 0;
+}
+
 int main() {
   int failed = 0;
+  const size_t K = 1024, M = 1024 * K;
+  failed += pieces(30, 60 * K, false, 1);         // fit one block of the runtime's
+  failed += pieces(30, 590 * K, false, 30);       // small: pieces of their own
+  failed += pieces(30, 590 * K, true, 1);         // little else allocated
+  failed += pieces(30, M, false, 30);             // one to a block
+  failed += pieces(8, M + 512 * K, false, 8);
+  failed += pieces(64, M, false, 64);             // the largest split
+  failed += pieces(65, M, false, 1);
+  failed += pieces(5, 2 * M, false, 1);           // past the runtime's block
+  failed += pieces(1, 0 + 5 * M, false, 1);
   for (size_t n : {0, 1, 63, 64, 65, 1000, 4096}) failed += buffers(n) + blocks(n);
   std::printf("%d scenario(s) failed\n", failed);
   return failed ? 1 : 0;
