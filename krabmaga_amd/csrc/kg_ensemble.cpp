@@ -400,8 +400,8 @@ int rebuild(kg_ensemble* e) {
   }
   if (agents >= (1ull << 31) || bins >= (1ull << 31) || tiles >= (1ull << 31))
     return set_error(KG_E_ADMIT, "ensemble too large for 32-bit indices");
-  // the old layout (replica tables, A) stays intact until its survivors
-  // are unloaded into A and copied into the build buffer A2
+  // the old layout (replica tables, rt) stays intact until its survivors are
+  // unloaded and copied into the build buffer A2
   if (int rc = reserve_buf(e, &e->A2, &e->cap_a2, std::max<uint64_t>(agents, 1))) return rc;
   const bool have_old = e->built && e->nreps > 0;
   const bool old_binned = have_old && e->binned;
@@ -426,9 +426,25 @@ int rebuild(kg_ensemble* e) {
     r.app_base = base;
     base += r.desc.agents;
   }
+  // Every run is in the build buffer at its new slot.  A build that fails from
+  // here on leaves them to the next one as the read buffer of a bin-grouped
+  // layout (which it reads run by run, in any order).
+  bool in_read_buffer = false;
+  auto fail = [&](int rc) {
+    if (!in_read_buffer) {
+      std::swap(e->R, e->A2);
+      std::swap(e->cap_r, e->cap_a2);
+    }
+    for (EnsRun& r : e->runs) r.fresh = false;
+    e->nreps = (uint32_t)e->runs.size();
+    e->built = e->binned = e->dirty = true;
+    e->binned_ready = false;
+    e->rt.G = G;
+    return rc;
+  };
   // the survivors have left the old read buffer: it may grow now
   if (old_binned)
-    if (int rc = reserve_buf(e, &e->R, &e->cap_r, std::max<uint64_t>(agents, 1))) return rc;
+    if (int rc = reserve_buf(e, &e->R, &e->cap_r, std::max<uint64_t>(agents, 1))) return fail(rc);
   e->drop_bgraphs();
   RtPlan plan;
   RtClassPlan cls;
@@ -440,11 +456,10 @@ int rebuild(kg_ensemble* e) {
       ltiles += r.g.ntiles;
     }
     if (lbins >= (1ull << 31) || ltiles >= (1ull << 31))
-      return set_error(KG_E_ADMIT, "ensemble too large for 32-bit indices");
-    // the old layout is no longer read: grow the tables and the unload buffer
+      return fail(set_error(KG_E_ADMIT, "ensemble too large for 32-bit indices"));
     if (int rc = reserve(e, std::max<uint64_t>(lbins, 1), std::max<size_t>(e->runs.size(), 1),
                          std::max<uint64_t>(ltiles, 1)))
-      return rc;
+      return fail(rc);
     // replica table
     const uint32_t nreps = (uint32_t)e->runs.size();
     e->h_reps.assign(nreps, RepDev{});
@@ -507,8 +522,9 @@ int rebuild(kg_ensemble* e) {
     uint32_t errflag = 0;
     KG_HIP(hipMemcpyAsync(&errflag, e->err, sizeof(errflag), hipMemcpyDeviceToHost, e->stream));
     KG_HIP(hipStreamSynchronize(e->stream));
+    in_read_buffer = true;
     if (errflag)
-      return set_error(KG_E_RANGE, "an agent discretized outside its run's bag grid");
+      return fail(set_error(KG_E_RANGE, "an agent discretized outside its run's bag grid"));
     if (binned) break;
     std::vector<double> expect(e->ntiles);
     for (uint32_t i = 0; i < nreps; ++i) {
@@ -528,7 +544,8 @@ int rebuild(kg_ensemble* e) {
     // tiles too crowded for every LDS class: shorter tiles for the runs that
     // hold the fullest ones, and bin again
     if (attempt >= kShrinkAttempts || !shrink_crowded(e, counts))
-      return set_error(KG_E_ADMIT, "the runs' tiles do not fit the LDS budget of the tile-resident step");
+      return fail(set_error(KG_E_ADMIT,
+                            "the runs' tiles do not fit the LDS budget of the tile-resident step"));
   }
   e->binned = binned;
   if (binned) {
@@ -539,7 +556,7 @@ int rebuild(kg_ensemble* e) {
     e->gather = false;
     e->parity = 0;
   } else {
-    if (int rc = e->rt.setup(plan, cls, e->nagents, e->stream, true)) return rc;
+    if (int rc = e->rt.setup(plan, cls, e->nagents, e->stream, true)) return fail(rc);
     if (int rc = e->rt.reset(G, e->stream)) return rc;
     const RtDev D = e->rt.dev();
     for (int c = 0; c < e->rt.ncls; ++c)

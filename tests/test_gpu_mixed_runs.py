@@ -74,3 +74,30 @@ def test_a_short_tail_is_not_rebuilt_for_the_resident_step():
         ref, rids = f.state_by_id(0)
         assert np.array_equal(order, rids)
         assert np.array_equal(state.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("before", [0, 5])
+def test_a_build_that_fails_leaves_the_runs_to_the_next(before):
+    """60,000 birds on 6 x 6 cells fit no LDS class of the tile-resident form:
+    the run is refused again and again, and steps in the bin-grouped form as it
+    would alone, with the run that was there before it."""
+    small, dense = _run(5000, 450.0, 40), _run(60000, 40.0, 41)
+    with Ensemble() as ens:
+        ids = ens.admit([small])
+        if before:
+            ens.run(before, tile_resident=True)
+        ids += ens.admit([dense])
+        for _ in range(2):
+            with pytest.raises(Exception, match="LDS budget"):
+                ens.run(1, tile_resident=True)
+        ens.run(2, binned=True)
+        got = [ens.state_by_id(i) for i in ids]
+        assert [ens.steps(i) for i in ids] == [before + 2, 2]
+    for s, steps, (state, order) in zip((small, dense), (before + 2, 2), got):
+        f = Field2D(s.width, s.height, s.discretization, True, s.agents)
+        f.init_uniform(s.agents, s.init_seed, s.heading_mode)
+        f.schedule_run(s.params, 0, steps)
+        ref, rids = f.state_by_id(0)
+        assert np.array_equal(order, rids)
+        assert np.array_equal(state.view(np.uint32), ref.view(np.uint32))
