@@ -54,18 +54,20 @@ hipError_t dmalloc(T** p, size_t n) {
   return hipMalloc((void**)p, (n ? n : 1) * sizeof(T));
 }
 
-// Device arrays that live and die together, in as few allocations as pay.
-// What an allocation costs depends on what else is allocated and freed
-// (MI355X, ROCm 7.2): arrays under 2 MiB come out of blocks that the runtime
-// keeps, about 1 us each; larger ones are mapped anew, 12 us, but once eight or
-// so have been freed in a row the frees are put off and every allocation after
-// them waits 0.2 to 1.2 ms.  So the arrays take one piece where they fit the
-// runtime's block or the object has little else (`whole`), pieces of their
-// own while all are small, pieces of the runtime's block size up to a total of
-// 64 MiB, and else one piece.  Ensembles admitted, run, read and closed, ms:
-// 12 runs up to 120,000 birds, 60 steps, 12.7 with 75 arrays apart, 8.2; 50 up
-// to 30,000, 100 steps, 28.0 and 17.9; 30 up to 5,000 served 10.0 and 10.1 (10.2
-// in one piece).
+// Device arrays that live and die together, in as many allocations as pay.
+// What one costs depends on what else is allocated and freed (MI355X, ROCm
+// 7.2).  Arrays under 1 MiB or so come out of 2 MiB blocks that the runtime
+// keeps while something is left in them, about 1 us each.  Larger ones are
+// mapped anew, 12 us, but once eight or so have been freed in a row the frees
+// are put off and whatever allocates next (a stream, a graph) waits 0.2 to 1.2
+// ms.  So arrays are allocated apart while all of them are small, then in
+// pieces of the runtime's block size up to a total of 64 MiB, then in one
+// piece; and in one piece where the object has little else (`whole`).
+// Ensembles admitted, run, read and closed, ms, every array apart and so: 12
+// runs up to 120,000 birds, 60 steps, 16.7 and 8.5; 50 up to 30,000, 100 steps,
+// 31.0 and 18.3; 30 up to 5,000, served, 9.8 and 9.7 (10.2 in one piece).
+constexpr size_t kOwnPiece = 1u << 20;  // smaller arrays are allocated by themselves
+
 class DevBlock {
  public:
   // n elements for *p, from the next alloc() on; p stays valid till release().
@@ -80,7 +82,7 @@ class DevBlock {
       largest = q.size > largest ? q.size : largest;
     }
     size_t cut = total;  // bytes of a piece, at most, or those of one array
-    if (!whole && total > kPiece && largest < kOwn) cut = 0;
+    if (!whole && largest < kOwnPiece) cut = 0;
     else if (!whole && largest <= kPiece && total <= kSplit) cut = kPiece;
     for (Part& q : parts_) {
       if (pieces_.empty() || pieces_.back().size + q.size > cut) pieces_.push_back({nullptr, 0});
@@ -120,7 +122,7 @@ class DevBlock {
     size_t piece, at;
   };
   static constexpr size_t kAlign = 256;
-  static constexpr size_t kPiece = (2u << 20) - (64u << 10), kOwn = 1u << 20, kSplit = 64u << 20;
+  static constexpr size_t kPiece = (2u << 20) - (64u << 10), kSplit = 64u << 20;
   void free_pieces() {
     for (Piece& q : pieces_) {
       if (q.base) (void)hipFree(q.base);

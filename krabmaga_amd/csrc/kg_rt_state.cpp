@@ -87,12 +87,13 @@ int RtState::setup(const RtPlan& pl, const RtClassPlan& cls, uint64_t spill_cap,
     }
     allocated = true;
   }
-  if (!ev_fork) {
+  // class 0 runs on the caller's stream, the others on streams of their own
+  // (0.15 ms each to create and destroy)
+  if (cls.ncls > 1 && !ev_fork)
     KG_HIP(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
-    for (int k = 0; k < kRtMaxClasses; ++k) {
-      KG_HIP(hipStreamCreateWithFlags(&aux[k], hipStreamNonBlocking));
-      KG_HIP(hipEventCreateWithFlags(&ev_done[k], hipEventDisableTiming));
-    }
+  for (int k = 1; k < cls.ncls; ++k) {
+    if (!aux[k]) KG_HIP(hipStreamCreateWithFlags(&aux[k], hipStreamNonBlocking));
+    if (!ev_done[k]) KG_HIP(hipEventCreateWithFlags(&ev_done[k], hipEventDisableTiming));
   }
   plan = pl;
   ntiles = (uint32_t)nt;

@@ -7,20 +7,31 @@
 
 namespace kg {
 
-// An agent buffer, its five arrays in one allocation (that of x), or part of a
-// block that owns them.
+// An agent buffer, its five arrays apart (small ones) or in one allocation,
+// that of x; or part of a block that owns them.
 struct DevBuf {
   Buf b{};
+  bool apart = false;
   hipError_t alloc(size_t cap) {
     const size_t stride = ((cap ? cap : 1) + 63) / 64 * 64;  // 256 bytes
-    float* p = nullptr;
-    const hipError_t e = dmalloc(&p, 5 * stride);
     b = Buf{};
-    if (e == hipSuccess)
+    apart = stride * sizeof(float) < kOwnPiece;
+    hipError_t e;
+    if (apart) {
+      if ((e = dmalloc(&b.x, stride)) != hipSuccess || (e = dmalloc(&b.y, stride)) != hipSuccess ||
+          (e = dmalloc(&b.hx, stride)) != hipSuccess ||
+          (e = dmalloc(&b.hy, stride)) != hipSuccess || (e = dmalloc(&b.id, stride)) != hipSuccess)
+        release();
+      return e;
+    }
+    float* p = nullptr;
+    if ((e = dmalloc(&p, 5 * stride)) == hipSuccess)
       b = Buf{p, p + stride, p + 2 * stride, p + 3 * stride, (uint32_t*)(p + 4 * stride)};
     return e;
   }
   void release() {
+    if (apart)
+      for (void* p : {(void*)b.y, (void*)b.hx, (void*)b.hy, (void*)b.id}) (void)hipFree(p);
     (void)hipFree(b.x);
     b = Buf{};
   }

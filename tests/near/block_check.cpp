@@ -68,21 +68,24 @@ static bool apart(std::initializer_list<std::pair<void*, size_t>> a) {
 static int buffers(size_t cap) {
   mallocs = 0;
   DevBuf d;
-  EXPECT(d.alloc(cap) == hipSuccess && mallocs == 1 && live.size() == 1);
+  const int want = (cap + 63) / 64 * 256 < kOwnPiece ? 5 : 1;
+  EXPECT(d.alloc(cap) == hipSuccess && mallocs == want && (int)live.size() == want);
   const size_t n = (cap ? cap : 1) * 4;
   EXPECT(apart({{d.b.x, n}, {d.b.y, n}, {d.b.hx, n}, {d.b.hy, n}, {d.b.id, n}}));
   d.release();
   EXPECT(live.empty() && !d.b.x && !d.b.y && !d.b.hx && !d.b.hy && !d.b.id);
   d.release();
-  fail_next = true;
-  EXPECT(d.alloc(cap) != hipSuccess && !d.b.x && !d.b.id);
-  fail_next = false;
+  for (int k = 0; k < want; ++k) {
+    fail_after = k;
+    EXPECT(d.alloc(cap) != hipSuccess && !d.b.x && !d.b.id && live.empty());
+  }
+  fail_after = -1;
   d.release();
   EXPECT(live.empty());
   return 0;
 }
 
-static int blocks(size_t n) {
+static int blocks(size_t n, bool whole) {
   mallocs = 0;
   DevBlock b;
   uint32_t *p = nullptr, *q = nullptr;
@@ -92,7 +95,7 @@ static int blocks(size_t n) {
   b.add(&r, 3);
   b.add(&q, 0);
   b.add(&s, n + 1);
-  EXPECT(b.alloc() == hipSuccess && mallocs == 1 && live.size() == 1);
+  EXPECT(b.alloc(whole) == hipSuccess && mallocs == (whole ? 1 : 4));
   EXPECT(apart({{p, n * 4}, {r, 24}, {q, 4}, {s, (n + 1) * 4}}));
   EXPECT(b.clear() == hipSuccess && (n == 0 || p[n - 1] == 0u) && r[2] == 0u && s[n] == 0.0f);
   std::swap(p, q);  // as the steps swap their offset tables
@@ -138,7 +141,7 @@ static int pieces(size_t n, size_t bytes, bool whole, int want) {
 int main() {
   int failed = 0;
   const size_t K = 1024, M = 1024 * K;
-  failed += pieces(30, 60 * K, false, 1);         // fit one block of the runtime's
+  failed += pieces(3, 60 * K, false, 3);
   failed += pieces(30, 590 * K, false, 30);       // small: pieces of their own
   failed += pieces(30, 590 * K, true, 1);         // little else allocated
   failed += pieces(30, M, false, 30);             // one to a block
@@ -147,7 +150,8 @@ int main() {
   failed += pieces(65, M, false, 1);
   failed += pieces(5, 2 * M, false, 1);           // past the runtime's block
   failed += pieces(1, 0 + 5 * M, false, 1);
-  for (size_t n : {0, 1, 63, 64, 65, 1000, 4096}) failed += buffers(n) + blocks(n);
+  for (size_t n : {0, 1, 63, 64, 65, 1000, 4096, 262080, 262081, 300000})
+    failed += buffers(n) + blocks(n % 5000, false) + blocks(n % 5000, true);
   std::printf("%d scenario(s) failed\n", failed);
   return failed ? 1 : 0;
 }
